@@ -5,9 +5,12 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -41,6 +44,11 @@ struct ptyk_ctx {
   // ePIE scratch
   float2* e_psi_old = nullptr;
   float2* e_psi = nullptr;
+  unsigned long long* e_flags = nullptr;  // team form: barrier flags (they stand at e_epoch)
+  float* e_rowmax = nullptr;
+  double* e_err = nullptr;
+  unsigned e_epoch = 1;
+  int cus = 0;  // compute units of the device
   // DM state
   float2* psi = nullptr;
   int* row_ptr = nullptr;
@@ -153,7 +161,7 @@ static void free_all(ptyk_ctx* c) {
     if (p) hipFree(p);
   void* ptrs[] = {c->tw, c->obj, c->obj_int, c->probe, c->probe_int, c->probe_tmp, c->amp, c->amp_scale,
                   c->amp_sum, c->avg, c->pos_dev, c->roi_dev, c->order_dev, c->scal, c->factors, c->e_psi_old,
-                  c->e_psi, c->psi, c->row_ptr, c->row_frames, c->probe_partial, c->obj_partial,
+                  c->e_psi, c->e_flags, c->e_rowmax, c->e_err, c->psi, c->row_ptr, c->row_frames, c->probe_partial, c->obj_partial,
                   c->probe_partial_sum, c->d_obj, c->d_probe, c->wave_row_ptr, c->wave_row_frames};
   for (void* p : ptrs)
     if (p) hipFree(p);
@@ -214,10 +222,17 @@ int ptyk_create(const ptyk_config* cfg, ptyk_ctx** out) {
   if ((e = dalloc(&c->pos_dev, n)) != hipSuccess) return bail(e, "positions");
   if ((e = dalloc(&c->roi_dev, n)) != hipSuccess) return bail(e, "roi");
   if ((e = dalloc(&c->order_dev, n)) != hipSuccess) return bail(e, "order");
-  if ((e = dalloc(&c->scal, PTYK_SCAL_COUNT)) != hipSuccess) return bail(e, "scalars");
+  if ((e = dalloc(&c->scal, PTYK_SCAL_COUNT + 1)) != hipSuccess) return bail(e, "scalars");
   if ((e = dalloc(&c->factors, 2)) != hipSuccess) return bail(e, "factors");
   if ((e = dalloc(&c->e_psi_old, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
   if ((e = dalloc(&c->e_psi, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
+  if ((e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, cfg->device)) != hipSuccess)
+    return bail(e, "device attribute");
+  if (epie_team_size((int)m, c->cus) > 0) {
+    if ((e = dalloc(&c->e_flags, PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE)) != hipSuccess) return bail(e, "epie flags");
+    if ((e = dalloc(&c->e_rowmax, cfg->obj_rows)) != hipSuccess) return bail(e, "epie row maxima");
+    if ((e = dalloc(&c->e_err, PTYK_EPIE_TEAM_MAX)) != hipSuccess) return bail(e, "epie errors");
+  }
   for (auto& ev : c->ev)
     if ((e = hipEventCreate(&ev)) != hipSuccess) return bail(e, "events");
   // Probe::m_maxIntensity starts at 1 (Probe.cpp:54-58); objMax at 0.
@@ -548,6 +563,45 @@ int ptyk_end_modal(ptyk_ctx* c) {
 }
 
 // ---------------------------------------------------------------- ePIE
+// The workgroups of an ePIE team wait for one another, so all of them have to be on the device at
+// once.  Iterations of several handles (from several threads) take their workgroups out of one
+// budget per device, one per CU whatever else fits there, and wait for their turn when it is spent.
+struct TeamBudget {
+  std::mutex mu;
+  std::condition_variable cv;
+  int left = -1;  // workgroups; set by the first use
+};
+class TeamSlots {
+ public:
+  TeamSlots(int device, int cus, int want) : b_(want > 0 ? budget(device) : nullptr), want_(want) {
+    if (!b_) return;
+    std::unique_lock<std::mutex> l(b_->mu);
+    if (b_->left < 0) b_->left = cus;
+    b_->cv.wait(l, [&] { return b_->left >= want_; });
+    b_->left -= want_;
+  }
+  ~TeamSlots() {
+    if (!b_) return;
+    {
+      std::lock_guard<std::mutex> l(b_->mu);
+      b_->left += want_;
+    }
+    b_->cv.notify_all();
+  }
+  TeamSlots(const TeamSlots&) = delete;
+  TeamSlots& operator=(const TeamSlots&) = delete;
+
+ private:
+  static TeamBudget* budget(int device) {
+    static std::mutex mu;
+    static std::map<int, TeamBudget> all;  // by device ordinal; elements stay where they are
+    std::lock_guard<std::mutex> l(mu);
+    return &all[device];
+  }
+  TeamBudget* b_;
+  int want_;
+};
+
 int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, double* err) {
   if (!c || !order) return fail(c, PTYK_EINVAL, "null argument");
   if (!c->have_frames || !c->have_pos || !c->have_probe)
@@ -589,10 +643,32 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
   a.update_probe = (flags & PTYK_FLAG_UPDATE_PROBE) ? 1 : 0;
   a.rms = (flags & PTYK_FLAG_RMS) ? 1 : 0;
   a.tex_quantize = c->cfg.tex_quantize;
-  HIPCHK(c, epie_iteration(a, c->stream));
-  double s[PTYK_SCAL_COUNT];
-  HIPCHK(c, hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const int team = epie_team_size(a.m, c->cus);
+  a.team_size = team;
+  a.team_flags = c->e_flags;
+  a.team_rowmax = c->e_rowmax;
+  a.team_err = c->e_err;
+  a.team_epoch = c->e_epoch;
+  a.team_limit = 1000000000LL;  // 10 s
+  double s[PTYK_SCAL_COUNT + 1];
+  {
+    TeamSlots slots(c->cfg.device, c->cus, team);
+    hipError_t e = epie_iteration(a, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->stream);
+    const hipError_t es = hipStreamSynchronize(c->stream);  // before the team's place is given back
+    HIPCHK(c, e);
+    HIPCHK(c, es);
+  }
+  if (team) {
+    const bool done = s[PTYK_EPIE_DONE] == (double)c->e_epoch;
+    c->e_epoch += epie_team_barriers(n);
+    if (!done) {  // the flags stand anywhere: bring them to where the next iteration starts
+      const std::vector<unsigned long long> at(PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE,
+                                               (unsigned long long)c->e_epoch << 32);
+      HIPCHK(c, hipMemcpy(c->e_flags, at.data(), at.size() * sizeof(at[0]), hipMemcpyHostToDevice));
+      return fail(c, PTYK_EDEVICE, "ePIE: the workgroups of a team were not on the device together; the iteration is incomplete");
+    }
+  }
   if (err) *err = a.rms ? s[PTYK_SCAL_ERROR] / n : 0.0;
   return PTYK_OK;
 }

@@ -5,13 +5,16 @@
 // d_updateProbe(M) (ProbeKernels.cu:425-458), the thrust maxima behind
 // Sample/Probe::updateMaxIntensity and d_calculateER (utilitiesKernels.cu:684-712)).
 //
-// ePIE is a chain of dependent position updates, so one persistent workgroup walks every
-// position of an iteration in the given order: one launch per iteration and no host round
-// trip per position. Single-mode frames of 64^2 and 128^2 keep the whole exit wave in LDS
-// (k_epie_lds); other sizes and the modal form keep the exit waves in an L2-resident scratch
-// and stage each 2D transform through LDS in row and column chunks (k_epie).
+// ePIE is a chain of dependent position updates, so one launch walks every position of an
+// iteration in the given order, with no host round trip per position.  Frames of 64^2 and more
+// are shared by a team of 8 to 32 workgroups (k_epie_team); smaller ones go to one workgroup that
+// keeps the exit waves in an L2-resident scratch and stages each 2D transform through LDS in row
+// and column chunks (k_epie).
+#include "../../include/ptyk.h"
 #include "ptyk_device.h"
 #include "ptyk_internal.h"
+
+#include <algorithm>
 
 namespace ptyk {
 
@@ -225,321 +228,607 @@ __global__ __launch_bounds__(PTYK_EPIE_NT) void k_epie(EpieArgs a) {
   }
 }
 
-// threadIdx.x behind an empty asm: per-lane addresses derived from it are recomputed in each
-// phase instead of being kept live (and spilled) across the transforms; the asm also bounds a
-// scheduling region, so each phase calls it once.
-__device__ __forceinline__ int lane() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
+// ---------------------------------------------------------------- team form (M >= 64)
+// A position's work is spread over a team of W workgroups that stay on the chip for the whole
+// iteration.  Workgroup w owns R = M / W rows of the frame (and of the probe) and, between the two
+// transform directions, C = R of its columns:
+//   rows    : ROI (bilinear) x P_k, row transform                     -> exchange buffer
+//   columns : column transform, modulus difference, inverse transform -> exchange buffer
+//   rows    : inverse row transform = psi - psi_old, object update, then the probe update
+// with a team barrier after each step (the last one also publishes the object for the next
+// position's ROI), so three barriers a position.  psi - psi_old comes out directly, since the
+// column step transforms Psi' - Psi / M^2 (the transform is linear); the Fourier error is of
+// psi_old's spectrum, which is Psi itself, and is summed there too.
+//
+// What bounds it: the chain of three exchanges through the cache shared by the XCDs, not bytes or
+// arithmetic.  So every value another workgroup reads (exchange buffer, object, |O|^2, maxima) is
+// written and read with device-scope accesses, which go to that cache by themselves, and a barrier
+// is a wait for the stores to be acknowledged, one flag store and a poll: no cache is written back
+// or invalidated (an agent-scope release here writes back a whole L2).  A thread holds 4 to 8
+// values, so a transform is 3 or 4 short stages between two LDS tiles with one workgroup barrier
+// each, its twiddles kept in registers for the whole iteration.
+//
+// Team sizes: 4 rows a workgroup.  More rows mean fewer flags to wait for but more instructions per
+// thread in every step of the chain (64^2 in 8 workgroups of 8 rows: 14.0 us a position, in 16 of 4:
+// 10.7; 128^2 in 16: 15.0, in 32: 12.0; 256^2 with three modes in 32: 42.6, in 64: 28.6; 512^2 in 64:
+// 33, in 128: 27).  One workgroup on one CU took 14.7, 44, 1120 and 1730.  The radix order of 128
+// is the one of the least error (median 1.5e-6 of the object over an iteration of the 12 x 12
+// benchmark scan; 2.0e-6 for 4 4 4 2).
+template <int M> struct TeamCfg;
+template <> struct TeamCfg<64>  { static constexpr int W = 16,  NT = 64,  S = 3, R0 = 4, R1 = 4, R2 = 4, R3 = 1; };
+template <> struct TeamCfg<128> { static constexpr int W = 32,  NT = 128, S = 4, R0 = 4, R1 = 4, R2 = 2, R3 = 4; };
+template <> struct TeamCfg<256> { static constexpr int W = 64,  NT = 256, S = 4, R0 = 4, R1 = 4, R2 = 4, R3 = 4; };
+template <> struct TeamCfg<512> { static constexpr int W = 128, NT = 512, S = 3, R0 = 8, R1 = 8, R2 = 8, R3 = 1; };
 
-// A f / |f| * nrm: the projection of modulus_phase without its atan2 / sincos (which would make
-// the modulus step the longest of a position on one CU), branch-free: f is first scaled by an
-// exact power of two so that |f|^2 cannot overflow or underflow; f = 0 gives A nrm, as there.
-__device__ __forceinline__ float2 modulus_unit(float2 f, float a, float nrm) {
-  const float s = fmaxf(fabsf(f.x), fabsf(f.y));
-  int e;
-  (void)frexpf(s, &e);
-  const float xs = ldexpf(f.x, -e), ys = ldexpf(f.y, -e);
-  const float k = a * nrm * rsqrtf(xs * xs + ys * ys);
-  return s > 0.f ? make_float2(xs * k, ys * k) : make_float2(a * nrm, 0.f);
-}
-
-// max of the |O|^2 cache over the canvas (non-negative values) and a flat index where it is
-// attained, 16 loads of 16 bytes in flight per thread
-struct MaxAt {
-  float v;
-  long at;
-};
-template <int NT>
-__device__ MaxAt canvas_max(const float* __restrict__ oi, long canvas, float* redf, long* redi) {
-  constexpr int U = 16;
-  const float4* oi4 = reinterpret_cast<const float4*>(oi);
-  const long c4 = canvas >> 2;
-  const int t = lane();
-  float mx = 0.f;
-  long ix = 0;
-  for (long q0 = 0; q0 < c4; q0 += (long)U * NT) {
-    float4 v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const long q = q0 + t + (long)u * NT;
-      v[u] = q < c4 ? oi4[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const long q = 4 * (q0 + t + (long)u * NT);
-      if (v[u].x > mx) { mx = v[u].x; ix = q; }
-      if (v[u].y > mx) { mx = v[u].y; ix = q + 1; }
-      if (v[u].z > mx) { mx = v[u].z; ix = q + 2; }
-      if (v[u].w > mx) { mx = v[u].w; ix = q + 3; }
-    }
-  }
-  for (long q = (c4 << 2) + t; q < canvas; q += NT)
-    if (oi[q] > mx) { mx = oi[q]; ix = q; }
-  const float m = block_max<NT>(mx, redf);
-  // a location of the maximum: the lowest index among the threads that hold it
-  long cand = mx == m ? ix : canvas;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) cand = min(cand, (long)__shfl_xor(cand, o, 64));
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) redi[threadIdx.x >> 6] = cand;
-  __syncthreads();
-  long best = redi[0];
-#pragma unroll
-  for (int i = 1; i < NT / 64; ++i) best = min(best, redi[i]);
-  __syncthreads();
-  return MaxAt{m, best};
-}
-
-// The object window [ib, ib + M + 2) x [jb, jb + M + 2) (indices clamped to the canvas) behind
-// a position's bilinear taps, staged in LDS with row pitch M + 2: every tap of the frame is an
-// element of it (the first tap of pixel (ii, jj) is at row ii or ii + 1 and column jj or jj + 1
-// of the window when ib = floor(pos.x), jb = floor(pos.y)).
-template <int M, int NT>
-__device__ __forceinline__ void load_window(const EpieArgs& a, int ib, int jb, float2* win) {
-  constexpr int WP = M + 2, WN = WP * WP, U = (WN + NT - 1) / NT;
-  const int t = lane();
-  float2 v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int e = t + u * NT;
-    const int r = min(max(ib + e / WP, 0), a.obj_rows - 1), c = min(max(jb + e % WP, 0), a.obj_cols - 1);
-    v[u] = e < WN ? a.obj[(long)r * a.obj_cols + c] : make_float2(0.f, 0.f);
-  }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int e = t + u * NT;
-    if (e < WN) win[e] = v[u];
-  }
-}
-
-// psi_old = ROI * P (bilinear ROI at the fractional position) from the staged window, into
-// registers (the caller writes it into the frame after a barrier: frame and window share LDS).
-template <int M, int NT, int PPT, bool QUANT>
-__device__ __forceinline__ void epie_roi(const EpieArgs& a, float2 pos, int ib, int jb, const float2* win,
-                                         float2 (&po)[PPT]) {
-  constexpr int WP = M + 2;
-  const int t = lane();
-  float2 pv[PPT];
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) pv[j] = a.probe[t + j * NT];
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) {
-    const int px = t + j * NT;
-    const TapPos q = tap_pos<QUANT>((float)(px % M) + pos.y + 0.5f, (float)(px / M) + pos.x + 0.5f);
-    const int r = min(max(q.j0 - ib, 0), M), c = min(max(q.i0 - jb, 0), M);
-    const float2* w = win + r * WP + c;
-    po[j] = cmul(bilinear_sum(q.al, q.be, w[0], w[1], w[WP], w[WP + 1]), pv[j]);
-  }
-}
-
-// Resident-frame layout: row pitch M + 1 (conflict-free rows and columns in LDS).
 template <int M>
-__device__ __forceinline__ int at(int px) {
-  return (px / M) * (M + 1) + (px % M);
+struct Team : TeamCfg<M> {
+  using T = TeamCfg<M>;
+  static constexpr int R = M / T::W;         // rows (and columns) of a workgroup
+  static constexpr int P = M + 8;            // pitch of a sequence in an LDS tile
+  static constexpr int TILE = R * P;         // float2 elements
+  static constexpr int PPT = R * M / T::NT;  // values per thread
+  static constexpr int WR = R + 2, WC = M + 2, WIN = WR * WC;  // object window behind the rows' ROI
+  static constexpr int WU = (WIN + T::NT - 1) / T::NT;
+  static constexpr int TILE_B = TILE > WIN ? TILE : WIN;  // the second tile also stages the window
+  static constexpr int TPR = T::NT / R;      // threads per row of the scan beside the ROI
+  static_assert(T::R0 * T::R1 * T::R2 * T::R3 == M, "radices");
+  static_assert(PPT <= R && R % PPT == 0, "a thread's amplitudes lie in the workgroup's columns of one row");
+  static_assert(TPR % 8 == 0, "threads beside the ROI: whole groups of 8 lanes per row");
+  static_assert(R * M % T::NT == 0 && M % 64 == 0 && T::W <= PTYK_EPIE_TEAM_MAX, "tile shape");
+};
+
+// Device-scope relaxed accesses: coherent between workgroups on different XCDs by themselves.
+__device__ __forceinline__ float2 ld_dev(const float2* p) {
+  const unsigned long long u =
+      __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((unsigned)u), __uint_as_float((unsigned)(u >> 32)));
+}
+__device__ __forceinline__ void st_dev(float2* p, float2 v) {
+  const unsigned long long u = __float_as_uint(v.x) | ((unsigned long long)__float_as_uint(v.y) << 32);
+  __hip_atomic_store((unsigned long long*)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float ld_dev(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_dev(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Object update at the rounded position (d_updateObjectArray) from psi - psi_old in LDS: all
-// loads of G pixels before their stores (the stores could otherwise alias the next loads).
-// Leaves conj(O_new) (psi - psi_old), the probe update's increment before its scale, in its
-// place, and returns this thread's max of the new |O|^2 with its flat canvas index.
-template <int M, int NT, int PPT, bool PC>
-__device__ __forceinline__ MaxAt epie_obj_update(const EpieArgs& a, int rx, int ry, float co, float2* lds) {
-  constexpr int G = 4;
-  MaxAt m{0.f, 0};
+// Team barrier in two halves, so that work which needs nothing from the others can stand between.
+// arrive: this workgroup's stores have reached the coherence point (a store leaves vmcnt when it is
+// acknowledged there), then its flag: the epoch and a value of the workgroup (read by thread 0 from
+// LDS, in *value; a non-negative float).  wait: one wave polls all W flags, one per lane, and leaves
+// the largest of the values in *most.  The wait is bounded (limit ticks of the 100 MHz clock): the
+// host admits no more workgroups than the device can hold at once, so it ends unless the device is
+// lost to something else; then every workgroup gives up and the host reports it.
+__device__ __forceinline__ void team_arrive(unsigned long long* flags, int w, unsigned epoch, const unsigned* value) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flags + w * PTYK_EPIE_FLAG_STRIDE, ((unsigned long long)epoch << 32) | *value, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float wave_max_pos(float v);
+template <int W>
+__device__ __forceinline__ bool team_wait(const unsigned long long* flags, unsigned epoch, long long limit, int* gone,
+                                          float* most) {
+  if (threadIdx.x < 64) {
+    const int l = threadIdx.x;
+    bool ok = false;
+    long long t0 = 0;
+    unsigned long long v = 0;
+    for (int i = 0;; ++i) {
+      bool here = true;
+      v = 0;
 #pragma unroll
-  for (int j0 = 0; j0 < PPT; j0 += G) {
-    const int t = lane();
-    float2 ov[G], pv[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const int px = t + (j0 + u) * NT;
-      ov[u] = a.obj[(long)(rx + px / M) * a.obj_cols + (ry + px % M)];
-      pv[u] = a.probe[px];
+      for (int q = 0; q < (W + 63) / 64; ++q)
+        if (W >= 64 || l < W) {
+          const unsigned long long f = __hip_atomic_load(flags + (l + q * 64) * PTYK_EPIE_FLAG_STRIDE, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
+          here = here && (int)((unsigned)(f >> 32) - epoch) >= 0;
+          v = max(v, f & 0xffffffffull);  // values are non-negative floats: ordered as integers
+        }
+      ok = __all(here);
+      if (ok) break;
+      if (i == 1024) t0 = wall_clock64();
+      if (i > 1024 && (i & 255) == 0 && wall_clock64() - t0 > limit) break;
     }
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const int px = t + (j0 + u) * NT;
-      const long oi = (long)(rx + px / M) * a.obj_cols + (ry + px % M);
-      const float2 d = lds[at<M>(px)];  // psi - psi_old
-      float2 o = cadd(ov[u], cscale(cmulcj(pv[u], d), co));
-      const float mag = sqrtf(o.x * o.x + o.y * o.y);
-      if (PC) o = clamp_phase(o);
-      a.obj[oi] = o;
-      a.obj_int[oi] = mag * mag;
-      if (mag * mag > m.v) m = MaxAt{mag * mag, oi};
-      lds[at<M>(px)] = cmulcj(o, d);
+    const float m = wave_max_pos(__uint_as_float((unsigned)v));
+    if (l == 0) {
+      *most = m;
+      if (!ok) *gone = 1;
     }
-    __builtin_amdgcn_sched_barrier(0);
   }
-  return m;
+  __syncthreads();
+  return *gone == 0;
 }
 
-// Probe update with the updated object (d_updateProbe), from the increment the object update
-// left in LDS; returns this thread's max |P|^2. The |P|^2 cache of the updated mode is written
-// once, after the last position (nothing reads it in between).
-template <int M, int NT, int PPT>
-__device__ __forceinline__ float epie_probe_update(const EpieArgs& a, float cp, const float2* lds) {
-  const int t = lane();
-  float2 pv[PPT];
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) pv[j] = a.probe[t + j * NT];
-  float mx = 0.f;
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) {
-    const int px = t + j * NT;
-    const float2 p = cadd(cscale(lds[at<M>(px)], cp), pv[j]);
-    a.probe[px] = p;
-    const float ia = sqrtf(p.x * p.x + p.y * p.y);
-    mx = fmaxf(mx, ia * ia);
-  }
-  return mx;
+// Maximum over a wave of non-negative values: in each row of 16 lanes by DPP moves, then the four
+// rows' values through scalar registers (about 40 cycles; six dependent LDS permutes took 0.3 us).
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float v) {
+  const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true);
+  return fmaxf(v, __int_as_float(o));
+}
+__device__ __forceinline__ float row16_max(float v) {
+  v = max_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  v = max_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  v = max_dpp<0x141>(v);  // row_half_mirror
+  return max_dpp<0x140>(v);  // row_mirror
+}
+__device__ __forceinline__ float wave_max_pos(float v) {
+  v = row16_max(v);
+  const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+  const float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+  const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+  const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
+  return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
-// Single-mode ePIE with the whole M x M exit wave resident in LDS (M (M + 1) complex values;
-// the object window of the bilinear ROI, (M + 2)^2, shares the space, 132 KiB at M = 128): both
-// 2D transforms and the modulus constraint run without a global round trip, and psi_old is
-// never stored (the modulus step transforms the difference). Each thread owns the pixels
-// px = tid + j NT of the frame in every phase. Same update equations and order as k_epie, with
-// psi - psi_old = IFFT(Psi' - Psi / M^2) in place of IFFT(Psi') - psi_old. One CU moves every
-// byte of a position, so the phases are arranged to move few: the ROI gathers come from the staged
-// window, the probe update takes its increment from LDS, and the canvas max after an object
-// update is rescanned only when the previous maximum lay inside the updated ROI (otherwise it is
-// the larger of the previous maximum and the ROI's new maximum, exactly).
-template <int M, int NT>
-__global__ __launch_bounds__(NT) void k_epie_lds(EpieArgs a) {
-  constexpr int P = M + 1;
-  constexpr int FRAME = (M + 2) * (M + 2);  // >= M * P
-  extern __shared__ float2 lds[];           // frame (pitch P) or window (pitch M + 2), then twiddles
-  float2* tws = lds + FRAME;
-  __shared__ float redf[NT / 64];
+// One radix-RX Stockham stage of R sequences from one tile to the other.
+template <int M, int RX>
+struct TeamStage {
+  using T = Team<M>;
+  static constexpr int NB = T::R * (M / RX);                 // butterflies
+  static constexpr int BPT = (NB + T::NT - 1) / T::NT;       // per thread
+  static constexpr bool ALL = NB % T::NT == 0;               // every thread has BPT of them
+  static constexpr int NW = RX > 1 ? BPT * (RX - 1) : 1;     // twiddles per thread
+};
+template <int M, int RX, int NS, bool INV>
+__device__ __forceinline__ void team_stage(const float2* src, float2* dst, const float2* w, int tid) {
+  using T = Team<M>;
+  using G = TeamStage<M, RX>;
+#pragma unroll
+  for (int q = 0; q < G::BPT; ++q) {
+    const int t = tid + q * T::NT, b = t / (M / RX), j = t % (M / RX);
+    if (G::ALL || t < G::NB) {
+      float2 v[RX];
+#pragma unroll
+      for (int r = 0; r < RX; ++r) v[r] = src[b * T::P + j + r * (M / RX)];
+      if (NS > 1) {
+#pragma unroll
+        for (int r = 1; r < RX; ++r)
+          v[r] = cmul(v[r], INV ? cconj(w[q * (RX - 1) + r - 1]) : w[q * (RX - 1) + r - 1]);
+      }
+      Dft<RX, INV>::run(v);
+      const int idx = (j / NS) * NS * RX + (j % NS);
+#pragma unroll
+      for (int r = 0; r < RX; ++r) dst[b * T::P + idx + r * NS] = v[r];
+    }
+  }
+  __syncthreads();
+}
+template <int M, int RX, int NS>
+__device__ __forceinline__ void team_twiddles(float2* w, const float2* __restrict__ tw, int tid) {
+  using T = Team<M>;
+#pragma unroll
+  for (int q = 0; q < TeamStage<M, RX>::BPT; ++q) {
+    const int j = (tid + q * T::NT) % (M / RX);
+#pragma unroll
+    for (int r = 1; r < RX; ++r) w[q * (RX - 1) + r - 1] = tw[((j % NS) * r * (PTYK_TWN / (NS * RX))) & (PTYK_TWN - 1)];
+  }
+}
+// Twiddles of stages 1.. of this thread (the same for rows and columns, conjugated for the inverse).
+template <int M>
+struct TeamTw {
+  using T = Team<M>;
+  float2 a[TeamStage<M, T::R1>::NW], b[TeamStage<M, T::R2>::NW], c[TeamStage<M, T::R3>::NW];
+  __device__ __forceinline__ void load(const float2* __restrict__ tw, int tid) {
+    team_twiddles<M, T::R1, T::R0>(a, tw, tid);
+    if constexpr (T::S > 2) team_twiddles<M, T::R2, T::R0 * T::R1>(b, tw, tid);
+    if constexpr (T::S > 3) team_twiddles<M, T::R3, T::R0 * T::R1 * T::R2>(c, tw, tid);
+  }
+};
+// R sequences from tile t0, with t1 as the other tile; returns the tile that holds the result (t0
+// where the number of stages is even).
+template <int M, bool INV>
+__device__ __forceinline__ float2* team_fft(float2* t0, float2* t1, const TeamTw<M>& w, int tid) {
+  using T = Team<M>;
+  __syncthreads();
+  team_stage<M, T::R0, 1, INV>(t0, t1, nullptr, tid);
+  team_stage<M, T::R1, T::R0, INV>(t1, t0, w.a, tid);
+  if constexpr (T::S == 2) return t0;
+  if constexpr (T::S > 2) team_stage<M, T::R2, T::R0 * T::R1, INV>(t0, t1, w.b, tid);
+  if constexpr (T::S > 3) {
+    team_stage<M, T::R3, T::R0 * T::R1 * T::R2, INV>(t1, t0, w.c, tid);
+    return t0;
+  }
+  return t1;
+}
+
+// Psi' - Psi / M^2 of one mode: f (A / |f| - 1) nrm, parallel to f whatever the rounding of its factor;
+// outside the range in which |f|^2 is safe in 32 bits (zero, infinities and NaN among it) the phase
+// form of the projection decides.
+__device__ __forceinline__ float2 modulus_delta(float2 f, float a, float nrm) {
+  const float s = fmaxf(fabsf(f.x), fabsf(f.y));
+  if (!(s > 1e-18f && s < 1e18f)) return csub(modulus_phase(f, a, nrm), cscale(f, nrm));
+  return cscale(f, (a * rsqrtf(f.x * f.x + f.y * f.y) - 1.f) * nrm);
+}
+
+// MULTI: k_use modes, one after another in each step; the first k_res of them keep their spectra in
+// LDS tiles of their own through the column step, the others in the exchange buffer, and all keep
+// psi - psi_old in a.psi_old until the probe update.  Otherwise one mode, whose probe rows and
+// psi - psi_old stay in registers.
+template <int M, bool MULTI>
+__global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
+  using T = Team<M>;
+  constexpr int W = T::W, NT = T::NT, R = T::R, P = T::P, PPT = T::PPT, MM = M * M, CR = R * R;
+  constexpr bool ODD = T::S % 2 == 1;  // a transform ends in the other tile
+  extern __shared__ float2 lds[];
+  float2* const t0 = lds;
+  float2* const t1 = lds + T::TILE;              // also stages the object window
+  float2* const res = lds + T::TILE + T::TILE_B;  // k_res tiles
   __shared__ double redd[NT / 64];
-  __shared__ long redi[NT / 64];
-  constexpr int MM = M * M;
-  constexpr int PPT = MM / NT;
-  static_assert(MM % NT == 0, "pixels must divide among the threads");
-  const int tid = threadIdx.x;
+  __shared__ unsigned rowm[R], value[3];  // row maxima; values sent with the three barriers
+  __shared__ float most[3];               // largest values received with them
+  __shared__ int gone;
+  const int tid = threadIdx.x, w = blockIdx.x, lane = tid & 63;
+  const int ku = MULTI ? a.k_use : 1;
+  const int px0 = w * R * M;  // first frame pixel of this workgroup's rows
+  const float nrm = 1.f / (float)MM;
+  unsigned long long* const flags = a.team_flags;
+  unsigned epoch = a.team_epoch;
+  if (tid < 3) value[tid] = 0u;
+  if (tid == 0) gone = 0;
+
+  TeamTw<M> tw;
+  tw.load(a.tw, tid);
   float obj_max = (float)a.scal[0];
   float probe_max = (float)a.scal[1];
+  float2 pv[PPT];
+#pragma unroll
+  for (int j = 0; j < PPT; ++j) pv[j] = a.probe[px0 + tid + j * NT];
+  // modes that take no part keep their intensities, which count in the probe maximum
+  float rest = 0.f;
+  if (a.update_probe && !a.modal)
+    for (int k = ku; k < a.k_total; ++k)
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) rest = fmaxf(rest, a.probe_int[(long)k * MM + px0 + tid + j * NT]);
+  // max |O|^2 of every canvas row, kept up to date per position
+  if (a.update_probe)
+    for (int r = w + W * (tid >> 6); r < a.obj_rows; r += W * (NT / 64)) {
+      const float* row = a.obj_int + (long)r * a.obj_cols;
+      float m = 0.f;
+      for (int c = lane; c < a.obj_cols; c += 64) m = fmaxf(m, row[c]);
+      m = wave_max_pos(m);
+      if (lane == 0) st_dev(a.team_rowmax + r, m);
+    }
   double err = 0.0;
-  const long canvas = (long)a.obj_rows * a.obj_cols;
-  const float nrm = 1.f / (float)MM;
-  for (int i = tid; i < PTYK_TWN; i += NT) tws[i] = a.tw[i];
-  // where the current obj_max is attained (valid while the probe is updated)
-  long max_at = 0;
-  if (a.update_probe) {
-    const MaxAt m = canvas_max<NT>(a.obj_int, canvas, redf, redi);
-    obj_max = m.v;
-    max_at = m.at;
-  }
+
+  // What a position needs as soon as the one before has left the object: the window behind the rows'
+  // ROI, and beside the ROI the start of its rows' |O|^2.
+  float2 win[T::WU];
+  float beside[4];
+  const int nout = a.obj_cols - M, brow = tid / T::TPR, bcol = tid % T::TPR;
+  auto load_object = [&](float2 pos) __attribute__((always_inline)) {
+    const int ib = (int)floorf(pos.x) + w * R, jb = (int)floorf(pos.y);
+#pragma unroll
+    for (int u = 0; u < T::WU; ++u) {
+      const int e = min(tid + u * NT, T::WIN - 1);
+      const int r = min(max(ib + e / T::WC, 0), a.obj_rows - 1), c = min(max(jb + e % T::WC, 0), a.obj_cols - 1);
+      win[u] = ld_dev(a.obj + (long)r * a.obj_cols + c);
+    }
+    if (a.update_probe && nout > 0) {
+      const int ry = (int)roundf(pos.y);
+      const float* row = a.obj_int + (long)((int)roundf(pos.x) + w * R + brow) * a.obj_cols;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = min(bcol + u * T::TPR, nout - 1);
+        beside[u] = ld_dev(row + (c < ry ? c : c + M));
+      }
+    }
+  };
+  // amplitudes of the column step: PPT consecutive columns of one frame row, loaded a position ahead
+  const int crow = tid / (R / PPT), ccol = tid % (R / PPT) * PPT;
+  struct alignas(2 * PPT) Halves { __half h[PPT]; };
+  auto load_amps = [&](int f) __attribute__((always_inline)) {
+    return *reinterpret_cast<const Halves*>(a.amp + (long)f * MM + (long)crow * M + w * R + ccol);
+  };
+  int fi = a.order[0];
+  float2 pos = a.pos[fi];
+  load_object(pos);
+  Halves ah = load_amps(fi);
+  team_arrive(flags, w, ++epoch, value);  // the row maxima are there
+  if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[0])) return;
 
   for (int s = 0; s < a.n_pos; ++s) {
-    const int fi = a.order[s];
-    const float2 pos = a.pos[fi];
     const float ascale = a.amp_scale[fi];
-    const __half* amp = a.amp + (long)fi * MM;
-
-    const int ib = (int)floorf(pos.x), jb = (int)floorf(pos.y);
-    load_window<M, NT>(a, ib, jb, lds);
-    __syncthreads();
-    {
-      float2 po[PPT];
-      if (a.tex_quantize)
-        epie_roi<M, NT, PPT, true>(a, pos, ib, jb, lds, po);
-      else
-        epie_roi<M, NT, PPT, false>(a, pos, ib, jb, lds, po);
-      __syncthreads();
-      const int t = lane();
+    const int rx = (int)roundf(pos.x), ry = (int)roundf(pos.y);
+    if (tid < R) rowm[tid] = 0u;
+    // ---- rows: ROI x P_k, row transform
 #pragma unroll
-      for (int j = 0; j < PPT; ++j) lds[at<M>(t + j * NT)] = po[j];
+    for (int u = 0; u < T::WU; ++u) {
+      const int e = tid + u * NT;
+      if (e < T::WIN) t1[e] = win[u];
     }
     __syncthreads();
-    fft_lds<M, false, M, NT, RowLayout<M, P>, true>(lds, tws, lane());
-    fft_lds<M, false, M, NT, ColLayout<P>, true>(lds, tws, lane());
-    // The modulus step leaves Psi' - Psi / M^2 in place of Psi, so the inverse transform yields
-    // psi - psi_old directly (the transform is linear) and psi_old need not be kept. The optional
-    // Fourier error (PhaserUtil::calculateER, ePIE.cpp:124-125) is of psi_old's spectrum, which
-    // is Psi itself: it is summed here instead of by a third transform.
+    float2 roi[PPT], oo[PPT];  // bilinear ROI; object at the rounded position
     {
-      const int t = lane();
-      __half ah[PPT];
+      const int ib = (int)floorf(pos.x), jb = (int)floorf(pos.y);
 #pragma unroll
-      for (int j = 0; j < PPT; ++j) ah[j] = amp[t + j * NT];
+      for (int j = 0; j < PPT; ++j) {
+        const int e = tid + j * NT, lr = e / M, c = e % M, row = w * R + lr;
+        const float u = (float)c + pos.y + 0.5f, v = (float)row + pos.x + 0.5f;
+        const TapPos q = a.tex_quantize ? tap_pos<true>(u, v) : tap_pos<false>(u, v);
+        const int wr = min(max(q.j0 - ib - w * R, 0), R), wc = min(max(q.i0 - jb, 0), M);
+        const float2* x = t1 + wr * T::WC + wc;
+        roi[j] = bilinear_sum(q.al, q.be, x[0], x[1], x[T::WC], x[T::WC + 1]);
+        oo[j] = t1[(lr + rx - ib) * T::WC + c + ry - jb];
+      }
+    }
+    for (int k = 0; k < ku; ++k) {
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        const int e = tid + j * NT;
+        t0[e / M * P + e % M] = cmul(pv[j], roi[j]);
+      }
+      if (MULTI) {  // the next mode's rows (the first one's again after the last)
+        const float2* p = a.probe + (long)(k + 1 < ku ? k + 1 : 0) * MM + px0;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) pv[j] = p[tid + j * NT];
+      }
+      const float2* f = team_fft<M, false>(t0, t1, tw, tid);
+      float2* x = a.psi + (long)k * MM;
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {  // blocks of R columns x R rows, one per owner of the columns
+        const int e = tid + j * NT, v = e / CR, c = e / R % R, r = e % R;
+        st_dev(x + (v * W + w) * CR + e % CR, f[r * P + v * R + c]);
+      }
+      if (MULTI) __syncthreads();
+    }
+    team_arrive(flags, w, ++epoch, value);
+    // meanwhile: max |O|^2 of this workgroup's ROI rows beside the ROI and of the rows above and below
+    // it, which no one changes now
+    float omax = 0.f;
+    if (a.update_probe) {
+      if (nout > 0) {
+        float m = fmaxf(fmaxf(beside[0], beside[1]), fmaxf(beside[2], beside[3]));
+        const float* row = a.obj_int + (long)(rx + w * R + brow) * a.obj_cols;
+        for (int c0 = bcol + T::TPR * 4; c0 < nout; c0 += T::TPR * 8) {
+          float v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int c = min(c0 + T::TPR * u, nout - 1);
+            v[u] = ld_dev(row + (c < ry ? c : c + M));
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
+        }
+        m = max_dpp<0x141>(max_dpp<0x4E>(max_dpp<0xB1>(m)));  // over 8 lanes, of one row
+        if (tid % 8 == 0) atomicMax(&rowm[brow], __float_as_uint(fmaxf(m, 0.f)));
+      }
+      const int nrow = a.obj_rows - M;  // by every wave for itself
+      for (int r0 = lane; r0 < nrow; r0 += 64 * 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = min(r0 + 64 * u, nrow - 1);
+          v[u] = ld_dev(a.team_rowmax + (r < rx ? r : r + M));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) omax = fmaxf(omax, v[u]);
+      }
+      omax = wave_max_pos(omax);
+    }
+    if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[0])) return;
+    if (a.update_probe && s > 0) probe_max = most[0];
+
+    // ---- columns
+    float ms[PPT];
+    float2 sm[PPT];
+    if (MULTI) {
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        ms[j] = 0.f;
+        sm[j] = make_float2(0.f, 0.f);
+      }
+    }
+    float2* const xc = a.psi + (long)w * R * M;  // this workgroup's columns (mode 0)
+    float2 g[PPT];
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) g[j] = ld_dev(xc + tid + j * NT);
+    for (int k = 0; k < ku; ++k) {
+      float2* x = xc + (long)k * MM;
+      // a resident mode's spectrum has to end in its own tile
+      float2* const own = MULTI && k < a.k_res ? res + k * T::TILE : (ODD ? t1 : t0);
+      float2* const in = ODD ? t0 : own;
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        const int e = tid + j * NT;
+        in[e / R % R * P + e / CR * R + e % R] = g[j];
+      }
+      if (MULTI && k + 1 < ku) {
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) g[j] = ld_dev(x + MM + tid + j * NT);
+      }
+      float2* f = team_fft<M, false>(in, ODD ? own : t1, tw, tid);
+      if (MULTI) {
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const float2 v = f[(ccol + j) * P + crow];
+          ms[j] += cabs2(v);
+          sm[j] = cadd(sm[j], v);
+          if (k >= a.k_res) st_dev(x + tid + j * NT, v);  // its own slots: only this thread reads them back
+        }
+        __syncthreads();
+      } else {
+        double acc = 0.0;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          float2* v = f + (ccol + j) * P + crow;
+          const float A = __half2float(ah.h[j]) * ascale;
+          if (a.rms) acc += fabs((double)A - sqrt((double)v->x * v->x + (double)v->y * v->y));
+          *v = modulus_delta(*v, A, nrm);
+        }
+        if (a.rms) err += acc / (double)a.amp_sum[fi];
+        f = team_fft<M, true>(f, f == t0 ? t1 : t0, tw, tid);
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const int e = tid + j * NT;
+          st_dev(x + e, f[e / R % R * P + e / CR * R + e % R]);
+        }
+      }
+    }
+    if (MULTI) {
       double acc = 0.0;
 #pragma unroll
       for (int j = 0; j < PPT; ++j) {
-        const int q = at<M>(t + j * NT);
-        const float2 f = lds[q];
-        const float A = __half2float(ah[j]) * ascale;
-        if (a.rms) acc += fabs((double)A - sqrt((double)f.x * f.x + (double)f.y * f.y));
-        lds[q] = csub(modulus_unit(f, A, nrm), cscale(f, nrm));
+        const float A = __half2float(ah.h[j]) * ascale;
+        if (a.rms) acc += fabs((double)A - sqrt((double)sm[j].x * sm[j].x + (double)sm[j].y * sm[j].y));
+        ms[j] = A * rsqrtf(ms[j]) * nrm - nrm;
       }
-      if (a.rms) {
-        acc = block_sum<NT>(acc, redd);
-        err += acc / (double)a.amp_sum[fi];
-      }
-    }
-    __syncthreads();
-    fft_lds<M, true, M, NT, RowLayout<M, P>, true>(lds, tws, lane());
-    fft_lds<M, true, M, NT, ColLayout<P>, true>(lds, tws, lane());
-
-    const int rx = (int)roundf(pos.x), ry = (int)roundf(pos.y);
-    const float co = (float)(1.0 / (double)probe_max);
-    const MaxAt mo = a.phase_constraint ? epie_obj_update<M, NT, PPT, true>(a, rx, ry, co, lds)
-                                        : epie_obj_update<M, NT, PPT, false>(a, rx, ry, co, lds);
-    __syncthreads();
-
-    // the probe update needs max |O|^2 after this position, which otherwise is only reported
-    // after the last one
-    if (a.update_probe) {
-      const long mr = max_at / a.obj_cols, mc = max_at % a.obj_cols;
-      if (mr >= rx && mr < rx + M && mc >= ry && mc < ry + M) {
-        const MaxAt m = canvas_max<NT>(a.obj_int, canvas, redf, redi);
-        obj_max = m.v;
-        max_at = m.at;
-      } else {
-        const float m = block_max<NT>(mo.v, redf);
-        if (m > obj_max) {
-          // a location of the new maximum: the lowest index among the threads that hold it
-          long cand = mo.v == m ? mo.at : canvas;
+      if (a.rms) err += acc / ku / (double)a.amp_sum[fi];
+      for (int k = 0; k < ku; ++k) {
+        float2* x = xc + (long)k * MM;
+        float2* const in = k < a.k_res ? res + k * T::TILE : t0;
 #pragma unroll
-          for (int o = 32; o > 0; o >>= 1) cand = min(cand, (long)__shfl_xor(cand, o, 64));
-          if ((tid & 63) == 0) redi[tid >> 6] = cand;
-          __syncthreads();
-          long best = redi[0];
-#pragma unroll
-          for (int i = 1; i < NT / 64; ++i) best = min(best, redi[i]);
-          __syncthreads();
-          obj_max = m;
-          max_at = best;
+        for (int j = 0; j < PPT; ++j) {
+          float2* v = in + (ccol + j) * P + crow;
+          *v = cscale(k < a.k_res ? *v : ld_dev(x + tid + j * NT), ms[j]);
         }
+        const float2* f = team_fft<M, true>(in, t1, tw, tid);
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const int e = tid + j * NT;
+          st_dev(x + e, f[e / R % R * P + e / CR * R + e % R]);
+        }
+        __syncthreads();
       }
-      const float cp = (float)(1.0 / (double)obj_max);
-      float mx = epie_probe_update<M, NT, PPT>(a, cp, lds);
-      // the other (unused) modes keep their intensities
-      for (long q = MM + lane(); q < (long)a.k_total * MM; q += NT) mx = fmaxf(mx, a.probe_int[q]);
-      probe_max = block_max<NT>(mx, redf);
     }
+    team_arrive(flags, w, ++epoch, value + 1);
+    const float co = (float)(1.0 / (double)probe_max);
+    // next position
+    const int fn = s + 1 < a.n_pos ? a.order[s + 1] : fi;
+    const float2 posn = a.pos[fn];
+    ah = load_amps(fn);
+    if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[1])) return;
 
-    __syncthreads();
-  }
-  if (!a.update_probe && a.n_pos > 0) obj_max = canvas_max<NT>(a.obj_int, canvas, redf, redi).v;
-  if (a.update_probe && a.n_pos > 0) {
-    // each thread rereads only the probe pixels it wrote itself
-    const int t = lane();
+    // ---- rows: psi - psi_old, object update at the rounded position (d_updateObjectArray(M))
+    float2 d[PPT], up[PPT];
+    const float2* const xr = a.psi + w * CR;
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-      const float2 p = a.probe[t + j * NT];
-      const float ia = sqrtf(p.x * p.x + p.y * p.y);
-      a.probe_int[t + j * NT] = ia * ia;
+      const int e = tid + j * NT;
+      g[j] = ld_dev(xr + e / CR * W * CR + e % CR);
     }
+    for (int k = 0; k < ku; ++k) {
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        const int e = tid + j * NT;
+        t0[e % R * P + e / CR * R + e / R % R] = g[j];
+      }
+      if (MULTI && k + 1 < ku) {
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const int e = tid + j * NT;
+          g[j] = ld_dev(xr + (long)(k + 1) * MM + e / CR * W * CR + e % CR);
+        }
+      }
+      const float2* f = team_fft<M, true>(t0, t1, tw, tid);
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        const int e = tid + j * NT;
+        d[j] = f[e / M * P + e % M];
+        const float2 t = cconj(cmulcj(d[j], pv[j]));
+        up[j] = MULTI && k ? cadd(up[j], t) : t;
+        if (MULTI) {
+          a.psi_old[(long)k * MM + px0 + e] = d[j];
+          pv[j] = a.probe[(long)(k + 1 < ku ? k + 1 : 0) * MM + px0 + e];
+        }
+      }
+      if (MULTI) __syncthreads();
+    }
+    float2 on[PPT];
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+      const int e = tid + j * NT, lr = e / M;
+      const long oi = (long)(rx + w * R + lr) * a.obj_cols + (ry + e % M);
+      float2 o = cadd(oo[j], cscale(up[j], co));
+      const float mag = sqrtf(o.x * o.x + o.y * o.y);
+      if (a.phase_constraint) o = clamp_phase(o);
+      st_dev(a.obj + oi, o);
+      st_dev(a.obj_int + oi, mag * mag);
+      on[j] = o;
+      if (a.update_probe) {  // a wave's 64 pixels lie in one row
+        const float m = wave_max_pos(fmaxf(mag * mag, 0.f));
+        if (lane == 0) atomicMax(&rowm[lr], __float_as_uint(m));
+      }
+    }
+    if (a.update_probe) {
+      __syncthreads();
+      if (tid < R) {
+        const unsigned m = rowm[tid];
+        st_dev(a.team_rowmax + rx + w * R + tid, __uint_as_float(m));
+        atomicMax(&value[2], m);
+      }
+    }
+    team_arrive(flags, w, ++epoch, value + 2);
+    if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[2])) return;
+    load_object(posn);
+
+    // ---- probe update with the updated object (d_updateProbe(M)), own rows
+    if (a.update_probe) {
+      obj_max = fmaxf(omax, most[2]);
+      if (tid == 0) value[0] = value[2] = 0u;  // both sent; set again after the barriers below
+      const float cp = (float)(1.0 / (double)obj_max);
+      float pm = rest, im[PPT];
+      for (int k = 0; k < ku; ++k) {
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const long q = (long)k * MM + px0 + tid + j * NT;
+          if (MULTI) {
+            const float2 p = cadd(cscale(cmulcj(on[j], a.psi_old[q]), cp), a.probe[q]);
+            a.probe[q] = p;
+            if (k == 0) pv[j] = p;
+            const float ia = sqrtf(p.x * p.x + p.y * p.y);
+            im[j] = k ? im[j] + ia * ia : ia * ia;
+          } else {
+            pv[j] = cadd(cscale(cmulcj(on[j], d[j]), cp), pv[j]);
+            const float ia = sqrtf(pv[j].x * pv[j].x + pv[j].y * pv[j].y);
+            im[j] = ia * ia;
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) pm = fmaxf(pm, im[j]);
+      pm = wave_max_pos(pm);
+      __syncthreads();  // value[0] is cleared
+      if (lane == 0) atomicMax(&value[0], __float_as_uint(pm));
+    }
+    fi = fn;
+    pos = posn;
   }
+
+  // ---- state: probe, its intensities, maxima, error
+  if (a.update_probe) {
+    for (int k = 0; k < ku; ++k)
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        const long q = (long)k * MM + px0 + tid + j * NT;
+        const float2 p = MULTI ? a.probe[q] : pv[j];
+        if (!MULTI) a.probe[q] = p;
+        const float ia = sqrtf(p.x * p.x + p.y * p.y);
+        a.probe_int[q] = ia * ia;
+      }
+  } else {
+    const long canvas = (long)a.obj_rows * a.obj_cols;
+    float m = 0.f;
+    for (long q = (long)w * NT + tid; q < canvas; q += (long)W * NT) m = fmaxf(m, ld_dev(a.obj_int + q));
+    m = wave_max_pos(m);
+    if (lane == 0) atomicMax(&value[0], __float_as_uint(m));
+  }
+  err = block_sum<NT>(err, redd);
+  if (tid == 0) __hip_atomic_store(a.team_err + w, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  team_arrive(flags, w, ++epoch, value);
+  if (w != 0) return;
+  if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[0])) return;
   if (tid == 0) {
-    a.scal[0] = obj_max;
-    a.scal[1] = probe_max;
-    a.scal[2] = err;
+    double e = 0.0;
+    for (int i = 0; i < W; ++i) e += __hip_atomic_load(a.team_err + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    a.scal[0] = a.update_probe ? obj_max : most[0];
+    a.scal[1] = a.update_probe ? most[0] : probe_max;
+    a.scal[2] = e;
+    a.scal[PTYK_EPIE_DONE] = a.team_epoch;  // the whole chain ran
   }
 }
 
@@ -552,27 +841,41 @@ static hipError_t epie_impl(const EpieArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Frames whose exit wave fits in LDS take the resident form (single mode only).
-template <int M, int NT>
-static hipError_t epie_lds_impl(const EpieArgs& a, hipStream_t s) {
-  const size_t lds = (size_t)((M + 2) * (M + 2) + PTYK_TWN) * sizeof(float2);
-  hipError_t e = hipFuncSetAttribute((const void*)k_epie_lds<M, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+template <int M, bool MULTI>
+static hipError_t epie_team_launch(EpieArgs a, hipStream_t s) {
+  using T = Team<M>;
+  constexpr size_t base = (size_t)(T::TILE + T::TILE_B) * sizeof(float2), tile = (size_t)T::TILE * sizeof(float2);
+  constexpr size_t room = 128 * 1024;  // of the CU's 160 KiB, beside the static arrays
+  a.k_res = MULTI ? (int)std::min<size_t>(a.k_use, (room - base) / tile) : 0;
+  const size_t lds = base + a.k_res * tile;
+  hipError_t e = hipFuncSetAttribute((const void*)k_epie_team<M, MULTI>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_epie_lds<M, NT>), dim3(1), dim3(NT), lds, s, a);
+  hipLaunchKernelGGL((k_epie_team<M, MULTI>), dim3(T::W), dim3(T::NT), lds, s, a);
   return hipGetLastError();
 }
+template <int M>
+static hipError_t epie_team_impl(const EpieArgs& a, hipStream_t s) {
+  if (a.team_size == 0) return epie_impl<M>(a, s);
+  return a.k_use > 1 ? epie_team_launch<M, true>(a, s) : epie_team_launch<M, false>(a, s);
+}
+
+// 0 where one workgroup takes the frame: below 64^2, and where the device (a partition of the part)
+// has fewer CUs than the team has workgroups.
+int epie_team_size(int m, int cus) {
+  const int w = m == 64 ? Team<64>::W : m == 128 ? Team<128>::W : m == 256 ? Team<256>::W : m == 512 ? Team<512>::W : 0;
+  return w <= cus ? w : 0;
+}
+unsigned epie_team_barriers(int n_pos) { return 3u * (unsigned)n_pos + 2u; }
 
 hipError_t epie_iteration(const EpieArgs& a, hipStream_t s) {
-  if (a.k_use == 1 && a.m == 128) return epie_lds_impl<128, 1024>(a, s);
-  if (a.k_use == 1 && a.m == 64) return epie_lds_impl<64, 512>(a, s);
   switch (a.m) {
     case 16: return epie_impl<16>(a, s);
     case 32: return epie_impl<32>(a, s);
-    case 64: return epie_impl<64>(a, s);
-    case 128: return epie_impl<128>(a, s);
-    case 256: return epie_impl<256>(a, s);
-    case 512: return epie_impl<512>(a, s);
+    case 64: return epie_team_impl<64>(a, s);
+    case 128: return epie_team_impl<128>(a, s);
+    case 256: return epie_team_impl<256>(a, s);
+    case 512: return epie_team_impl<512>(a, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -202,7 +202,17 @@ struct EpieArgs {
   const float2* tw;
   int n_pos, m, k_use, k_total, obj_rows, obj_cols;
   int phase_constraint, update_probe, modal, rms, tex_quantize;
+  // team form (team_size = epie_team_size(m, CUs) > 0): barrier flags, row maxima of |O|^2 and the
+  // workgroups' errors; the flags stand at team_epoch and move by epie_team_barriers(n_pos);
+  // team_limit bounds a barrier's wait (ticks of the 100 MHz clock); k_res is set by the launch
+  unsigned long long* team_flags; float* team_rowmax; double* team_err;
+  unsigned team_epoch; int team_size, k_res; long long team_limit;
 };
+#define PTYK_EPIE_TEAM_MAX 128                     // workgroups of the largest team
+#define PTYK_EPIE_FLAG_STRIDE 16                   // flags (epoch, value) of one team: one 128-byte line each
+#define PTYK_EPIE_DONE PTYK_SCAL_COUNT             // scal slot the team form sets to team_epoch when the iteration ran
+int epie_team_size(int m, int cus);                // workgroups that share a frame; 0: one workgroup
+unsigned epie_team_barriers(int n_pos);
 hipError_t epie_iteration(const EpieArgs& a, hipStream_t s);
 
 // ---- MLs (maximum likelihood with least-squares steps), ptyk_mls.hip.

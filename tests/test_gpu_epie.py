@@ -1,7 +1,7 @@
 """ePIE iteration on the GPU against the FP64 oracle (same state, same position order).
 
-Single-mode 64^2 and 128^2 frames run the LDS-resident form (the exit wave held in LDS, the
-canvas maximum tracked by location); 16^2 / 32^2 frames and the modal form run the staged form.
+Frames of 64^2 and more are shared by a team of workgroups; 16^2 and 32^2 frames run on one
+workgroup with the exit waves staged through LDS.
 Both are checked, with and without texture-weight quantisation, with a second (unused) probe mode
 whose intensities enter the probe maximum, and in the modal form."""
 import numpy as np
@@ -114,3 +114,79 @@ def test_modal_epie_matches_oracle(gpu, orc, m, seed):
         assert np.abs(e.get_probe()[1]).max() > 0
         for rms in (False, True):
             _check(e, orc, p, amp, rng.permutation(p["n"]), modal | (E.FLAG_RMS if rms else 0), k_use=2, modal=True)
+
+
+def _near_engine(p, amp=None):
+    """An engine a few steps from the truth (spectra well above rounding wherever counts are)."""
+    from ptychopy_amd import _engine as E
+    rng = np.random.default_rng(3)
+    e = E.Engine(p["n"], p["m"], p["shape"], n_modes=p["k"])
+    e.set_frames(p["amp"] if amp is None else amp)
+    e.set_positions(p["pos"])
+    e.set_object((0.95 * p["obj"]).astype(np.complex64))
+    modes = [p["probe"]] + [0.4 * p["probe"] * (rng.standard_normal(p["probe"].shape) + 1j) for _ in range(p["k"] - 1)]
+    modes = np.array(modes) * np.exp(0.5j * rng.standard_normal(p["probe"].shape))
+    if p["k"] > 1:
+        e.set_probe(modes)
+        e.begin_modal()
+    e.set_probe(modes)
+    e.refresh_maxima()
+    s = e.get_scalars()
+    s[E.SCAL_PROBE_MAX] = float((np.abs(e.get_probe().astype(np.complex128)) ** 2).sum(axis=0).max())
+    e.set_scalars(s)
+    return e
+
+
+def _flat_counts(p):
+    """Amplitudes without dark pixels: the model's own spectrum is nowhere decided by rounding alone."""
+    return (p["amp"] + 0.05 * p["amp"].mean(axis=(1, 2), keepdims=True) + 1.0).astype(np.float32)
+
+
+@pytest.mark.parametrize("m,n_side,step,modes,rms,pc", [
+    (64, 1, 5.0, 1, True, False),     # one position: the canvas is hardly larger than the ROI
+    (64, 3, 150.3, 2, False, True),   # canvas rows and columns far beyond the ROI
+    (128, 2, 331.7, 3, True, False),
+    (256, 2, 40.2, 1, True, True),
+    (256, 2, 21.9, 4, True, False),
+    (512, 2, 33.3, 1, False, False),
+    (512, 2, 27.1, 3, True, False),   # more modes than LDS tiles
+])
+def test_team_iterations_match_oracle(gpu, orc, m, n_side, step, modes, rms, pc):
+    """Frames shared by a team of workgroups: sizes, modes in and out of LDS, small and wide canvases."""
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=m, n_side=n_side, step=step, seed=m + modes, modes=modes, photons=100.0 * m * m)
+    rng = np.random.default_rng(m)
+    flags = E.FLAG_UPDATE_PROBE | (E.FLAG_RMS if rms else 0) | (E.FLAG_UPDATE_MODES if modes > 1 else 0)
+    with _near_engine(p, _flat_counts(p)) as e:
+        amp = e.get_frames().astype(np.float64)
+        kw = dict(k_use=modes, modal=modes > 1)
+        _check(e, orc, p, amp, rng.permutation(p["n"]), flags, **kw)
+        _check(e, orc, p, amp, rng.permutation(p["n"]),
+               (flags & ~E.FLAG_UPDATE_PROBE) | (E.FLAG_PHASE_CONSTRAINT if pc else 0), **kw)
+        _check(e, orc, p, amp, rng.permutation(p["n"]), flags, **kw)
+
+
+def test_teams_of_several_threads_give_their_own_results(gpu):
+    """More teams at once than the device holds: each handle's result is the one it gives alone."""
+    import threading
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=256, n_side=2, step=30.0, seed=5)
+    orders = [np.random.default_rng(i).permutation(p["n"]) for i in range(6)]
+
+    def go(out, i):
+        with _near_engine(p) as e:
+            for _ in range(3):
+                e.epie_iteration(orders[i], E.FLAG_UPDATE_PROBE)
+            out[i] = (e.get_object(), e.get_probe())
+
+    alone, together = {}, {}
+    for i in range(6):
+        go(alone, i)
+    ts = [threading.Thread(target=go, args=(together, i)) for i in range(6)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for i in range(6):
+        for a, b in zip(alone[i], together[i]):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
