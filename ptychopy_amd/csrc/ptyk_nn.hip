@@ -2,16 +2,18 @@
 // c, 2c, 4c, 8c with c = 32 by default) mapping a log-scaled diffraction amplitude (1 x S x S)
 // to the object patch's amplitude and phase (2 x S x S).  No reference counterpart.
 //
-// Every convolution is an implicit GEMM on the matrix cores: v_mfma_f32_16x16x32_bf16 with BF16
-// operands and FP32 accumulation, operands gathered straight from the activation tensors (no
-// im2col buffer).  One templated kernel covers the forward pass (M = Cout, N = pixels,
-// K = Cin * ks^2), the data gradient (M = Cin, N = pixels, K = Cout * ks^2) and the weight
-// gradient (M = Cout, N = Cin * ks^2, K = pixels, split over K into partial tiles summed in a
-// fixed order).  Activations are BF16, gradients FP32 (rounded to BF16 where they enter a GEMM),
-// master weights FP32 with Adam.  Tensors are NCHW views with a channel stride, so the decoder's
-// skip concatenations are channel ranges of one buffer.
+// Tensors are pixel-major (NHWC) with the channels padded to a multiple of 32 by zeros, so that the
+// 8 channels a lane feeds to a matrix instruction are 16 contiguous bytes.  Every 3 x 3 convolution
+// between them is an implicit GEMM on v_mfma_f32_32x32x16_bf16 (BF16 operands, FP32 accumulation;
+// no im2col buffer): k_conv3 for the forward pass and the data gradient, k_wgrad3 for the weight
+// gradient (split over pixels into partial tiles summed in a fixed order).  The first layer (one
+// input channel) and the last (1 x 1 to two channels) are bound by memory and run on the vector
+// units.  Activations are BF16, gradients FP32 (rounded to BF16 where they enter a product), master
+// weights FP32 with Adam.  Skip concatenations and nearest upsampling are never stored: a layer's
+// input is up to two tensors, one of which may be read at half resolution.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <random>
@@ -25,484 +27,771 @@
 namespace ptyk {
 
 typedef __bf16 bf16;
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16;
 
 namespace {
 
-constexpr int GT = 256;  // threads per GEMM block (4 waves)
-constexpr int TM = 64, TN = 64, TK = 32;
-constexpr int LDP = TK + 8;  // LDS row pitch (bf16) of the A and transposed-B tiles
-constexpr int BIAS_PARTS = 256;  // slices of the bias-gradient reduction per channel
-
-// NCHW view: element (b, c, y, x) at p[((b * ctot) + c) * hw + y * w + x]; p already offset to
-// the view's first channel.
-struct View {
-  void* p;
-  int c, ctot, h, w;
-};
-
-enum { GEMM_FWD = 0, GEMM_BWD_DATA = 1, GEMM_BWD_W = 2 };
-
-struct GemmArgs {
-  View x;        // FWD: input activation (bf16); BWD_DATA: dZ (f32); BWD_W: input activation (bf16)
-  View y;        // FWD: output (bf16, or f32 when out_f32); BWD_DATA: dX (f32); BWD_W: dZ (f32)
-  const bf16* wt;      // weights Cout x Cin x ks x ks (bf16)
-  const float* bias;   // FWD
-  float* partial;      // BWD_W: chunks x M x N
-  int batch, cin, cout, relu, out_f32;
-  int M, N, K, kchunk;
-  int w_sh, hw_sh;     // log2 of the image width and of the pixels per image (powers of two)
-  int vec_a;           // FWD: weight rows 16-byte aligned and K % 8 == 0 (8 bf16 per load)
-};
+constexpr int CT = 256;      // threads of the convolution kernels (4 waves)
+constexpr int NN_LAYERS = 15;
+inline int pad32(int c) { return (c + 31) / 32 * 32; }
 
 __device__ __forceinline__ bf16 to_bf(float v) { return (bf16)v; }
+__device__ __forceinline__ unsigned bf_bits(float v) { return __builtin_bit_cast(u16, to_bf(v)); }
+__device__ __forceinline__ float bf_val(unsigned bits16) { return __uint_as_float(bits16 << 16); }
+__device__ __forceinline__ unsigned bf_pair(float a, float b) { return bf_bits(a) | (bf_bits(b) << 16); }
 
-// A(m, k) for BWD_DATA and BWD_W (FWD reads the weight rows directly)
-template <int MODE, int KS>
-__device__ __forceinline__ bf16 load_a(const GemmArgs& a, int m, int k) {
-  if (m >= a.M || k >= a.K) return to_bf(0.f);
-  constexpr int KK2 = KS * KS;
-  if (MODE == GEMM_FWD) return a.wt[(long)m * a.K + k];
-  if (MODE == GEMM_BWD_DATA) {  // A(ci, (co, d)) = W[co][ci][d]
-    const int co = k / KK2, d = k - co * KK2;
-    return a.wt[((long)co * a.cin + m) * KK2 + d];
-  }
-  // BWD_W: A(co, (b, p)) = dZ[b][co][p]
-  const int b = k >> a.hw_sh, p = k & ((1 << a.hw_sh) - 1);
-  return to_bf(((const float*)a.y.p)[(((long)b * a.y.ctot + m) << a.hw_sh) + p]);
+// A layer's input: channels [0, cp0) from p0, [cp0, cp0 + cp1) from p1, both NHWC with those padded
+// channel counts; up0: p0 has half the resolution (nearest upsampling).
+struct Src {
+  const void* p0;
+  const void* p1;
+  int cp0, cp1, up0;
+};
+
+// Element offset of 8-channel group c8 (of 32-channel chunk ch) of pixel (b, y, x), and its tensor.
+__device__ __forceinline__ const void* src_base(const Src& s, int ch, int* cp, int* coff, int* up) {
+  const bool first = ch * 32 < s.cp0;
+  *cp = first ? s.cp0 : s.cp1;
+  *coff = first ? ch * 32 : ch * 32 - s.cp0;
+  *up = first ? s.up0 : 0;
+  return first ? s.p0 : s.p1;
 }
 
-// Implicit-GEMM convolution tile: D[m0 .. m0+64) x [n0 .. n0+64) over K in steps of 32.
-template <int MODE, int KS>
-__global__ __launch_bounds__(GT) void k_conv_gemm(GemmArgs a) {
-  constexpr int KK2 = KS * KS, R = KS / 2;
-  __shared__ bf16 As[TM * LDP];
-  __shared__ bf16 Bt[TN * LDP];  // transposed: Bt[n][k]
+// Where a tile of 32 output channels goes.  Forward: bias, ReLU, BF16.  Data gradient: FP32, zeroed
+// where the BF16 activation mask is not positive (the ReLU of the layer that made it; NULL: no ReLU);
+// sum4: the 2 x 2 sums go to a half-resolution tensor (the gradient of the upsampling).
+struct Dst {
+  void* p;
+  const bf16* mask;
+  int cp, coff, sum4;
+};
+
+struct ConvArgs {
+  Src in;               // forward: BF16; data gradient: FP32
+  const bf16* w;        // fragments: [output tile of 32][input chunk of 32][tap][2][lane][8]
+  const float* bias;    // forward: cout values
+  Dst out0, out1;       // output tiles below out0_tiles, and the others
+  int out0_tiles, cout; // cout: real output channels (forward)
+  int batch, h, w_px, chunks, tiles_x, tiles_y, groups, relu;
+};
+
+// 3 x 3 convolution, zero edges.  A workgroup makes a tile of 4 ROWS x 32 pixels of NCO x 32 output
+// channels; wave v its rows v ROWS .. v ROWS + ROWS - 1.  Per chunk of 32 input channels, the tile
+// with its one-pixel border and the chunk's weights go to LDS once and serve all nine taps.  The
+// matrix instruction takes weights as its rows and 32 pixels of an image row as its columns, so a
+// lane ends with groups of 4 adjacent channels of one pixel.  For one horizontal shift the ROWS + 2
+// pixel operands of a wave serve its three vertical shifts from registers: (ROWS + 2 + 3 NCO) LDS
+// reads of 16 bytes a lane for 3 ROWS NCO instructions, which keeps the LDS (128 B a clock) below
+// the matrix cores' time.  Pixels are 64 bytes apart in LDS; the 16-byte quarter q of column c is
+// stored at q ^ ((c >> 1) & 3), so that 8 adjacent lanes' reads spread over all banks.
+// GRAD: the data gradient (input FP32, rounded to BF16 on the way to LDS; weights with their taps
+// reversed and their channels exchanged).
+// AHEAD: the next chunk's loads are in flight during a chunk's products (as long as the registers for
+// them are there).
+template <int NCO, int ROWS, bool GRAD>
+__global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
+  constexpr bool AHEAD = NCO * ROWS <= 4;
+  constexpr int TR = 4 * ROWS + 2, TC = 34, XN = TR * TC * 4, WF = 9 * 2 * 64, WN = NCO * WF;  // 16-byte pieces
+  extern __shared__ u32x4 conv_lds[];
+  u32x4* const xs = conv_lds;
+  u32x4* const ws = conv_lds + XN;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int kbeg = MODE == GEMM_BWD_W ? blockIdx.z * a.kchunk : 0;
-  const int kend = MODE == GEMM_BWD_W ? min(a.K, kbeg + a.kchunk) : a.K;
-  const int wmask = (1 << a.w_sh) - 1, hwmask = (1 << a.hw_sh) - 1;
-  // FWD / BWD_DATA: each thread always loads the same B column n0 + tid % 64
-  const int bn = n0 + (tid & (TN - 1));
-  const bool bn_ok = bn < a.N;
-  const int bb = bn >> a.hw_sh, bp = bn & hwmask, by = bp >> a.w_sh, bx = bp & wmask;
-  v4f acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;
-  for (int k0 = kbeg; k0 < kend; k0 += TK) {
-    // A tile 64 x 32
-    if (MODE == GEMM_FWD && a.vec_a) {
-      const int mm = tid >> 2, kk = (tid & 3) * 8;
-      const int m = m0 + mm, k = k0 + kk;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (m < a.M && k < a.K) v = *reinterpret_cast<const uint4*>(a.wt + (long)m * a.K + k);
-      *reinterpret_cast<uint4*>(&As[mm * LDP + kk]) = v;
+  // blocks go round the 8 XCDs: the output groups of one pixel tile follow each other on one XCD,
+  // whose L2 then holds the tile's input
+  const int bid = blockIdx.x, tile = (bid / 8 / a.groups) * 8 + bid % 8, grp = bid / 8 % a.groups;
+  if (tile >= a.batch * a.tiles_x * a.tiles_y) return;
+  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x % a.tiles_y, b = tile / (a.tiles_x * a.tiles_y);
+  const int x0 = tx * 32, y0 = ty * 4 * ROWS;
+  v16f acc[NCO][ROWS];
+#pragma unroll
+  for (int t = 0; t < NCO; ++t)
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][r][i] = 0.f;
+  constexpr int XU = (XN + CT - 1) / CT, WU = (WN + CT - 1) / CT;
+  const u32x4* const w0 = reinterpret_cast<const u32x4*>(a.w) + (long)grp * NCO * a.chunks * WF;
+  u32x4 xv[AHEAD ? XU : 1], wr[AHEAD ? WU : 1];
+  f32x4 gv[AHEAD && GRAD ? XU : 1][2];
+  // one 16-byte piece of a chunk's input tile: FP32 rounded to BF16 for GRAD
+  auto pack = [](f32x4 u, f32x4 w) __attribute__((always_inline)) {
+    return u32x4{bf_pair(u[0], u[1]), bf_pair(u[2], u[3]), bf_pair(w[0], w[1]), bf_pair(w[2], w[3])};
+  };
+#define PTYK_CONV_PIECE(i)                                                                              \
+  const int e = tid + (i)*CT, q = e & 3, pc = e >> 2, r = pc / TC, c = pc - r * TC;                     \
+  const int y = y0 + r - 1, x = x0 + c - 1;                                                             \
+  const bool in = e < XN && y >= 0 && y < a.h && x >= 0 && x < a.w_px;                                  \
+  const long off = in ? (img + (y >> up) * sw + (x >> up)) * cp + coff + q * 8 : 0
+#define PTYK_CONV_CHUNK(ch)                                                                             \
+  int cp, coff, up;                                                                                     \
+  const void* const base = src_base(a.in, ch, &cp, &coff, &up);                                         \
+  const int sw = a.w_px >> up;                                                                          \
+  const long img = (long)b * (a.h >> up) * sw
+#define PTYK_CONV_LOAD(ch)                                                                              \
+  {                                                                                                     \
+    PTYK_CONV_CHUNK(ch);                                                                                \
+    _Pragma("unroll") for (int i = 0; i < XU; ++i) {                                                    \
+      PTYK_CONV_PIECE(i);                                                                               \
+      if constexpr (GRAD) {                                                                             \
+        const f32x4* g = reinterpret_cast<const f32x4*>((const float*)base + off);                      \
+        gv[i][0] = in ? g[0] : f32x4{0.f, 0.f, 0.f, 0.f};                                               \
+        gv[i][1] = in ? g[1] : f32x4{0.f, 0.f, 0.f, 0.f};                                               \
+      } else {                                                                                          \
+        xv[i] = in ? *reinterpret_cast<const u32x4*>((const bf16*)base + off) : u32x4{0u, 0u, 0u, 0u};  \
+      }                                                                                                 \
+    }                                                                                                   \
+    _Pragma("unroll") for (int i = 0; i < WU; ++i) {                                                    \
+      const int e = min(tid + i * CT, WN - 1);                                                          \
+      wr[i] = w0[((long)(e / WF) * a.chunks + (ch)) * WF + e % WF];                                     \
+    }                                                                                                   \
+  }
+  if constexpr (AHEAD) PTYK_CONV_LOAD(0)
+  for (int ch = 0; ch < a.chunks; ++ch) {
+    if (ch) __syncthreads();
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int i = 0; i < XU; ++i) {
+        const int e = tid + i * CT, q = e & 3, pc = e >> 2, c = pc % TC;
+        if (e < XN) xs[pc * 4 + (q ^ ((c >> 1) & 3))] = GRAD ? pack(gv[GRAD ? i : 0][0], gv[GRAD ? i : 0][1]) : xv[i];
+      }
+#pragma unroll
+      for (int i = 0; i < WU; ++i)
+        if (tid + i * CT < WN) ws[tid + i * CT] = wr[i];
+    } else {
+      PTYK_CONV_CHUNK(ch);
+#pragma unroll
+      for (int i = 0; i < XU; ++i) {
+        PTYK_CONV_PIECE(i);
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (in) {
+          if constexpr (GRAD) {
+            const f32x4* g = reinterpret_cast<const f32x4*>((const float*)base + off);
+            v = pack(g[0], g[1]);
+          } else {
+            v = *reinterpret_cast<const u32x4*>((const bf16*)base + off);
+          }
+        }
+        if (e < XN) xs[pc * 4 + (q ^ ((c >> 1) & 3))] = v;
+      }
+#pragma unroll
+      for (int t = 0; t < NCO; ++t)
+        for (int i = tid; i < WF; i += CT) ws[t * WF + i] = w0[((long)t * a.chunks + ch) * WF + i];
+    }
+    __syncthreads();
+    if constexpr (AHEAD)
+      if (ch + 1 < a.chunks) PTYK_CONV_LOAD(ch + 1)
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const int c = (lane & 31) + dx, q = ks * 2 + (lane >> 5), qs = q ^ ((c >> 1) & 3);
+        v8bf x[ROWS + 2];
+#pragma unroll
+        for (int r = 0; r < ROWS + 2; ++r)
+          x[r] = __builtin_bit_cast(v8bf, xs[((wv * ROWS + r) * TC + c) * 4 + qs]);
+#pragma unroll
+        for (int t = 0; t < NCO; ++t)
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy) {
+            const v8bf w = __builtin_bit_cast(v8bf, ws[((t * 9 + dy * 3 + dx) * 2 + ks) * 64 + lane]);
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+              acc[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x[r + dy], acc[t][r], 0, 0, 0);
+          }
+      }
+  }
+  // lane holds pixel x0 + lane % 32, channels 8 g + 4 (lane / 32) + 0..3 in registers 4 g + 0..3
+  const int x = x0 + (lane & 31), half = lane >> 5;
+#pragma unroll
+  for (int t = 0; t < NCO; ++t) {
+    const int ot = grp * NCO + t;
+    const Dst d = ot < a.out0_tiles ? a.out0 : a.out1;
+    const int c0 = (ot < a.out0_tiles ? ot : ot - a.out0_tiles) * 32 + d.coff;
+    if (!GRAD) {
+      float bias[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int co = ot * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+        bias[i] = co < a.cout ? a.bias[co] : 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const int y = y0 + wv * ROWS + r;
+        if (y >= a.h || x >= a.w_px) continue;
+        bf16* o = (bf16*)d.p + (((long)b * a.h + y) * a.w_px + x) * d.cp + c0 + 4 * half;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[i] = acc[t][r][4 * g + i] + bias[4 * g + i];
+            if (a.relu) v[i] = fmaxf(v[i], 0.f);
+          }
+          *reinterpret_cast<uint2*>(o + 8 * g) = make_uint2(bf_pair(v[0], v[1]), bf_pair(v[2], v[3]));
+        }
+      }
+    } else if (d.sum4) {  // image sizes are even here: whole 2 x 2 blocks, rows in pairs, columns in lane pairs
+      if (ROWS % 2 == 0) {
+#pragma unroll
+        for (int r = 0; r + 1 < ROWS; r += 2) {
+          const int y = y0 + wv * ROWS + r;
+          const long px = ((long)b * (a.h >> 1) + (y >> 1)) * (a.w_px >> 1) + (x >> 1);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float s = acc[t][r][4 * g + i], u = acc[t][r + 1][4 * g + i];
+              const float sx = __shfl_xor(s, 1, 64), ux = __shfl_xor(u, 1, 64);
+              v[i] = s + sx + u + ux;
+            }
+            if (y < a.h && x < a.w_px && !(lane & 1)) {
+              const long o = px * d.cp + c0 + 8 * g + 4 * half;
+              const uint2 m = *reinterpret_cast<const uint2*>(d.mask + o);
+              const unsigned mm[4] = {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16};
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (!(bf_val(mm[i]) > 0.f)) v[i] = 0.f;
+              *reinterpret_cast<float4*>((float*)d.p + o) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+          }
+        }
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < TM * TK / GT; ++i) {
-        const int e = tid + i * GT;
-        const int mm = e / TK, kk = e % TK;
-        const int k = k0 + kk;
-        As[mm * LDP + kk] = k < kend ? load_a<MODE, KS>(a, m0 + mm, k) : to_bf(0.f);
-      }
-    }
-    // B tile 32 x 64
-    if (MODE == GEMM_FWD || MODE == GEMM_BWD_DATA) {
-      const View& v = a.x;
+      for (int r = 0; r < ROWS; ++r) {
+        const int y = y0 + wv * ROWS + r;
+        if (y >= a.h || x >= a.w_px) continue;
+        const long o0 = (((long)b * a.h + y) * a.w_px + x) * d.cp + c0 + 4 * half;
 #pragma unroll
-      for (int i = 0; i < TN * TK / GT; ++i) {
-        const int kk = (tid >> 6) + i * (GT / TN);
-        const int k = k0 + kk;
-        bf16 val = to_bf(0.f);
-        if (bn_ok && k < kend) {
-          const int ch = k / KK2, d = k - ch * KK2;
-          int dy = d / KS - R, dx = d % KS - R;
-          if (MODE == GEMM_BWD_DATA) {
-            dy = -dy;
-            dx = -dx;
+        for (int g = 0; g < 4; ++g) {
+          float v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = acc[t][r][4 * g + i];
+          if (d.mask) {
+            const uint2 m = *reinterpret_cast<const uint2*>(d.mask + o0 + 8 * g);
+            const unsigned mm[4] = {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (!(bf_val(mm[i]) > 0.f)) v[i] = 0.f;
           }
-          const int sy = by + dy, sx = bx + dx;
-          if (sy >= 0 && sy < v.h && sx >= 0 && sx < v.w) {
-            const long idx = (((long)bb * v.ctot + ch) << a.hw_sh) + (sy << a.w_sh) + sx;
-            val = MODE == GEMM_FWD ? ((const bf16*)v.p)[idx] : to_bf(((const float*)v.p)[idx]);
-          }
-        }
-        Bt[(tid & (TN - 1)) * LDP + kk] = val;
-      }
-    } else {  // BWD_W: B((b, p), (ci, d)) = x[b][ci][p + d]; consecutive threads along k
-      const View& v = a.x;
-#pragma unroll
-      for (int i = 0; i < TN * TK / GT; ++i) {
-        const int e = tid + i * GT;
-        const int kk = e % TK, nn = e / TK;
-        const int k = k0 + kk, n = n0 + nn;
-        bf16 val = to_bf(0.f);
-        if (k < kend && n < a.N) {
-          const int b = k >> a.hw_sh, p = k & hwmask, yy = p >> a.w_sh, xx = p & wmask;
-          const int ci = n / KK2, d = n - ci * KK2;
-          const int sy = yy + d / KS - R, sx = xx + d % KS - R;
-          if (sy >= 0 && sy < v.h && sx >= 0 && sx < v.w)
-            val = ((const bf16*)v.p)[(((long)b * v.ctot + ci) << a.hw_sh) + (sy << a.w_sh) + sx];
-        }
-        Bt[nn * LDP + kk] = val;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const v8bf va = *reinterpret_cast<const v8bf*>(&As[(wm + i * 16 + (lane & 15)) * LDP + 8 * (lane >> 4)]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const v8bf vb = *reinterpret_cast<const v8bf*>(&Bt[(wn + j * 16 + (lane & 15)) * LDP + 8 * (lane >> 4)]);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, vb, acc[i][j], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  // epilogue: lane holds D[4 (lane / 16) + r][lane % 16] of each 16 x 16 sub-tile
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
-        const int n = n0 + wn + j * 16 + (lane & 15);
-        if (m >= a.M || n >= a.N) continue;
-        float v = acc[i][j][r];
-        if (MODE == GEMM_BWD_W) {
-          a.partial[((long)blockIdx.z * a.M + m) * a.N + n] = v;
-        } else {
-          const View& o = a.y;
-          const int b = n >> a.hw_sh, p = n & hwmask;
-          const long idx = (((long)b * o.ctot + m) << a.hw_sh) + p;
-          if (MODE == GEMM_FWD) {
-            v += a.bias[m];
-            if (a.relu) v = fmaxf(v, 0.f);
-            if (a.out_f32) ((float*)o.p)[idx] = v;
-            else ((bf16*)o.p)[idx] = to_bf(v);
-          } else {
-            ((float*)o.p)[idx] = v;
-          }
+          *reinterpret_cast<float4*>((float*)d.p + o0 + 8 * g) = make_float4(v[0], v[1], v[2], v[3]);
         }
       }
-}
-
-// ---- vector-operand form (image width >= 8): each thread moves 8 consecutive pixels of one
-// image row per K step -- one aligned 16-byte (or two for FP32) load plus the neighbour element
-// a +-1 tap shift needs -- instead of 8 gathered elements.
-typedef unsigned short u16;
-
-__device__ __forceinline__ u16 bf_bits(float v) { return __builtin_bit_cast(u16, to_bf(v)); }
-
-// row[x0 + dx .. x0 + dx + 7] (bf16 bits), zero outside [0, w); x0 % 8 == 0, |dx| <= 1
-__device__ __forceinline__ void row8_bf16(const u16* __restrict__ row, int x0, int dx, int w, u16 out[8]) {
-  union {
-    uint4 v;
-    u16 h[8];
-  } u;
-  u.v = *reinterpret_cast<const uint4*>(row + x0);
-  if (dx == 0) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = u.h[i];
-  } else if (dx < 0) {
-    out[0] = x0 > 0 ? row[x0 - 1] : (u16)0;
-#pragma unroll
-    for (int i = 1; i < 8; ++i) out[i] = u.h[i - 1];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 7; ++i) out[i] = u.h[i + 1];
-    out[7] = x0 + 8 < w ? row[x0 + 8] : (u16)0;
+    }
   }
 }
 
-// the same for an FP32 row, rounded to bf16
-__device__ __forceinline__ void row8_f32(const float* __restrict__ row, int x0, int dx, int w, u16 out[8]) {
-  const float4 a = *reinterpret_cast<const float4*>(row + x0);
-  const float4 b = *reinterpret_cast<const float4*>(row + x0 + 4);
-  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  if (dx == 0) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = bf_bits(v[i]);
-  } else if (dx < 0) {
-    out[0] = x0 > 0 ? bf_bits(row[x0 - 1]) : (u16)0;
-#pragma unroll
-    for (int i = 1; i < 8; ++i) out[i] = bf_bits(v[i - 1]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 7; ++i) out[i] = bf_bits(v[i + 1]);
-    out[7] = x0 + 8 < w ? bf_bits(row[x0 + 8]) : (u16)0;
-  }
-}
+#undef PTYK_CONV_LOAD
+#undef PTYK_CONV_PIECE
+#undef PTYK_CONV_CHUNK
 
-// Same tile and MFMA schedule as k_conv_gemm (so the same sums in the same order). a.wt holds
-// the weights for FWD and their [C_in][C_out x taps] transpose for BWD_DATA.
-template <int MODE, int KS>
-__global__ __launch_bounds__(GT) void k_conv_gemm_vec(GemmArgs a) {
-  constexpr int KK2 = KS * KS, R = KS / 2;
-  __shared__ __align__(16) u16 As[TM * LDP];
-  __shared__ __align__(16) u16 Bt[TN * LDP];  // transposed: Bt[n][k]
+struct WgradArgs {
+  Src x;              // BF16 input of the layer
+  const float* dz;    // FP32 gradient of its pre-activation output, NHWC with cpo channels
+  float* part;        // [chunk][output tile][input tile][tap][32][32] (output, input channel)
+  double* bpart;      // [chunk][cpo]: bias gradient
+  int batch, h, w_px, cpo, tiles_o, tiles_i, tiles_x, tiles_y, chunks;
+};
+
+// Weight gradient: D[co][ci] per tap = sum over pixels of dZ[p][co] x[p + tap][ci], a GEMM whose
+// contraction runs over pixels.  A workgroup owns one 32 x 32 channel tile of all nine taps and a
+// share of the 8 x 32-pixel tiles; its four waves take two rows each and add up at the end.  The
+// matrix instruction wants 8 adjacent pixels of one channel per lane, so tiles are transposed on
+// their way to LDS ([channel][pixel]); x is kept three times, shifted by -1, 0 and 1 pixels, so that
+// every operand is one aligned 16-byte read.  Per wave and 16 pixels: 2 + 12 reads for 18
+// instructions.  Channel pitches of 528 and 656 bytes spread 8 lanes over the banks.
+constexpr int WG_R = 8, WG_ZP = WG_R * 64 + 16, WG_XP = (WG_R + 2) * 64 + 16;  // bytes per channel
+__global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
+  extern __shared__ __align__(16) unsigned char wg_lds[];
+  unsigned char* const zs = wg_lds;                // 32 x WG_ZP
+  unsigned char* const xs = wg_lds + 32 * WG_ZP;   // 3 x 32 x WG_XP
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int kbeg = MODE == GEMM_BWD_W ? blockIdx.z * a.kchunk : 0;
-  const int kend = MODE == GEMM_BWD_W ? min(a.K, kbeg + a.kchunk) : a.K;
-  const int w = 1 << a.w_sh, wmask = w - 1, hwmask = (1 << a.hw_sh) - 1;
-  const View& v = a.x;
-  // FWD / BWD_DATA B roles: k row tid / 8 of the step, pixels nb .. nb + 7 of one image row
-  const int nb = n0 + ((tid & 7) << 3);
-  const bool nb_ok = nb < a.N;
-  const int bb = nb >> a.hw_sh, bp = nb & hwmask, by = bp >> a.w_sh, bx0 = bp & wmask;
-  v4f acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;
-  for (int k0 = kbeg; k0 < kend; k0 += TK) {
-    // ---- A tile 64 x 32
-    if (MODE != GEMM_BWD_W) {
-      const u16* wt = reinterpret_cast<const u16*>(a.wt);
-      if (a.vec_a) {
-        const int mm = tid >> 2, kk = (tid & 3) * 8;
-        const int m = m0 + mm, k = k0 + kk;
-        uint4 val = make_uint4(0u, 0u, 0u, 0u);
-        if (m < a.M && k < a.K) val = *reinterpret_cast<const uint4*>(wt + (long)m * a.K + k);
-        *reinterpret_cast<uint4*>(&As[mm * LDP + kk]) = val;
-      } else {
+  const int pairs = a.tiles_o * a.tiles_i, pr = blockIdx.x % pairs, chunk = blockIdx.x / pairs;
+  const int ot = pr / a.tiles_i, it = pr % a.tiles_i;
+  int cp, coff, up;
+  const void* base = src_base(a.x, it, &cp, &coff, &up);
+  const int sw = a.w_px >> up, sh = a.h >> up;
+  const int cpair = tid & 15, slot = tid >> 4;  // 2 channels, one of 16 pixel groups of 8
+  v16f acc[9];
 #pragma unroll
-        for (int i = 0; i < TM * TK / GT; ++i) {
-          const int e = tid + i * GT;
-          const int mm = e / TK, kk = e % TK;
-          const int m = m0 + mm, k = k0 + kk;
-          As[mm * LDP + kk] = (m < a.M && k < a.K) ? wt[(long)m * a.K + k] : (u16)0;
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+  double bs0 = 0.0, bs1 = 0.0;
+  const int tiles = a.batch * a.tiles_x * a.tiles_y;
+  const int lo = (int)((long)tiles * chunk / a.chunks), hi = (int)((long)tiles * (chunk + 1) / a.chunks);
+  for (int tile = lo; tile < hi; ++tile) {
+    const int tx = tile % a.tiles_x, ty = tile / a.tiles_x % a.tiles_y, b = tile / (a.tiles_x * a.tiles_y);
+    const int x0 = tx * 32, y0 = ty * WG_R;
+    if (tile != lo) __syncthreads();
+    // dZ: 8 rows x 4 groups of 8 pixels x 16 channel pairs
+#pragma unroll
+    for (int i = 0; i < WG_R * 4 / 16; ++i) {
+      const int g = slot + i * 16, r = g >> 2, xg = (g & 3) * 8, y = y0 + r;
+      float2 v[8];
+      const int left = y < a.h ? a.w_px - (x0 + xg) : 0;  // pixels from here to the row's end
+      const float* zp = a.dz + (((long)b * a.h + min(y, a.h - 1)) * a.w_px + x0 + xg) * a.cpo + ot * 32 + cpair * 2;
+#pragma unroll
+      for (int p = 0; p < 8; ++p)
+        v[p] = p < left ? *reinterpret_cast<const float2*>(zp + p * a.cpo) : make_float2(0.f, 0.f);
+      if (it == 0) {
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+          bs0 += v[p].x;
+          bs1 += v[p].y;
         }
       }
-    } else {  // A(co, (b, p)) = dZ[b][co][p]: 8 consecutive pixels of one image
-      const int mm = tid >> 2, kg = (tid & 3) * 8;
-      const int m = m0 + mm, k = k0 + kg;
-      u16 h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (m < a.M && k < kend) {
-        const int b = k >> a.hw_sh, p = k & hwmask;
-        row8_f32((const float*)a.y.p + (((long)b * a.y.ctot + m) << a.hw_sh), p, 0, 1 << a.hw_sh, h);
-      }
-      uint4 val;
-      val.x = h[0] | ((unsigned)h[1] << 16);
-      val.y = h[2] | ((unsigned)h[3] << 16);
-      val.z = h[4] | ((unsigned)h[5] << 16);
-      val.w = h[6] | ((unsigned)h[7] << 16);
-      *reinterpret_cast<uint4*>(&As[mm * LDP + kg]) = val;
+      unsigned char* z = zs + (cpair * 2) * WG_ZP + r * 64 + xg * 2;
+      *reinterpret_cast<uint4*>(z) = make_uint4(bf_pair(v[0].x, v[1].x), bf_pair(v[2].x, v[3].x),
+                                                bf_pair(v[4].x, v[5].x), bf_pair(v[6].x, v[7].x));
+      *reinterpret_cast<uint4*>(z + WG_ZP) = make_uint4(bf_pair(v[0].y, v[1].y), bf_pair(v[2].y, v[3].y),
+                                                        bf_pair(v[4].y, v[5].y), bf_pair(v[6].y, v[7].y));
     }
-    // ---- B tile 32 x 64 (stored transposed)
-    if (MODE == GEMM_FWD || MODE == GEMM_BWD_DATA) {
-      const int kk = tid >> 3, k = k0 + kk;
-      u16 h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (nb_ok && k < kend) {
-        const int ch = k / KK2, d = k - ch * KK2;
-        int dy = d / KS - R, dx = d % KS - R;
-        if (MODE == GEMM_BWD_DATA) {
-          dy = -dy;
-          dx = -dx;
+    // x: 10 rows, each group with its neighbours on both sides
+#pragma unroll
+    for (int i = 0; i < ((WG_R + 2) * 4 + 15) / 16; ++i) {
+      const int g = slot + i * 16, r = g >> 2, xg = (g & 3) * 8, y = y0 + r - 1;
+      if (g >= (WG_R + 2) * 4) break;
+      unsigned v[10];  // two channels of pixels xg - 1 .. xg + 8
+      const int left = y >= 0 && y < a.h ? a.w_px - (x0 + xg - 1) : 0;
+      const bf16* xp = (const bf16*)base + ((long)b * sh + (max(y, 0) >> up)) * sw * cp + coff + cpair * 2;
+#pragma unroll
+      for (int p = 0; p < 10; ++p)
+        v[p] = p < left && (p > 0 || x0 + xg > 0)
+                   ? *reinterpret_cast<const unsigned*>(xp + ((x0 + xg + p - 1) >> up) * cp)
+                   : 0u;
+      unsigned char* d = xs + (cpair * 2) * WG_XP + r * 64 + xg * 2;
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {  // copy s holds x[p + s - 1]
+        unsigned lo4[4], hi4[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          lo4[k] = (v[s + 2 * k] & 0xffffu) | (v[s + 2 * k + 1] << 16);
+          hi4[k] = (v[s + 2 * k] >> 16) | (v[s + 2 * k + 1] & 0xffff0000u);
         }
-        const int sy = by + dy;
-        if (sy >= 0 && sy < v.h) {
-          const long off = (((long)bb * v.ctot + ch) << a.hw_sh) + ((long)sy << a.w_sh);
-          if (MODE == GEMM_FWD) row8_bf16((const u16*)v.p + off, bx0, dx, w, h);
-          else row8_f32((const float*)v.p + off, bx0, dx, w, h);
-        }
-      }
-      const int ng = (tid & 7) << 3;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) Bt[(ng + i) * LDP + kk] = h[i];
-    } else {  // B((b, p), (ci, d)) = x[b][ci][p + d]: 8 consecutive pixels of one row
-      const int nn = tid >> 2, kg = (tid & 3) * 8;
-      const int n = n0 + nn, k = k0 + kg;
-      u16 h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (n < a.N && k < kend) {
-        const int b = k >> a.hw_sh, p = k & hwmask, yy = p >> a.w_sh, x0 = p & wmask;
-        const int ci = n / KK2, d = n - ci * KK2;
-        const int sy = yy + d / KS - R, dx = d % KS - R;
-        if (sy >= 0 && sy < v.h)
-          row8_bf16((const u16*)v.p + (((long)b * v.ctot + ci) << a.hw_sh) + ((long)sy << a.w_sh), x0, dx, w, h);
-      }
-      uint4 val;
-      val.x = h[0] | ((unsigned)h[1] << 16);
-      val.y = h[2] | ((unsigned)h[3] << 16);
-      val.z = h[4] | ((unsigned)h[5] << 16);
-      val.w = h[6] | ((unsigned)h[7] << 16);
-      *reinterpret_cast<uint4*>(&Bt[nn * LDP + kg]) = val;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const v8bf va = *reinterpret_cast<const v8bf*>(&As[(wm + i * 16 + (lane & 15)) * LDP + 8 * (lane >> 4)]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const v8bf vb = *reinterpret_cast<const v8bf*>(&Bt[(wn + j * 16 + (lane & 15)) * LDP + 8 * (lane >> 4)]);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, vb, acc[i][j], 0, 0, 0);
+        *reinterpret_cast<uint4*>(d + s * 32 * WG_XP) = make_uint4(lo4[0], lo4[1], lo4[2], lo4[3]);
+        *reinterpret_cast<uint4*>(d + s * 32 * WG_XP + WG_XP) = make_uint4(hi4[0], hi4[1], hi4[2], hi4[3]);
       }
     }
     __syncthreads();
+    const int ch = lane & 31, half = lane >> 5;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int po = ks * 32 + half * 16;  // bytes: 8 pixels
+      v8bf z[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        z[r] = *reinterpret_cast<const v8bf*>(zs + ch * WG_ZP + (wv * 2 + r) * 64 + po);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        v8bf x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          x[r] = *reinterpret_cast<const v8bf*>(xs + (s * 32 + ch) * WG_XP + (wv * 2 + r) * 64 + po);
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+            acc[dy * 3 + s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(z[r], x[r + dy], acc[dy * 3 + s], 0, 0, 0);
+      }
+    }
+  }
+  // waves add up through LDS, 3 taps at a time, in wave order; wave 0 writes
+  float* red = reinterpret_cast<float*>(wg_lds);  // 3 waves x 3 taps x 1024 floats
+  float* out = a.part + ((long)chunk * pairs + pr) * (9 * 1024);
+#pragma unroll
+  for (int t3 = 0; t3 < 3; ++t3) {
+    __syncthreads();
+    if (wv > 0)
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) red[(((wv - 1) * 3 + t) * 16 + i) * 64 + lane] = acc[t3 * 3 + t][i];
+    __syncthreads();
+    if (wv == 0)
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          float s = acc[t3 * 3 + t][i];
+#pragma unroll
+          for (int u = 0; u < 3; ++u) s += red[((u * 3 + t) * 16 + i) * 64 + lane];
+          out[(t3 * 3 + t) * 1024 + (8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * 32 + (lane & 31)] = s;
+        }
+  }
+  if (it == 0) {  // bias: 16 pixel slots per channel pair
+    double* rb = reinterpret_cast<double*>(wg_lds);
+    __syncthreads();
+    rb[tid * 2] = bs0;
+    rb[tid * 2 + 1] = bs1;
+    __syncthreads();
+    if (tid < 32) {
+      double s = 0.0;
+      for (int k = 0; k < 16; ++k) s += rb[(k * 16 + (tid >> 1)) * 2 + (tid & 1)];
+      a.bpart[(long)chunk * a.cpo + ot * 32 + tid] = s;
+    }
+  }
+}
+
+// Position of an input channel among the padded channels of a layer's (up to) two input tensors.
+struct LayerMap {
+  long woff, boff, foff, goff;  // parameters; forward and data-gradient fragments
+  int cin, cout, ks, c0;        // c0: real channels of the first input tensor (cin when there is one)
+  int cp0, cpi, cpo;            // padded: first input tensor, all inputs, outputs
+};
+struct LayerTable {
+  LayerMap l[NN_LAYERS];
+};
+__device__ __forceinline__ int pad_channel(const LayerMap& m, int ci) { return ci < m.c0 ? ci : m.cp0 + (ci - m.c0); }
+
+// Chunk sums (fixed order) of the weight and bias gradients, scattered to the parameter order.  A
+// block makes 32 values (adjacent input channels of one partial tile's row: 128-byte reads), its 8
+// lanes of 32 threads taking every eighth chunk; the biases follow behind the weights' blocks.
+__global__ __launch_bounds__(256) void k_wgrad_sum(LayerMap m, const float* __restrict__ part,
+                                                   const double* __restrict__ bpart, int chunks, float* __restrict__ g) {
+  __shared__ double red[8][32];
+  const int k = threadIdx.x & 31, ln = threadIdx.x >> 5;
+  const int rows = m.cpo / 32 * (m.cpi / 32) * 9 * 32;  // partial tiles' rows: (pair, tap, output channel)
+  const bool weight = (int)blockIdx.x < rows;
+  double s = 0.0;
+  if (weight) {
+    const float* p = part + (long)blockIdx.x * 32 + k;
+    const long stride = (long)rows * 32;
+    float f = 0.f;
+    for (int c = ln; c < chunks; c += 8) f += p[c * stride];
+    s = f;
+  } else {
+    const int co = (blockIdx.x - rows) * 32 + k;
+    for (int c = ln; c < chunks; c += 8) s += bpart[(long)c * m.cpo + co];
+  }
+  red[ln][k] = s;
+  __syncthreads();
+  if (ln) return;
+  s = red[0][k];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) s += red[i][k];
+  if (!weight) {
+    const int co = (blockIdx.x - rows) * 32 + k;
+    if (co < m.cout) g[m.boff + co] = (float)s;
+    return;
+  }
+  const int pair = blockIdx.x / (9 * 32), tap = blockIdx.x / 32 % 9;
+  const int co = pair / (m.cpi / 32) * 32 + blockIdx.x % 32, cc = pair % (m.cpi / 32) * 32 + k;
+  const int ci = cc < m.cp0 ? cc : m.c0 + (cc - m.cp0);  // the channel behind a padded position
+  if (co < m.cout && (cc < m.cp0 ? cc < m.c0 : ci < m.cin)) g[m.woff + ((long)co * m.cin + ci) * 9 + tap] = (float)s;
+}
+
+// The BF16 copies of parameter i: plain (first and last layer), and its places among the forward and
+// data-gradient fragments ([output tile][input chunk][tap][2][lane][8]).
+__device__ __forceinline__ void store_weight(const LayerTable& tb, long i, float v, bf16* __restrict__ wb,
+                                             bf16* __restrict__ wf, bf16* __restrict__ wg) {
+  const bf16 h = to_bf(v);
+  wb[i] = h;
+  int l = 0;
+  while (l + 1 < NN_LAYERS && i >= tb.l[l + 1].woff) ++l;
+  const LayerMap& m = tb.l[l];
+  if (i >= m.boff || m.ks != 3 || m.cin == 1) return;
+  const int k = (int)(i - m.woff), t = k % 9, ci = pad_channel(m, k / 9 % m.cin), co = k / (9 * m.cin);
+  auto frag = [](int o, int chunks, int c, int tap) {
+    return ((((long)(o >> 5) * chunks + (c >> 5)) * 9 + tap) * 2 + (c >> 4 & 1)) * 512 + ((o & 31) + 32 * (c >> 3 & 1)) * 8 +
+           (c & 7);
+  };
+  wf[m.foff + frag(co, m.cpi / 32, ci, t)] = h;
+  wg[m.goff + frag(ci, m.cpo / 32, co, 8 - t)] = h;
+}
+
+__global__ void k_pack(LayerTable tb, const float* __restrict__ w, long n, bf16* __restrict__ wb, bf16* __restrict__ wf,
+                       bf16* __restrict__ wg) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) store_weight(tb, i, w[i], wb, wf, wg);
+}
+
+// Adam on FP32 master weights; refreshes the BF16 copies
+__global__ void k_adam(LayerTable tb, float* __restrict__ w, float* __restrict__ mo, float* __restrict__ ve,
+                       const float* __restrict__ g, bf16* __restrict__ wb, bf16* __restrict__ wf, bf16* __restrict__ wg,
+                       long n, float lr, float b1, float b2, float eps, float c1, float c2) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float gi = g[i];
+  const float m = b1 * mo[i] + (1.f - b1) * gi;
+  const float v = b2 * ve[i] + (1.f - b2) * gi * gi;
+  mo[i] = m;
+  ve[i] = v;
+  const float wn = w[i] - lr * (m / c1) / (sqrtf(v / c2) + eps);
+  w[i] = wn;
+  store_weight(tb, i, wn, wb, wf, wg);
+}
+
+// First layer: one input channel, 3 x 3, ReLU.  A thread keeps the weights of 8 channels and makes
+// them for one pixel after another (bound by the output's bytes).
+__global__ __launch_bounds__(256) void k_first_fwd(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                   const float* __restrict__ bias, bf16* __restrict__ out, int cout,
+                                                   int cp, int cg0, long npx, int sh, int s) {
+  const int groups = min(cp / 8 - cg0, 32), lanes = 256 / groups;
+  const int g = (cg0 + threadIdx.x % groups) * 8, pl = threadIdx.x / groups;
+  if (pl >= lanes) return;
+  float wv[8][9], bv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    bv[i] = g + i < cout ? bias[g + i] : 0.f;
+#pragma unroll
+    for (int t = 0; t < 9; ++t) wv[i][t] = g + i < cout ? (float)w[(g + i) * 9 + t] : 0.f;
+  }
+  for (long px = (long)blockIdx.x * lanes + pl; px < npx; px += (long)gridDim.x * lanes) {
+    const int xx = (int)(px & (s - 1)), yy = (int)(px >> sh) & (s - 1);
+    float v[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+      const int y = yy + t / 3 - 1, c = xx + t % 3 - 1;
+      v[t] = y >= 0 && y < s && c >= 0 && c < s ? (float)x[px + (long)(t / 3 - 1) * s + t % 3 - 1] : 0.f;
+    }
+    float o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float acc = 0.f;
+#pragma unroll
+      for (int t = 0; t < 9; ++t) acc = fmaf(wv[i][t], v[t], acc);
+      o[i] = fmaxf(acc + bv[i], 0.f);
+    }
+    *reinterpret_cast<uint4*>(out + px * cp + g) =
+        make_uint4(bf_pair(o[0], o[1]), bf_pair(o[2], o[3]), bf_pair(o[4], o[5]), bf_pair(o[6], o[7]));
+  }
+}
+
+// Its weight and bias gradient: thread = one of 32 channels (blockIdx.y) x one of 8 lanes, which take
+// segments of up to 16 pixels of a row and slide the 3 x 3 window along them; the block's sums go to
+// part[block][tap][cp] and bpart[block][cp].
+__global__ __launch_bounds__(256) void k_first_wgrad(const bf16* __restrict__ x, const float* __restrict__ dz, int cp,
+                                                     long npx, int sh, int s, float* __restrict__ part,
+                                                     double* __restrict__ bpart) {
+  __shared__ float red[8][9][32];
+  __shared__ double redb[8][32];
+  constexpr int SEG = 16;
+  const int c = threadIdx.x & 31, pl = threadIdx.x >> 5, co = blockIdx.y * 32 + c;
+  const int len = min(SEG, s);
+  float acc[9] = {};
+  double bs = 0.0;
+  for (long sg = (long)blockIdx.x * 8 + pl; sg < npx / len; sg += (long)gridDim.x * 8) {
+    const long px = sg * len;
+    const int xx = (int)(px & (s - 1)), yy = (int)(px >> sh) & (s - 1);
+    const bool up = yy > 0, dn = yy + 1 < s;
+    float d[SEG], v[3][SEG + 2];
+#pragma unroll
+    for (int i = 0; i < SEG; ++i) d[i] = i < len ? dz[(px + i) * cp + co] : 0.f;
+#pragma unroll
+    for (int i = 0; i < SEG + 2; ++i) {
+      const int cx = xx + i - 1;
+      const bool in = cx >= 0 && cx < s && i < len + 2;
+      v[0][i] = in && up ? (float)x[px + i - 1 - s] : 0.f;
+      v[1][i] = in ? (float)x[px + i - 1] : 0.f;
+      v[2][i] = in && dn ? (float)x[px + i - 1 + s] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < SEG; ++i) {
+      bs += d[i];
+      const float dr = (float)to_bf(d[i]);
+#pragma unroll
+      for (int t = 0; t < 9; ++t) acc[t] = fmaf(dr, v[t / 3][i + t % 3], acc[t]);
+    }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int t = 0; t < 9; ++t) red[pl][t][c] = acc[t];
+  redb[pl][c] = bs;
+  __syncthreads();
+  for (int i = threadIdx.x; i < 9 * 32; i += 256) {
+    float v = 0.f;
+    for (int p = 0; p < 8; ++p) v += red[p][i / 32][i % 32];
+    part[((long)blockIdx.x * 9 + i / 32) * cp + blockIdx.y * 32 + i % 32] = v;
+  }
+  if (threadIdx.x < 32) {
+    double v = 0.0;
+    for (int p = 0; p < 8; ++p) v += redb[p][c];
+    bpart[(long)blockIdx.x * cp + co] = v;
+  }
+}
+// g[co][t] and the bias from the blocks' sums, one wave per value
+__global__ __launch_bounds__(64) void k_first_sum(const float* __restrict__ part, const double* __restrict__ bpart,
+                                                  int blocks, int cp, float* __restrict__ gw, float* __restrict__ gb) {
+  const int co = blockIdx.x, t = blockIdx.y;
+  double s = 0.0;
+  for (int b = threadIdx.x; b < blocks; b += 64)
+    s += t < 9 ? (double)part[((long)b * 9 + t) * cp + co] : bpart[(long)b * cp + co];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) {
+    if (t < 9) gw[co * 9 + t] = (float)s;
+    else gb[co] = (float)s;
+  }
+}
+
+// Last layer: 1 x 1 to two channels (NCHW, FP32 out), one pixel per thread.
+__global__ __launch_bounds__(256) void k_last_fwd(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                  const float* __restrict__ bias, float* __restrict__ out, int cin, int cp,
+                                                  long npx, long ss) {
+  for (long px = (long)blockIdx.x * 256 + threadIdx.x; px < npx; px += (long)gridDim.x * 256) {
+    float a0 = 0.f, a1 = 0.f;
+    for (int g = 0; g < cin; g += 8) {
+      const uint4 v = *reinterpret_cast<const uint4*>(x + px * cp + g);
+      const unsigned u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int i = 0; i < 8; ++i) {
+        if (g + i >= cin) break;
+        const float f = bf_val(i & 1 ? u[i >> 1] >> 16 : u[i >> 1] & 0xffffu);
+        a0 = fmaf((float)w[g + i], f, a0);
+        a1 = fmaf((float)w[cin + g + i], f, a1);
+      }
+    }
+    const long b = px / ss, p = px - b * ss;
+    out[(b * 2) * ss + p] = a0 + bias[0];
+    out[(b * 2 + 1) * ss + p] = a1 + bias[1];
+  }
+}
+
+// Its backward pass: the gradient of the input (masked by the input's ReLU) and the block's sums of
+// the weight gradient, part[block][2][cp], and of the bias gradient, bpart[block][2].  A thread keeps
+// 8 channels and strides over pixels; blockDim = 256 threads = 256 / (cp / 8) pixels at a time.
+__global__ __launch_bounds__(256) void k_last_bwd(const float* __restrict__ gout, const bf16* __restrict__ x,
+                                                  const bf16* __restrict__ w, float* __restrict__ gx, int cin, int cp,
+                                                  int cg0, long npx, long ss, float* __restrict__ part,
+                                                  double* __restrict__ bpart) {
+  __shared__ float red[256][17];
+  __shared__ double redb[256][2];
+  const int groups = min(cp / 8 - cg0, 32), lanes = 256 / groups;
+  const int g = threadIdx.x % groups, pl = threadIdx.x / groups, c0 = (cg0 + g) * 8;
+  float w0[8], w1[8], s0[8] = {}, s1[8] = {};
+  double b0 = 0.0, b1 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    w0[i] = c0 + i < cin ? (float)w[c0 + i] : 0.f;
+    w1[i] = c0 + i < cin ? (float)w[cin + c0 + i] : 0.f;
+  }
+  if (pl < lanes)
+    for (long px = (long)blockIdx.x * lanes + pl; px < npx; px += (long)gridDim.x * lanes) {
+      const long b = px / ss, p = px - b * ss;
+      const float d0 = gout[(b * 2) * ss + p], d1 = gout[(b * 2 + 1) * ss + p];
+      const float r0 = (float)to_bf(d0), r1 = (float)to_bf(d1);
+      b0 += d0;
+      b1 += d1;
+      const uint4 v = *reinterpret_cast<const uint4*>(x + px * cp + c0);
+      const unsigned u[4] = {v.x, v.y, v.z, v.w};
+      float o[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f = bf_val(i & 1 ? u[i >> 1] >> 16 : u[i >> 1] & 0xffffu);
+        s0[i] = fmaf(r0, f, s0[i]);
+        s1[i] = fmaf(r1, f, s1[i]);
+        o[i] = f > 0.f ? fmaf(r1, w1[i], r0 * w0[i]) : 0.f;
+      }
+      float4* q = reinterpret_cast<float4*>(gx + px * cp + c0);
+      q[0] = make_float4(o[0], o[1], o[2], o[3]);
+      q[1] = make_float4(o[4], o[5], o[6], o[7]);
+    }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    red[threadIdx.x][i] = s0[i];
+    red[threadIdx.x][8 + i] = s1[i];
+  }
+  redb[threadIdx.x][0] = b0;
+  redb[threadIdx.x][1] = b1;
+  __syncthreads();
+  for (int i = threadIdx.x; i < groups * 16; i += 256) {
+    const int gg = i / 16, k = i % 16;
+    float v = 0.f;
+    for (int p = 0; p < lanes; ++p) v += red[p * groups + gg][k];
+    part[((long)blockIdx.x * 2 + k / 8) * cp + (cg0 + gg) * 8 + k % 8] = v;
+  }
+  if (cg0 == 0 && threadIdx.x < 2) {
+    double v = 0.0;
+    for (int p = 0; p < lanes; ++p) v += redb[p * groups][threadIdx.x];
+    bpart[blockIdx.x * 2 + threadIdx.x] = v;
+  }
+}
+__global__ __launch_bounds__(64) void k_last_sum(const float* __restrict__ part, const double* __restrict__ bpart,
+                                                 int blocks, int cin, int cp, float* __restrict__ gw,
+                                                 float* __restrict__ gb) {
+  const int ci = blockIdx.x, o = blockIdx.y;
+  double s = 0.0;
+  for (int b = threadIdx.x; b < blocks; b += 64)
+    s += ci < cin ? (double)part[((long)b * 2 + o) * cp + ci] : bpart[b * 2 + o];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) {
+    if (ci < cin) gw[o * cin + ci] = (float)s;
+    else gb[o] = (float)s;
+  }
+}
+
+// 2 x 2 max pooling, 8 channels of one output pixel per thread; arg holds the winning offsets (0..3)
+// for the backward pass, the first of equal ones
+__global__ __launch_bounds__(256) void k_pool_fwd(const bf16* __restrict__ in, bf16* __restrict__ out,
+                                                  uint8_t* __restrict__ arg, int cp, long total, int osh, int ow) {
+  const int groups = cp / 8;
+  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
+    const long px = e / groups;
+    const int g = (int)(e - px * groups) * 8, x = (int)(px & (ow - 1));
+    const long row = px >> osh;  // (b, y)
+    uint4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      v[q] = *reinterpret_cast<const uint4*>(in + ((2 * row + (q >> 1)) * (2 * ow) + 2 * x + (q & 1)) * cp + g);
+    unsigned o[4], am[2] = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float best = -INFINITY;
+      unsigned bits = 0xff80u, bi = 0;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m0 + wm + i * 16 + 4 * (lane >> 4) + q;
-        const int n = n0 + wn + j * 16 + (lane & 15);
-        if (m >= a.M || n >= a.N) continue;
-        float val = acc[i][j][q];
-        if (MODE == GEMM_BWD_W) {
-          a.partial[((long)blockIdx.z * a.M + m) * a.N + n] = val;
-        } else {
-          const View& o = a.y;
-          const int b = n >> a.hw_sh, p = n & hwmask;
-          const long idx = (((long)b * o.ctot + m) << a.hw_sh) + p;
-          if (MODE == GEMM_FWD) {
-            val += a.bias[m];
-            if (a.relu) val = fmaxf(val, 0.f);
-            if (a.out_f32) ((float*)o.p)[idx] = val;
-            else ((bf16*)o.p)[idx] = to_bf(val);
-          } else {
-            ((float*)o.p)[idx] = val;
-          }
+        const unsigned u = i < 2 ? v[q].x : i < 4 ? v[q].y : i < 6 ? v[q].z : v[q].w;
+        const unsigned h = i & 1 ? u >> 16 : u & 0xffffu;
+        if (bf_val(h) > best) {
+          best = bf_val(h);
+          bits = h;
+          bi = q;
         }
       }
-}
-
-// WT[ci][co * taps + d] = W[co][ci][d] (bf16), the data-gradient GEMM's weight rows
-__global__ void k_transpose_w(const bf16* __restrict__ w, bf16* __restrict__ wt, int cout, int cin, int kk2) {
-  const long total = (long)cout * cin * kk2;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-    const int d = (int)(i % kk2);
-    const long r = i / kk2;
-    const int ci = (int)(r % cin), co = (int)(r / cin);
-    wt[((long)ci * cout + co) * kk2 + d] = w[i];
-  }
-}
-
-// vec: the vector-operand form (image width >= 8; for BWD_DATA a.wt is the transposed copy)
-template <int MODE>
-static void launch_gemm(const GemmArgs& a, int ks, dim3 g, hipStream_t st, bool vec) {
-  if (vec) {
-    if (ks == 3) hipLaunchKernelGGL((k_conv_gemm_vec<MODE, 3>), g, dim3(GT), 0, st, a);
-    else hipLaunchKernelGGL((k_conv_gemm_vec<MODE, 1>), g, dim3(GT), 0, st, a);
-  } else {
-    if (ks == 3) hipLaunchKernelGGL((k_conv_gemm<MODE, 3>), g, dim3(GT), 0, st, a);
-    else hipLaunchKernelGGL((k_conv_gemm<MODE, 1>), g, dim3(GT), 0, st, a);
-  }
-}
-
-static int ilog2(int v) {
-  int r = 0;
-  while ((1 << r) < v) ++r;
-  return r;
-}
-
-// dW = sum over chunks (fixed order); db[co] = sum over (b, p) of dZ (block partials, fixed order)
-__global__ void k_sum_chunks(const float* __restrict__ part, int chunks, long mn, float* __restrict__ out) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= mn) return;
-  float s = 0.f;
-  for (int c = 0; c < chunks; ++c) s += part[(long)c * mn + i];
-  out[i] = s;
-}
-
-// db[co] = sum over (b, p) of dZ: slice sums (grid cout x parts), then one fixed-order sum per
-// channel -- deterministic, and enough blocks to fill the GPU at full resolution
-__global__ __launch_bounds__(256) void k_bias_partial(View dz, int batch, int hw_sh, long slice,
-                                                      double* __restrict__ part) {
-  __shared__ double red[4];
-  const int co = blockIdx.x, parts = gridDim.y;
-  const long total = (long)batch << hw_sh, hwm = (1L << hw_sh) - 1;
-  const long lo = blockIdx.y * slice, hi = min(total, lo + slice);
-  double s = 0.0;
-  for (long e = lo + threadIdx.x; e < hi; e += 256)
-    s += ((const float*)dz.p)[(((e >> hw_sh) * dz.ctot + co) << hw_sh) + (e & hwm)];
-  s = block_sum<256>(s, red);
-  if (threadIdx.x == 0) part[(long)co * parts + blockIdx.y] = s;
-}
-
-__global__ __launch_bounds__(64) void k_bias_final(const double* __restrict__ part, int parts,
-                                                   float* __restrict__ db) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < parts; i += 64) s += part[(long)blockIdx.x * parts + i];
-  s = wave_sum(s);
-  if (threadIdx.x == 0) db[blockIdx.x] = (float)s;
-}
-
-// Elementwise layers on a (pixel blocks x planes) grid: plane = b * C + c (one block row per
-// sample and channel), pixels of the plane strided over blockIdx.x; widths are powers of two.
-__device__ __forceinline__ int lg2(int v) { return __ffs(v) - 1; }
-
-// g <- g * (a > 0): gradient through the ReLU (a is the post-activation, bf16)
-__global__ void k_relu_grad(View g, View a) {
-  const int plane = blockIdx.y, b = plane / g.c, c = plane - b * g.c;
-  const int hw = g.h * g.w;
-  float* gp = (float*)g.p + ((long)b * g.ctot + c) * hw;
-  const bf16* ap = (const bf16*)a.p + ((long)b * a.ctot + c) * hw;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < hw; p += gridDim.x * blockDim.x)
-    if (!((float)ap[p] > 0.f)) gp[p] = 0.f;
-}
-
-// 2 x 2 max pooling; arg holds the winning offset (0..3) for the backward pass
-__global__ void k_pool_fwd(View in, View out, uint8_t* __restrict__ arg) {
-  const int plane = blockIdx.y, b = plane / out.c, c = plane - b * out.c;
-  const int ohw = out.h * out.w, osh = lg2(out.w);
-  const bf16* src = (const bf16*)in.p + ((long)b * in.ctot + c) * in.h * in.w;
-  bf16* dst = (bf16*)out.p + ((long)b * out.ctot + c) * ohw;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ohw; p += gridDim.x * blockDim.x) {
-    const int y = p >> osh, x = p & (out.w - 1);
-    float best = -INFINITY;
-    int bi = 0;
-    for (int q = 0; q < 4; ++q) {
-      const float v = (float)src[(2 * y + (q >> 1)) * in.w + 2 * x + (q & 1)];
-      if (v > best) {
-        best = v;
-        bi = q;
-      }
+      o[i >> 1] = i & 1 ? o[i >> 1] | (bits << 16) : bits;
+      am[i >> 2] |= bi << (8 * (i & 3));
     }
-    dst[p] = to_bf(best);
-    arg[(long)plane * ohw + p] = (uint8_t)bi;
+    *reinterpret_cast<uint4*>(out + px * cp + g) = make_uint4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<uint2*>(arg + px * cp + g) = make_uint2(am[0], am[1]);
   }
 }
 
-// gin (f32, the skip gradient already there) += scatter of gout to the winning offsets
-__global__ void k_pool_bwd(View gout, View gin, const uint8_t* __restrict__ arg) {
-  const int plane = blockIdx.y, b = plane / gout.c, c = plane - b * gout.c;
-  const int ohw = gout.h * gout.w, osh = lg2(gout.w);
-  const float* src = (const float*)gout.p + ((long)b * gout.ctot + c) * ohw;
-  float* dst = (float*)gin.p + ((long)b * gin.ctot + c) * gin.h * gin.w;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ohw; p += gridDim.x * blockDim.x) {
-    const int y = p >> osh, x = p & (gout.w - 1);
-    const int q = arg[(long)plane * ohw + p];
-    dst[(2 * y + (q >> 1)) * gin.w + 2 * x + (q & 1)] += src[p];
-  }
-}
-
-// nearest x2 upsampling (bf16) of in's channels into out's first channels, and its gradient
-// (sum of the four children)
-__global__ void k_up_fwd(View in, View out) {
-  const int plane = blockIdx.y, b = plane / in.c, c = plane - b * in.c;
-  const int ohw = out.h * out.w, osh = lg2(out.w);
-  const bf16* src = (const bf16*)in.p + ((long)b * in.ctot + c) * in.h * in.w;
-  bf16* dst = (bf16*)out.p + ((long)b * out.ctot + c) * ohw;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ohw; p += gridDim.x * blockDim.x) {
-    const int y = p >> osh, x = p & (out.w - 1);
-    dst[p] = src[(y >> 1) * in.w + (x >> 1)];
-  }
-}
-__global__ void k_up_bwd(View gout, View gin) {
-  const int plane = blockIdx.y, b = plane / gin.c, c = plane - b * gin.c;
-  const int ihw = gin.h * gin.w, ish = lg2(gin.w);
-  const float* src = (const float*)gout.p + ((long)b * gout.ctot + c) * gout.h * gout.w;
-  float* dst = (float*)gin.p + ((long)b * gin.ctot + c) * ihw;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ihw; p += gridDim.x * blockDim.x) {
-    const int y = p >> ish, x = p & (gin.w - 1);
-    dst[p] = src[(2 * y) * gout.w + 2 * x] + src[(2 * y) * gout.w + 2 * x + 1] + src[(2 * y + 1) * gout.w + 2 * x] +
-             src[(2 * y + 1) * gout.w + 2 * x + 1];
+// Gradient of the pooled tensor's input: the skip gradient already in gin plus gout at the winning
+// offsets, zeroed where the activation is not positive (its ReLU).  8 channels of one pooled pixel
+// (4 input pixels) per thread.
+__global__ __launch_bounds__(256) void k_pool_bwd(const float* __restrict__ gout, float* __restrict__ gin,
+                                                  const bf16* __restrict__ act, const uint8_t* __restrict__ arg, int cp,
+                                                  long total, int osh, int ow) {
+  const int groups = cp / 8;
+  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
+    const long px = e / groups;
+    const int g = (int)(e - px * groups) * 8, x = (int)(px & (ow - 1));
+    const long row = px >> osh;
+    const float4 ga = *reinterpret_cast<const float4*>(gout + px * cp + g);
+    const float4 gb = *reinterpret_cast<const float4*>(gout + px * cp + g + 4);
+    const float gv[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+    const uint2 am = *reinterpret_cast<const uint2*>(arg + px * cp + g);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long o = ((2 * row + (q >> 1)) * (2 * ow) + 2 * x + (q & 1)) * cp + g;
+      float4* p = reinterpret_cast<float4*>(gin + o);
+      const float4 u = p[0], w = p[1];
+      const uint4 a = *reinterpret_cast<const uint4*>(act + o);
+      const unsigned au[4] = {a.x, a.y, a.z, a.w};
+      float r[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const unsigned bi = ((i < 4 ? am.x : am.y) >> (8 * (i & 3))) & 0xffu;
+        if ((int)bi == q) r[i] += gv[i];
+        if (!(bf_val(i & 1 ? au[i >> 1] >> 16 : au[i >> 1] & 0xffffu) > 0.f)) r[i] = 0.f;
+      }
+      p[0] = make_float4(r[0], r[1], r[2], r[3]);
+      p[1] = make_float4(r[4], r[5], r[6], r[7]);
+    }
   }
 }
 
@@ -525,37 +814,19 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ y, const 
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// Adam on FP32 master weights; refreshes the BF16 copy
-__global__ void k_adam(float* __restrict__ w, float* __restrict__ mo, float* __restrict__ ve,
-                       const float* __restrict__ g, bf16* __restrict__ wb, long n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float m = b1 * mo[i] + (1.f - b1) * gi;
-  const float v = b2 * ve[i] + (1.f - b2) * gi * gi;
-  mo[i] = m;
-  ve[i] = v;
-  const float wn = w[i] - lr * (m / c1) / (sqrtf(v / c2) + eps);
-  w[i] = wn;
-  wb[i] = to_bf(wn);
-}
-
 __global__ void k_to_bf(const float* __restrict__ s, bf16* __restrict__ d, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) d[i] = to_bf(s[i]);
 }
 
-// (pixel blocks, planes) grid of an elementwise layer over `batch` samples of view v
-inline dim3 plane_grid(const View& v, int batch) {
-  const long hw = (long)v.h * v.w;
-  return dim3((unsigned)std::min<long>((hw + 255) / 256, 64), (unsigned)(batch * v.c));
+inline int ilog2(int v) {
+  int r = 0;
+  while ((1 << r) < v) ++r;
+  return r;
 }
-
-inline dim3 grid_of(long n) {
-  long b = (n + 255) / 256;
-  return dim3((unsigned)std::min<long>(b, 65535L * 4));
-}
+inline dim3 grid_of(long n) { return dim3((unsigned)std::min<long>((n + 255) / 256, 65535L * 4)); }
+// enough blocks of an element loop to fill the GPU, no more
+inline unsigned loop_blocks(long n) { return (unsigned)std::max<long>(1, std::min<long>((n + 255) / 256, 8192)); }
 
 }  // namespace
 
@@ -565,23 +836,25 @@ struct NnLayer {
   long woff, boff;  // offsets in the parameter vector
 };
 
+constexpr int NN_CHUNKS = 512;       // workgroups that share a layer's weight gradient, about
+constexpr int PREP_PARTS = 32;         // blocks per sample of the input's preparation
+constexpr int NN_FIRST_BLOCKS = 1024;  // blocks of the first and last layer's gradients
+
 struct NnNet {
   int s = 256, c = 32, batch = 8;
   std::vector<NnLayer> layers;
-  long nparam = 0;
+  LayerTable table{};
+  long nparam = 0, nfwd = 0, ngrad = 0;  // parameters; elements of the fragment arrays
   float *w = nullptr, *mo = nullptr, *ve = nullptr, *g = nullptr;
-  bf16* wb = nullptr;
-  bf16* wbt = nullptr;  // per layer [C_in][C_out x taps] transpose of wb (data-gradient weights)
-  double* bpart = nullptr;  // bias-gradient slice sums, 8c x BIAS_PARTS
-  float* partial = nullptr;
-  long partial_cap = 0;
+  bf16 *wb = nullptr, *wf = nullptr, *wg = nullptr;  // BF16 copies: plain, forward and data-gradient fragments
+  float* partial = nullptr;   // weight-gradient partial tiles
+  double* bpart = nullptr;    // bias-gradient partial sums
   double* lpart = nullptr;
   long step = 0;
-  // activations (bf16) and their gradients (f32)
   struct Buf {
-    int c, h;
-    bf16* a = nullptr;
-    float* g = nullptr;
+    int cp = 0, h = 0;
+    bf16* a = nullptr;   // activation
+    float* g = nullptr;  // its gradient
   };
   std::vector<Buf> bufs;
   uint8_t* arg[3] = {nullptr, nullptr, nullptr};
@@ -589,27 +862,29 @@ struct NnNet {
   float* gout = nullptr;
   float* lw = nullptr;    // s x s loss weight (NULL: uniform)
   double lw_sum = 0.0;    // sum of the weight (s^2 when uniform)
+  bf16* x = nullptr;      // batch x s x s
   bf16* target = nullptr; // batch x 2 x s x s (staging)
   hipStream_t stream = nullptr;
 };
 
-// Buffer indices (see build): 0 x, 1 a0, 2 cat0, 3 p0, 4 a1, 5 cat1, 6 p1, 7 a2, 8 cat2, 9 p2,
-// 10 a3, 11 bneck, 12 a4, 13 d2, 14 a5, 15 d1, 16 a6, 17 d0
-enum { B_X, B_A0, B_CAT0, B_P0, B_A1, B_CAT1, B_P1, B_A2, B_CAT2, B_P2, B_A3, B_BN, B_A4, B_D2, B_A5, B_D1, B_A6,
-       B_D0, B_COUNT };
-
-static View vw(const NnNet& n, int bi, int c0, int c, bool grad) {
-  const auto& b = n.bufs[bi];
-  const long hw = (long)b.h * b.h;
-  void* base = grad ? (void*)(b.g + (long)c0 * hw) : (void*)(b.a + (long)c0 * hw);
-  return View{base, c, b.c, b.h, b.h};
-}
+// Activations: A = first convolution of a level, E = encoder output, P = pooled, BN = bottleneck,
+// D = decoder output of a level.
+enum { B_A0, B_E0, B_P0, B_A1, B_E1, B_P1, B_A2, B_E2, B_P2, B_A3, B_BN, B_A4, B_D2, B_A5, B_D1, B_A6, B_D0, B_COUNT };
+// The 13 convolutions between them: layer, inputs (in1 < 0: one; else in0 is upsampled), output, level.
+struct ConvStep {
+  int layer, in0, in1, out, level;
+};
+static const ConvStep kSteps[13] = {{1, B_A0, -1, B_E0, 0},  {2, B_P0, -1, B_A1, 1},   {3, B_A1, -1, B_E1, 1},
+                                    {4, B_P1, -1, B_A2, 2},  {5, B_A2, -1, B_E2, 2},   {6, B_P2, -1, B_A3, 3},
+                                    {7, B_A3, -1, B_BN, 3},  {8, B_BN, B_E2, B_A4, 2}, {9, B_A4, -1, B_D2, 2},
+                                    {10, B_D2, B_E1, B_A5, 1}, {11, B_A5, -1, B_D1, 1}, {12, B_D1, B_E0, B_A6, 0},
+                                    {13, B_A6, -1, B_D0, 0}};
 
 int nn_layer_table(int c, std::vector<NnLayer>* out, long* nparam) {
-  const int tab[15][4] = {{1, c, 3, 1},          {c, c, 3, 1},          {c, 2 * c, 3, 1},     {2 * c, 2 * c, 3, 1},
-                          {2 * c, 4 * c, 3, 1},  {4 * c, 4 * c, 3, 1},  {4 * c, 8 * c, 3, 1}, {8 * c, 8 * c, 3, 1},
-                          {12 * c, 4 * c, 3, 1}, {4 * c, 4 * c, 3, 1},  {6 * c, 2 * c, 3, 1}, {2 * c, 2 * c, 3, 1},
-                          {3 * c, c, 3, 1},      {c, c, 3, 1},          {c, 2, 1, 0}};
+  const int tab[NN_LAYERS][4] = {{1, c, 3, 1},          {c, c, 3, 1},          {c, 2 * c, 3, 1},     {2 * c, 2 * c, 3, 1},
+                                 {2 * c, 4 * c, 3, 1},  {4 * c, 4 * c, 3, 1},  {4 * c, 8 * c, 3, 1}, {8 * c, 8 * c, 3, 1},
+                                 {12 * c, 4 * c, 3, 1}, {4 * c, 4 * c, 3, 1},  {6 * c, 2 * c, 3, 1}, {2 * c, 2 * c, 3, 1},
+                                 {3 * c, c, 3, 1},      {c, c, 3, 1},          {c, 2, 1, 0}};
   out->clear();
   long off = 0;
   for (auto& t : tab) {
@@ -621,129 +896,143 @@ int nn_layer_table(int c, std::vector<NnLayer>* out, long* nparam) {
     out->push_back(l);
   }
   *nparam = off;
-  return 15;
+  return NN_LAYERS;
 }
 
-static hipError_t conv_fwd(NnNet& n, int li, View x, View y, bool out_f32) {
-  const NnLayer& L = n.layers[li];
-  GemmArgs a{};
-  a.x = x;
-  a.y = y;
-  a.wt = n.wb + L.woff;
-  a.bias = n.w + L.boff;
+template <int NCO, int ROWS, bool GRAD>
+static long conv3_blocks(const ConvArgs& a, int out_tiles) {
+  const long tiles = (long)a.batch * ((a.w_px + 31) / 32) * ((a.h + 4 * ROWS - 1) / (4 * ROWS));
+  return (tiles + 7) / 8 * 8 * (out_tiles / NCO);
+}
+template <int NCO, int ROWS, bool GRAD>
+static hipError_t conv3_launch(ConvArgs a, int out_tiles, hipStream_t st) {
+  constexpr size_t lds = (size_t)((4 * ROWS + 2) * 34 * 4 + NCO * 9 * 2 * 64) * sizeof(uint4);
+  static_assert(lds <= 80 * 1024, "two workgroups per CU");
+  const hipError_t e = hipFuncSetAttribute((const void*)k_conv3<NCO, ROWS, GRAD>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  a.tiles_x = (a.w_px + 31) / 32;
+  a.tiles_y = (a.h + 4 * ROWS - 1) / (4 * ROWS);
+  a.groups = out_tiles / NCO;
+  const long blocks = conv3_blocks<NCO, ROWS, GRAD>(a, out_tiles);
+  if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_conv3<NCO, ROWS, GRAD>), dim3((unsigned)blocks), dim3(CT), lds, st, a);
+  return hipGetLastError();
+}
+// The largest tile that still gives the 256 CUs two workgroups each: two output tiles of 32 channels
+// halve the input reads, 16 rows halve the border; the small levels (32 x 32 and 64 x 64 pixels of 8
+// samples) run on finer tiles instead of on a quarter of the chip.
+template <bool GRAD>
+static hipError_t conv3(const ConvArgs& a, int out_tiles, hipStream_t st) {
+  constexpr long FULL = 512;
+  if (out_tiles % 2 == 0 && a.h > 8 && conv3_blocks<2, 4, GRAD>(a, out_tiles) >= FULL)
+    return conv3_launch<2, 4, GRAD>(a, out_tiles, st);
+  if (out_tiles % 2 == 0 && conv3_blocks<2, 2, GRAD>(a, out_tiles) >= FULL)
+    return conv3_launch<2, 2, GRAD>(a, out_tiles, st);
+  if (a.h > 8 && conv3_blocks<1, 4, GRAD>(a, out_tiles) >= FULL) return conv3_launch<1, 4, GRAD>(a, out_tiles, st);
+  return conv3_launch<1, 2, GRAD>(a, out_tiles, st);
+}
+
+static Src conv_src(const NnNet& n, const ConvStep& s) {
+  const auto& b0 = n.bufs[s.in0];
+  if (s.in1 < 0) return Src{b0.a, nullptr, b0.cp, 0, 0};
+  const auto& b1 = n.bufs[s.in1];
+  return Src{b0.a, b1.a, b0.cp, b1.cp, 1};
+}
+
+static hipError_t conv_fwd(NnNet& n, const ConvStep& s) {
+  const LayerMap& m = n.table.l[s.layer];
+  ConvArgs a{};
+  a.in = conv_src(n, s);
+  a.w = n.wf + m.foff;
+  a.bias = n.w + m.boff;
+  a.out0 = Dst{n.bufs[s.out].a, nullptr, m.cpo, 0, 0};
+  a.out0_tiles = m.cpo / 32;
+  a.cout = m.cout;
   a.batch = n.batch;
-  a.cin = L.cin;
-  a.cout = L.cout;
-  a.relu = L.relu;
-  a.out_f32 = out_f32 ? 1 : 0;
-  a.M = L.cout;
-  a.N = n.batch * x.h * x.w;
-  a.K = L.cin * L.ks * L.ks;
-  a.w_sh = ilog2(x.w);
-  a.hw_sh = ilog2(x.h * x.w);
-  a.vec_a = (a.K % 8 == 0 && L.woff % 8 == 0 && ((uintptr_t)n.wb & 15) == 0) ? 1 : 0;
-  dim3 g((a.N + TN - 1) / TN, (a.M + TM - 1) / TM, 1);
-  launch_gemm<GEMM_FWD>(a, L.ks, g, n.stream, x.w >= 8);
-  return hipGetLastError();
+  a.h = a.w_px = n.s >> s.level;
+  a.chunks = m.cpi / 32;
+  a.relu = n.layers[s.layer].relu;
+  return conv3<false>(a, m.cpo / 32, n.stream);
 }
 
-// dz: gradient w.r.t. the layer's pre-activation output (f32 view); x: its input (bf16 view);
-// dx (nullable): gradient w.r.t. the input, overwritten.
-static hipError_t conv_bwd(NnNet& n, int li, View x, View dz, View* dx) {
-  const NnLayer& L = n.layers[li];
-  const int kk2 = L.ks * L.ks;
-  {  // weight gradient, split over pixels
-    GemmArgs a{};
-    a.x = x;
-    a.y = dz;
-    a.batch = n.batch;
-    a.cin = L.cin;
-    a.cout = L.cout;
-    a.M = L.cout;
-    a.N = L.cin * kk2;
-    a.K = n.batch * x.h * x.w;
-    a.w_sh = ilog2(x.w);
-    a.hw_sh = ilog2(x.h * x.w);
-    int chunks = std::max(1, std::min(256, a.K / 4096));
-    a.kchunk = ((a.K + chunks - 1) / chunks + TK - 1) / TK * TK;
-    chunks = (a.K + a.kchunk - 1) / a.kchunk;
-    if ((long)chunks * a.M * a.N > n.partial_cap) return hipErrorInvalidValue;
-    a.partial = n.partial;
-    dim3 g((a.N + TN - 1) / TN, (a.M + TM - 1) / TM, chunks);
-    launch_gemm<GEMM_BWD_W>(a, L.ks, g, n.stream, x.w >= 8);
-    const long mn = (long)a.M * a.N;
-    hipLaunchKernelGGL(k_sum_chunks, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, n.stream, n.partial, chunks,
-                       mn, n.g + L.woff);
-    {
-      const int hw_sh = ilog2(dz.h * dz.w);
-      const long total = (long)n.batch << hw_sh;
-      const int parts = (int)std::max<long>(1, std::min<long>(BIAS_PARTS, total / 4096));
-      const long slice = (total + parts - 1) / parts;
-      hipLaunchKernelGGL(k_bias_partial, dim3(L.cout, parts), dim3(256), 0, n.stream, dz, n.batch, hw_sh, slice,
-                         n.bpart);
-      hipLaunchKernelGGL(k_bias_final, dim3(L.cout), dim3(64), 0, n.stream, n.bpart, parts, n.g + L.boff);
-    }
-  }
-  if (dx) {
-    GemmArgs a{};
-    a.x = dz;
-    a.y = *dx;
-    const bool vec = dz.w >= 8;
-    a.wt = (vec ? n.wbt : n.wb) + L.woff;
-    a.batch = n.batch;
-    a.cin = L.cin;
-    a.cout = L.cout;
-    a.M = L.cin;
-    a.N = n.batch * dz.h * dz.w;
-    a.K = L.cout * kk2;
-    a.w_sh = ilog2(dz.w);
-    a.hw_sh = ilog2(dz.h * dz.w);
-    a.vec_a = (a.K % 8 == 0 && L.woff % 8 == 0 && ((uintptr_t)n.wbt & 15) == 0) ? 1 : 0;
-    dim3 g((a.N + TN - 1) / TN, (a.M + TM - 1) / TM, 1);
-    launch_gemm<GEMM_BWD_DATA>(a, L.ks, g, n.stream, vec);
-  }
-  return hipGetLastError();
+// The share of a layer's 8 x 32-pixel tiles: about NN_CHUNKS workgroups in all.
+static int wgrad_chunks(const LayerMap& m, int batch, int hw) {
+  const long tiles = (long)batch * ((hw + WG_R - 1) / WG_R) * ((hw + 31) / 32);
+  const int pairs = (m.cpo / 32) * (m.cpi / 32);
+  return (int)std::max<long>(1, std::min<long>(tiles, (NN_CHUNKS + pairs - 1) / pairs));
 }
 
+// n.bufs[s.out].g holds the gradient of the layer's pre-activation output; makes the parameters'
+// gradient and the inputs' (masked by their ReLU, where no pooling gradient is still to be added).
+static hipError_t conv_bwd(NnNet& n, const ConvStep& s) {
+  const LayerMap& m = n.table.l[s.layer];
+  const int hw = n.s >> s.level;
+  const float* dz = n.bufs[s.out].g;
+  {
+    WgradArgs a{};
+    a.x = conv_src(n, s);
+    a.dz = dz;
+    a.part = n.partial;
+    a.bpart = n.bpart;
+    a.batch = n.batch;
+    a.h = a.w_px = hw;
+    a.cpo = m.cpo;
+    a.tiles_o = m.cpo / 32;
+    a.tiles_i = m.cpi / 32;
+    a.tiles_x = (hw + 31) / 32;
+    a.tiles_y = (hw + WG_R - 1) / WG_R;
+    a.chunks = wgrad_chunks(m, n.batch, hw);
+    constexpr size_t lds = 32 * WG_ZP + 3 * 32 * WG_XP;
+    static_assert(lds >= 9 * 1024 * sizeof(float) && lds <= 80 * 1024, "reduction scratch; two workgroups per CU");
+    const hipError_t e = hipFuncSetAttribute((const void*)k_wgrad3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_wgrad3, dim3((unsigned)(a.tiles_o * a.tiles_i * a.chunks)), dim3(CT), lds, n.stream, a);
+    hipLaunchKernelGGL(k_wgrad_sum, dim3((unsigned)(a.tiles_o * a.tiles_i * 9 * 32 + a.tiles_o)), dim3(256), 0, n.stream, m,
+                       n.partial, n.bpart, a.chunks, n.g);
+  }
+  ConvArgs a{};
+  a.in = Src{dz, nullptr, m.cpo, 0, 0};
+  a.w = n.wg + m.goff;
+  const auto& b0 = n.bufs[s.in0];
+  const bool pooled = s.in0 == B_P0 || s.in0 == B_P1 || s.in0 == B_P2;
+  a.out0 = Dst{b0.g, pooled ? nullptr : b0.a, b0.cp, 0, s.in1 >= 0 ? 1 : 0};
+  a.out0_tiles = b0.cp / 32;
+  if (s.in1 >= 0) a.out1 = Dst{n.bufs[s.in1].g, nullptr, n.bufs[s.in1].cp, 0, 0};
+  a.batch = n.batch;
+  a.h = a.w_px = hw;
+  a.chunks = m.cpo / 32;
+  return conv3<true>(a, m.cpi / 32, n.stream);
+}
+
+static void pool_fwd(NnNet& n, int in, int out, int lv) {
+  const auto& o = n.bufs[out];
+  const long total = (long)n.batch * o.h * o.h * (o.cp / 8);
+  hipLaunchKernelGGL(k_pool_fwd, dim3(loop_blocks(total)), dim3(256), 0, n.stream, n.bufs[in].a, o.a, n.arg[lv], o.cp,
+                     total, ilog2(o.h), o.h);
+}
+static void pool_bwd(NnNet& n, int in, int out, int lv) {
+  const auto& o = n.bufs[out];
+  const long total = (long)n.batch * o.h * o.h * (o.cp / 8);
+  hipLaunchKernelGGL(k_pool_bwd, dim3(loop_blocks(total)), dim3(256), 0, n.stream, o.g, n.bufs[in].g, n.bufs[in].a,
+                     n.arg[lv], o.cp, total, ilog2(o.h), o.h);
+}
 
 hipError_t nn_forward(NnNet& n) {
-  const int c = n.c;
-  hipError_t e;
-  auto fwd = [&](int li, View x, View y) { return conv_fwd(n, li, x, y, false); };
-  if ((e = fwd(0, vw(n, B_X, 0, 1, false), vw(n, B_A0, 0, c, false)))) return e;
-  if ((e = fwd(1, vw(n, B_A0, 0, c, false), vw(n, B_CAT0, 2 * c, c, false)))) return e;
-  View p0 = vw(n, B_P0, 0, c, false);
-  hipLaunchKernelGGL(k_pool_fwd, plane_grid(p0, n.batch), dim3(256), 0, n.stream, vw(n, B_CAT0, 2 * c, c, false), p0,
-                     n.arg[0]);
-  if ((e = fwd(2, p0, vw(n, B_A1, 0, 2 * c, false)))) return e;
-  if ((e = fwd(3, vw(n, B_A1, 0, 2 * c, false), vw(n, B_CAT1, 4 * c, 2 * c, false)))) return e;
-  View p1 = vw(n, B_P1, 0, 2 * c, false);
-  hipLaunchKernelGGL(k_pool_fwd, plane_grid(p1, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_CAT1, 4 * c, 2 * c, false), p1, n.arg[1]);
-  if ((e = fwd(4, p1, vw(n, B_A2, 0, 4 * c, false)))) return e;
-  if ((e = fwd(5, vw(n, B_A2, 0, 4 * c, false), vw(n, B_CAT2, 8 * c, 4 * c, false)))) return e;
-  View p2 = vw(n, B_P2, 0, 4 * c, false);
-  hipLaunchKernelGGL(k_pool_fwd, plane_grid(p2, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_CAT2, 8 * c, 4 * c, false), p2, n.arg[2]);
-  if ((e = fwd(6, p2, vw(n, B_A3, 0, 8 * c, false)))) return e;
-  if ((e = fwd(7, vw(n, B_A3, 0, 8 * c, false), vw(n, B_BN, 0, 8 * c, false)))) return e;
-  View up2 = vw(n, B_CAT2, 0, 8 * c, false);
-  hipLaunchKernelGGL(k_up_fwd, plane_grid(up2, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_BN, 0, 8 * c, false), up2);
-  if ((e = fwd(8, vw(n, B_CAT2, 0, 12 * c, false), vw(n, B_A4, 0, 4 * c, false)))) return e;
-  if ((e = fwd(9, vw(n, B_A4, 0, 4 * c, false), vw(n, B_D2, 0, 4 * c, false)))) return e;
-  View up1 = vw(n, B_CAT1, 0, 4 * c, false);
-  hipLaunchKernelGGL(k_up_fwd, plane_grid(up1, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_D2, 0, 4 * c, false), up1);
-  if ((e = fwd(10, vw(n, B_CAT1, 0, 6 * c, false), vw(n, B_A5, 0, 2 * c, false)))) return e;
-  if ((e = fwd(11, vw(n, B_A5, 0, 2 * c, false), vw(n, B_D1, 0, 2 * c, false)))) return e;
-  View up0 = vw(n, B_CAT0, 0, 2 * c, false);
-  hipLaunchKernelGGL(k_up_fwd, plane_grid(up0, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_D1, 0, 2 * c, false), up0);
-  if ((e = fwd(12, vw(n, B_CAT0, 0, 3 * c, false), vw(n, B_A6, 0, c, false)))) return e;
-  if ((e = fwd(13, vw(n, B_A6, 0, c, false), vw(n, B_D0, 0, c, false)))) return e;
-  View out{n.out, 2, 2, n.s, n.s};
-  if ((e = conv_fwd(n, 14, vw(n, B_D0, 0, c, false), out, true))) return e;
+  const LayerMap &f = n.table.l[0], &l = n.table.l[14];
+  const long npx = (long)n.batch * n.s * n.s;
+  for (int cg = 0; cg < f.cpo / 8; cg += 32)
+    hipLaunchKernelGGL(k_first_fwd, dim3((unsigned)std::max<long>(1, std::min<long>(2048, npx / 64))), dim3(256), 0,
+                       n.stream, n.x, n.wb + f.woff, n.w + f.boff, n.bufs[B_A0].a, f.cout, f.cpo, cg, npx, ilog2(n.s), n.s);
+  for (const ConvStep& s : kSteps) {
+    const hipError_t e = conv_fwd(n, s);
+    if (e != hipSuccess) return e;
+    if (s.out == B_E0) pool_fwd(n, B_E0, B_P0, 0);
+    if (s.out == B_E1) pool_fwd(n, B_E1, B_P1, 1);
+    if (s.out == B_E2) pool_fwd(n, B_E2, B_P2, 2);
+  }
+  hipLaunchKernelGGL(k_last_fwd, dim3(loop_blocks(npx)), dim3(256), 0, n.stream, n.bufs[B_D0].a, n.wb + l.woff,
+                     n.w + l.boff, n.out, l.cin, l.cpi, npx, (long)n.s * n.s);
   return hipGetLastError();
 }
 
@@ -759,82 +1048,30 @@ hipError_t nn_loss(NnNet& n, bool with_grad, int* nparts) {
 }
 
 hipError_t nn_backward(NnNet& n) {
-  const int c = n.c;
-  hipError_t e;
-  for (const NnLayer& L : n.layers) {
-    const long cnt = (long)L.cout * L.cin * L.ks * L.ks;
-    hipLaunchKernelGGL(k_transpose_w, grid_of(cnt), dim3(256), 0, n.stream, n.wb + L.woff, n.wbt + L.woff, L.cout,
-                       L.cin, L.ks * L.ks);
+  const LayerMap &f = n.table.l[0], &l = n.table.l[14];
+  const long ss = (long)n.s * n.s, npx = n.batch * ss;
+  {
+    const unsigned nb = (unsigned)std::max<long>(1, std::min<long>(NN_FIRST_BLOCKS, npx / 64));
+    for (int cg = 0; cg < l.cpi / 8; cg += 32)
+      hipLaunchKernelGGL(k_last_bwd, dim3(nb), dim3(256), 0, n.stream, n.gout, n.bufs[B_D0].a, n.wb + l.woff,
+                         n.bufs[B_D0].g, l.cin, l.cpi, cg, npx, ss, n.partial, n.bpart);
+    hipLaunchKernelGGL(k_last_sum, dim3(l.cin + 1, 2), dim3(64), 0, n.stream, n.partial, n.bpart, (int)nb, l.cin, l.cpi,
+                       n.g + l.woff, n.g + l.boff);
   }
-  auto relu_g = [&](View g, View a) {
-    hipLaunchKernelGGL(k_relu_grad, plane_grid(g, n.batch), dim3(256), 0, n.stream, g, a);
-  };
-  View gout{n.gout, 2, 2, n.s, n.s};
-  View gd0 = vw(n, B_D0, 0, c, true);
-  if ((e = conv_bwd(n, 14, vw(n, B_D0, 0, c, false), gout, &gd0))) return e;
-  // level 0 decoder
-  relu_g(gd0, vw(n, B_D0, 0, c, false));
-  View ga6 = vw(n, B_A6, 0, c, true);
-  if ((e = conv_bwd(n, 13, vw(n, B_A6, 0, c, false), gd0, &ga6))) return e;
-  relu_g(ga6, vw(n, B_A6, 0, c, false));
-  View gcat0 = vw(n, B_CAT0, 0, 3 * c, true);
-  if ((e = conv_bwd(n, 12, vw(n, B_CAT0, 0, 3 * c, false), ga6, &gcat0))) return e;
-  View gd1 = vw(n, B_D1, 0, 2 * c, true);
-  hipLaunchKernelGGL(k_up_bwd, plane_grid(gd1, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_CAT0, 0, 2 * c, true), gd1);
-  // level 1 decoder
-  relu_g(gd1, vw(n, B_D1, 0, 2 * c, false));
-  View ga5 = vw(n, B_A5, 0, 2 * c, true);
-  if ((e = conv_bwd(n, 11, vw(n, B_A5, 0, 2 * c, false), gd1, &ga5))) return e;
-  relu_g(ga5, vw(n, B_A5, 0, 2 * c, false));
-  View gcat1 = vw(n, B_CAT1, 0, 6 * c, true);
-  if ((e = conv_bwd(n, 10, vw(n, B_CAT1, 0, 6 * c, false), ga5, &gcat1))) return e;
-  View gd2 = vw(n, B_D2, 0, 4 * c, true);
-  hipLaunchKernelGGL(k_up_bwd, plane_grid(gd2, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_CAT1, 0, 4 * c, true), gd2);
-  // level 2 decoder
-  relu_g(gd2, vw(n, B_D2, 0, 4 * c, false));
-  View ga4 = vw(n, B_A4, 0, 4 * c, true);
-  if ((e = conv_bwd(n, 9, vw(n, B_A4, 0, 4 * c, false), gd2, &ga4))) return e;
-  relu_g(ga4, vw(n, B_A4, 0, 4 * c, false));
-  View gcat2 = vw(n, B_CAT2, 0, 12 * c, true);
-  if ((e = conv_bwd(n, 8, vw(n, B_CAT2, 0, 12 * c, false), ga4, &gcat2))) return e;
-  View gbn = vw(n, B_BN, 0, 8 * c, true);
-  hipLaunchKernelGGL(k_up_bwd, plane_grid(gbn, n.batch), dim3(256), 0, n.stream,
-                     vw(n, B_CAT2, 0, 8 * c, true), gbn);
-  // bottleneck
-  relu_g(gbn, vw(n, B_BN, 0, 8 * c, false));
-  View ga3 = vw(n, B_A3, 0, 8 * c, true);
-  if ((e = conv_bwd(n, 7, vw(n, B_A3, 0, 8 * c, false), gbn, &ga3))) return e;
-  relu_g(ga3, vw(n, B_A3, 0, 8 * c, false));
-  View gp2 = vw(n, B_P2, 0, 4 * c, true);
-  if ((e = conv_bwd(n, 6, vw(n, B_P2, 0, 4 * c, false), ga3, &gp2))) return e;
-  View ge2 = vw(n, B_CAT2, 8 * c, 4 * c, true);
-  hipLaunchKernelGGL(k_pool_bwd, plane_grid(gp2, n.batch), dim3(256), 0, n.stream, gp2, ge2, n.arg[2]);
-  // level 2 encoder
-  relu_g(ge2, vw(n, B_CAT2, 8 * c, 4 * c, false));
-  View ga2 = vw(n, B_A2, 0, 4 * c, true);
-  if ((e = conv_bwd(n, 5, vw(n, B_A2, 0, 4 * c, false), ge2, &ga2))) return e;
-  relu_g(ga2, vw(n, B_A2, 0, 4 * c, false));
-  View gp1 = vw(n, B_P1, 0, 2 * c, true);
-  if ((e = conv_bwd(n, 4, vw(n, B_P1, 0, 2 * c, false), ga2, &gp1))) return e;
-  View ge1 = vw(n, B_CAT1, 4 * c, 2 * c, true);
-  hipLaunchKernelGGL(k_pool_bwd, plane_grid(gp1, n.batch), dim3(256), 0, n.stream, gp1, ge1, n.arg[1]);
-  // level 1 encoder
-  relu_g(ge1, vw(n, B_CAT1, 4 * c, 2 * c, false));
-  View ga1 = vw(n, B_A1, 0, 2 * c, true);
-  if ((e = conv_bwd(n, 3, vw(n, B_A1, 0, 2 * c, false), ge1, &ga1))) return e;
-  relu_g(ga1, vw(n, B_A1, 0, 2 * c, false));
-  View gp0 = vw(n, B_P0, 0, c, true);
-  if ((e = conv_bwd(n, 2, vw(n, B_P0, 0, c, false), ga1, &gp0))) return e;
-  View ge0 = vw(n, B_CAT0, 2 * c, c, true);
-  hipLaunchKernelGGL(k_pool_bwd, plane_grid(gp0, n.batch), dim3(256), 0, n.stream, gp0, ge0, n.arg[0]);
-  // level 0 encoder
-  relu_g(ge0, vw(n, B_CAT0, 2 * c, c, false));
-  View ga0 = vw(n, B_A0, 0, c, true);
-  if ((e = conv_bwd(n, 1, vw(n, B_A0, 0, c, false), ge0, &ga0))) return e;
-  relu_g(ga0, vw(n, B_A0, 0, c, false));
-  if ((e = conv_bwd(n, 0, vw(n, B_X, 0, 1, false), ga0, nullptr))) return e;
+  for (int i = 12; i >= 0; --i) {
+    const ConvStep& s = kSteps[i];
+    // the encoder outputs' gradients are whole once their pooled tensor's is there
+    if (s.out == B_E0) pool_bwd(n, B_E0, B_P0, 0);
+    if (s.out == B_E1) pool_bwd(n, B_E1, B_P1, 1);
+    if (s.out == B_E2) pool_bwd(n, B_E2, B_P2, 2);
+    const hipError_t e = conv_bwd(n, s);
+    if (e != hipSuccess) return e;
+  }
+  const unsigned nb = (unsigned)std::max<long>(1, std::min<long>(NN_FIRST_BLOCKS, npx / 64));
+  hipLaunchKernelGGL(k_first_wgrad, dim3(nb, f.cpo / 32), dim3(256), 0, n.stream, n.x, n.bufs[B_A0].g, f.cpo, npx,
+                     ilog2(n.s), n.s, n.partial, n.bpart);
+  hipLaunchKernelGGL(k_first_sum, dim3(f.cout, 10), dim3(64), 0, n.stream, n.partial, n.bpart, (int)nb, f.cpo,
+                     n.g + f.woff, n.g + f.boff);
   return hipGetLastError();
 }
 
@@ -842,13 +1079,14 @@ hipError_t nn_adam(NnNet& n, float lr) {
   n.step += 1;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = (float)(1.0 - std::pow(0.9, (double)n.step)), c2 = (float)(1.0 - std::pow(0.999, (double)n.step));
-  hipLaunchKernelGGL(k_adam, dim3((unsigned)((n.nparam + 255) / 256)), dim3(256), 0, n.stream, n.w, n.mo, n.ve, n.g,
-                     n.wb, n.nparam, lr, b1, b2, eps, c1, c2);
+  hipLaunchKernelGGL(k_adam, dim3((unsigned)((n.nparam + 255) / 256)), dim3(256), 0, n.stream, n.table, n.w, n.mo, n.ve,
+                     n.g, n.wb, n.wf, n.wg, n.nparam, lr, b1, b2, eps, c1, c2);
   return hipGetLastError();
 }
 
 hipError_t nn_refresh_bf16(NnNet& n) {
-  hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((n.nparam + 255) / 256)), dim3(256), 0, n.stream, n.w, n.wb, n.nparam);
+  hipLaunchKernelGGL(k_pack, dim3((unsigned)((n.nparam + 255) / 256)), dim3(256), 0, n.stream, n.table, n.w, n.nparam,
+                     n.wb, n.wf, n.wg);
   return hipGetLastError();
 }
 
@@ -864,23 +1102,36 @@ hipError_t nn_create(NnNet& n, int s, int c, int batch) {
   n.batch = batch;
   n.lw_sum = (double)s * s;
   nn_layer_table(c, &n.layers, &n.nparam);
-  const int ch[B_COUNT] = {1, c, 3 * c, c, 2 * c, 6 * c, 2 * c, 4 * c, 12 * c, 4 * c, 8 * c, 8 * c, 4 * c, 4 * c,
-                           2 * c, 2 * c, c, c};
-  const int lv[B_COUNT] = {0, 0, 0, 1, 1, 1, 2, 2, 2, 3, 3, 3, 2, 2, 1, 1, 0, 0};
+  const int ch[B_COUNT] = {c, c, c, 2 * c, 2 * c, 2 * c, 4 * c, 4 * c, 4 * c, 8 * c, 8 * c, 4 * c, 4 * c, 2 * c, 2 * c, c, c};
+  const int lv[B_COUNT] = {0, 0, 1, 1, 1, 2, 2, 2, 3, 3, 3, 2, 2, 1, 1, 0, 0};
+  for (int i = 0; i < NN_LAYERS; ++i) {
+    const NnLayer& L = n.layers[i];
+    LayerMap& m = n.table.l[i];
+    m = LayerMap{L.woff, L.boff, 0, 0, L.cin, L.cout, L.ks, L.cin, pad32(L.cin), pad32(L.cin), pad32(L.cout)};
+  }
+  for (const ConvStep& st : kSteps) {
+    LayerMap& m = n.table.l[st.layer];
+    m.c0 = ch[st.in0];
+    m.cp0 = pad32(m.c0);
+    m.cpi = m.cp0 + (st.in1 >= 0 ? pad32(ch[st.in1]) : 0);
+    m.foff = n.nfwd;
+    m.goff = n.ngrad;
+    n.nfwd += (long)m.cpo * m.cpi * 9;
+    n.ngrad += (long)m.cpo * m.cpi * 9;
+  }
   n.bufs.resize(B_COUNT);
   hipError_t e = hipSuccess;
   for (int i = 0; i < B_COUNT && e == hipSuccess; ++i) {
-    n.bufs[i].c = ch[i];
+    n.bufs[i].cp = pad32(ch[i]);
     n.bufs[i].h = s >> lv[i];
-    const size_t cnt = (size_t)batch * ch[i] * n.bufs[i].h * n.bufs[i].h;
+    const size_t cnt = (size_t)batch * n.bufs[i].cp * n.bufs[i].h * n.bufs[i].h;
     e = nn_alloc1((void**)&n.bufs[i].a, cnt * sizeof(bf16));
     if (e == hipSuccess) e = nn_alloc1((void**)&n.bufs[i].g, cnt * sizeof(float));
   }
-  for (int l = 0; l < 3 && e == hipSuccess; ++l) {
-    const size_t cnt = (size_t)batch * (c << l) * (s >> (l + 1)) * (s >> (l + 1));
-    e = nn_alloc1((void**)&n.arg[l], cnt);
-  }
+  for (int l = 0; l < 3 && e == hipSuccess; ++l)
+    e = nn_alloc1((void**)&n.arg[l], (size_t)batch * pad32(c << l) * (s >> (l + 1)) * (s >> (l + 1)));
   const size_t outc = (size_t)batch * 2 * s * s;
+  if (e == hipSuccess) e = nn_alloc1((void**)&n.x, outc / 2 * sizeof(bf16));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.out, outc * sizeof(float));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.gout, outc * sizeof(float));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.target, outc * sizeof(bf16));
@@ -889,23 +1140,20 @@ hipError_t nn_create(NnNet& n, int s, int c, int batch) {
   if (e == hipSuccess) e = nn_alloc1((void**)&n.ve, n.nparam * sizeof(float));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.g, n.nparam * sizeof(float));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.wb, n.nparam * sizeof(bf16));
-  if (e == hipSuccess) e = nn_alloc1((void**)&n.wbt, n.nparam * sizeof(bf16));
-  if (e == hipSuccess) e = nn_alloc1((void**)&n.bpart, (size_t)8 * c * BIAS_PARTS * sizeof(double));
+  if (e == hipSuccess) e = nn_alloc1((void**)&n.wf, n.nfwd * sizeof(bf16));
+  if (e == hipSuccess) e = nn_alloc1((void**)&n.wg, n.ngrad * sizeof(bf16));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.lpart, 1024 * sizeof(double));
-  // weight-gradient partial tiles: the largest chunks x Cout x Cin ks^2 over the layers
-  static const int level[15] = {0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0, 0};
-  long cap = 0;
-  for (size_t li = 0; li < n.layers.size(); ++li) {
-    const NnLayer& L = n.layers[li];
-    const int hh = s >> level[li];
-    const long K = (long)batch * hh * hh;
-    const int chunks = std::max(1, std::min(256, (int)(K / 4096)));
-    const long kc = ((K + chunks - 1) / chunks + TK - 1) / TK * TK;
-    const long nch = (K + kc - 1) / kc;
-    cap = std::max(cap, nch * L.cout * L.cin * L.ks * L.ks);
+  // partial sums of the gradients: the most any layer needs
+  const LayerMap &f = n.table.l[0], &l = n.table.l[14];
+  size_t part = std::max<size_t>((size_t)NN_FIRST_BLOCKS * std::max(9 * f.cpo, 2 * l.cpi), (size_t)batch * PREP_PARTS), bias = (size_t)NN_FIRST_BLOCKS * std::max(f.cpo, 2);
+  for (const ConvStep& st : kSteps) {
+    const LayerMap& m = n.table.l[st.layer];
+    const size_t chunks = wgrad_chunks(m, batch, s >> st.level);
+    part = std::max(part, chunks * m.cpo * m.cpi * 9);
+    bias = std::max(bias, chunks * m.cpo);
   }
-  n.partial_cap = cap;
-  if (e == hipSuccess) e = nn_alloc1((void**)&n.partial, cap * sizeof(float));
+  if (e == hipSuccess) e = nn_alloc1((void**)&n.partial, part * sizeof(float));
+  if (e == hipSuccess) e = nn_alloc1((void**)&n.bpart, bias * sizeof(double));
   if (e == hipSuccess) e = hipDeviceSynchronize();
   return e;
 }
@@ -918,8 +1166,8 @@ void nn_free(NnNet& n) {
   n.bufs.clear();
   for (auto& p : n.arg)
     if (p) hipFree(p);
-  for (void* p : {(void*)n.out, (void*)n.gout, (void*)n.target, (void*)n.w, (void*)n.mo, (void*)n.ve, (void*)n.g,
-                  (void*)n.wb, (void*)n.wbt, (void*)n.bpart, (void*)n.lpart, (void*)n.partial, (void*)n.lw})
+  for (void* p : {(void*)n.x, (void*)n.out, (void*)n.gout, (void*)n.target, (void*)n.w, (void*)n.mo, (void*)n.ve, (void*)n.g,
+                  (void*)n.wb, (void*)n.wf, (void*)n.wg, (void*)n.bpart, (void*)n.lpart, (void*)n.partial, (void*)n.lw})
     if (p) hipFree(p);
 }
 
@@ -933,18 +1181,26 @@ __global__ void k_gather_rows(const bf16* __restrict__ src, const int64_t* __res
   }
 }
 
-// Network input from raw amplitudes, one block per sample: x = log(1 + max(A, 0)) / max over the
-// sample (a sample whose maximum is 0 maps to 0).
-__global__ __launch_bounds__(256) void k_prep_amplitudes(const float* __restrict__ amp, long ss,
-                                                         bf16* __restrict__ x) {
+// Network input from raw amplitudes: x = log(1 + max(A, 0)) / max over the sample (a sample whose
+// maximum is 0 maps to 0), in two passes of PREP_PARTS blocks per sample: the parts' maxima, then the
+// values.  (One block per sample ran on as many CUs as there are samples: 243 us for 8 of 256 x 256.)
+__global__ __launch_bounds__(256) void k_prep_max(const float* __restrict__ amp, long ss, float* __restrict__ part) {
   __shared__ float red[4];
-  const float* a = amp + blockIdx.x * ss;
-  bf16* o = x + blockIdx.x * ss;
+  const float* a = amp + blockIdx.y * ss;
   float mx = 0.f;
-  for (long i = threadIdx.x; i < ss; i += 256) mx = fmaxf(mx, log1pf(fmaxf(a[i], 0.f)));
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < ss; i += PREP_PARTS * 256)
+    mx = fmaxf(mx, log1pf(fmaxf(a[i], 0.f)));
   mx = block_max<256>(mx, red);
+  if (threadIdx.x == 0) part[blockIdx.y * PREP_PARTS + blockIdx.x] = mx;
+}
+__global__ __launch_bounds__(256) void k_prep_amplitudes(const float* __restrict__ amp, long ss,
+                                                         const float* __restrict__ part, bf16* __restrict__ x) {
+  const float* a = amp + blockIdx.y * ss;
+  bf16* o = x + blockIdx.y * ss;
+  const float mx = wave_max(part[blockIdx.y * PREP_PARTS + (threadIdx.x & (PREP_PARTS - 1))]);
   const float inv = mx > 0.f ? 1.f / mx : 0.f;
-  for (long i = threadIdx.x; i < ss; i += 256) o[i] = to_bf(log1pf(fmaxf(a[i], 0.f)) * inv);
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < ss; i += PREP_PARTS * 256)
+    o[i] = to_bf(log1pf(fmaxf(a[i], 0.f)) * inv);
 }
 
 }  // namespace ptyk
@@ -1155,7 +1411,7 @@ static int net_load_batch(ptyk_net* h, const int64_t* order, int64_t off) {
   }
   NCHK(h, hipMemcpyAsync(h->idx, order + off, B * sizeof(int64_t), hipMemcpyHostToDevice, h->n.stream));
   hipLaunchKernelGGL(k_gather_rows, grid_of((long)B * ss), dim3(256), 0, h->n.stream, h->data_x, h->idx, ss, B,
-                     h->n.bufs[B_X].a);
+                     h->n.x);
   hipLaunchKernelGGL(k_gather_rows, grid_of((long)B * 2 * ss), dim3(256), 0, h->n.stream, h->data_y, h->idx, 2 * ss,
                      B, h->n.target);
   NCHK(h, hipStreamSynchronize(h->n.stream));  // the order slice is host memory of the caller
@@ -1243,11 +1499,13 @@ static int net_predict(ptyk_net* h, const float* inputs, int64_t n, float* outpu
       e = hipMemcpyAsync(stage, inputs + off * ss, (size_t)cnt * ss * sizeof(float), hipMemcpyHostToDevice,
                          h->n.stream);
     if (e == hipSuccess) {
-      if (raw)
-        hipLaunchKernelGGL(k_prep_amplitudes, dim3(B), dim3(256), 0, h->n.stream, stage, ss, h->n.bufs[B_X].a);
-      else
+      if (raw) {
+        float* part = h->n.partial;  // scratch of the gradients
+        hipLaunchKernelGGL(k_prep_max, dim3(PREP_PARTS, B), dim3(256), 0, h->n.stream, stage, ss, part);
+        hipLaunchKernelGGL(k_prep_amplitudes, dim3(PREP_PARTS, B), dim3(256), 0, h->n.stream, stage, ss, part, h->n.x);
+      } else
         hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((B * ss + 255) / 256)), dim3(256), 0, h->n.stream, stage,
-                           h->n.bufs[B_X].a, (long)(B * ss));
+                           h->n.x, (long)(B * ss));
       e = nn_forward(h->n);
     }
     if (e == hipSuccess)
@@ -1280,7 +1538,7 @@ int ptyk_net_gradient(ptyk_net* h, const float* inputs, const float* targets, do
   hipError_t e = hipMemcpyAsync(stage, inputs, (size_t)B * ss * sizeof(float), hipMemcpyHostToDevice, h->n.stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((B * ss + 255) / 256)), dim3(256), 0, h->n.stream, stage,
-                       h->n.bufs[B_X].a, (long)(B * ss));
+                       h->n.x, (long)(B * ss));
     e = hipStreamSynchronize(h->n.stream);
   }
   if (e == hipSuccess)

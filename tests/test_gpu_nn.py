@@ -173,3 +173,26 @@ def test_streamed_samples_equal_one_shot_samples():
         order = np.array([5, 0, 3, 2, 1, 4])
         assert a.train(order, 1e-3) == b.train(order, 1e-3)
         np.testing.assert_array_equal(a.get_params(), b.get_params())
+
+
+@pytest.mark.parametrize("s,c,batch", [(256, 32, 16), (64, 32, 64), (8, 3, 4)])
+def test_tile_shapes_agree_between_batch_sizes(s, c, batch):
+    """The convolutions' tile shapes follow the number of workgroups, so a batch of many samples and
+    one of a single sample run different kernels; each output is the same sum in the same order.  The
+    batch's gradient is the mean of its samples' (a power-of-two batch scales them exactly): only the
+    FP32 order of the pixel sums differs, about 1e-6 of a layer's norm over at most 2^20 pixels."""
+    rng = np.random.default_rng(s)
+    x, t = sample(rng, batch, s)
+    with warmstart.Net(size=s, c=c, batch=batch, seed=4) as big, warmstart.Net(size=s, c=c, batch=1, seed=4) as one:
+        sl, _ = layer_slices(c)
+        p = big.get_params()
+        for _, b in sl:
+            p[b] = rng.normal(0, 0.05, size=b.stop - b.start)
+        big.set_params(p)
+        one.set_params(p)
+        np.testing.assert_array_equal(big.predict(x), one.predict(x))
+        _, g = big.gradient(x, t)
+        gs = np.mean([one.gradient(x[i:i + 1], t[i:i + 1])[1].astype(np.float64) for i in range(batch)], axis=0)
+    for li, (wl, bl) in enumerate(sl):
+        for part in (wl, bl):
+            assert rel(g[part], gs[part]) <= 1e-4, (li, rel(g[part], gs[part]))
