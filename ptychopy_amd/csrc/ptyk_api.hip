@@ -51,8 +51,8 @@ struct ptyk_ctx {
   int cus = 0;  // compute units of the device
   // DM state
   float2* psi = nullptr;
-  int* row_ptr = nullptr;
-  int* row_frames = nullptr;
+  int* tile_ptr = nullptr;
+  int* tile_frames = nullptr;
   double2* probe_partial = nullptr;
   double* obj_partial = nullptr;
   double* probe_partial_sum = nullptr;
@@ -68,8 +68,8 @@ struct ptyk_ctx {
   int dm_wave = 0, dm_waves = 0;
   double2* d_obj = nullptr;
   double2* d_probe = nullptr;
-  int* wave_row_ptr = nullptr;
-  int* wave_row_frames = nullptr;
+  int* wave_tile_ptr = nullptr;
+  int* wave_tile_frames = nullptr;
   std::vector<int> wave_lo, wave_hi;
   // bumped whenever the DM launch tables or shapes may change (positions, tuning, a rebuild):
   // part of the batch graph signature, so a captured graph never replays stale row ranges
@@ -161,8 +161,8 @@ static void free_all(ptyk_ctx* c) {
     if (p) hipFree(p);
   void* ptrs[] = {c->tw, c->obj, c->obj_int, c->probe, c->probe_int, c->probe_tmp, c->amp, c->amp_scale,
                   c->amp_sum, c->avg, c->pos_dev, c->roi_dev, c->order_dev, c->scal, c->factors, c->e_psi_old,
-                  c->e_psi, c->e_flags, c->e_rowmax, c->e_err, c->psi, c->row_ptr, c->row_frames, c->probe_partial, c->obj_partial,
-                  c->probe_partial_sum, c->d_obj, c->d_probe, c->wave_row_ptr, c->wave_row_frames};
+                  c->e_psi, c->e_flags, c->e_rowmax, c->e_err, c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial,
+                  c->probe_partial_sum, c->d_obj, c->d_probe, c->wave_tile_ptr, c->wave_tile_frames};
   for (void* p : ptrs)
     if (p) hipFree(p);
   for (auto& e : c->ev)
@@ -318,16 +318,16 @@ int ptyk_get_frame_scales(ptyk_ctx* c, float* out) {
 
 // ---------------------------------------------------------------- positions
 static void free_dm(ptyk_ctx* c) {
-  void* ptrs[] = {c->psi, c->row_ptr, c->row_frames, c->probe_partial, c->obj_partial, c->probe_partial_sum,
-                  c->d_obj, c->d_probe, c->wave_row_ptr, c->wave_row_frames};
+  void* ptrs[] = {c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial, c->probe_partial_sum,
+                  c->d_obj, c->d_probe, c->wave_tile_ptr, c->wave_tile_frames};
   for (void* p : ptrs)
     if (p) hipFree(p);
   c->psi = nullptr;
-  c->row_ptr = c->row_frames = nullptr;
+  c->tile_ptr = c->tile_frames = nullptr;
   c->probe_partial = nullptr;
   c->obj_partial = c->probe_partial_sum = nullptr;
   c->d_obj = c->d_probe = nullptr;
-  c->wave_row_ptr = c->wave_row_frames = nullptr;
+  c->wave_tile_ptr = c->wave_tile_frames = nullptr;
   c->dm_wave = c->dm_waves = 0;
   c->dm_started = false;
   ++c->dm_gen;
@@ -359,15 +359,15 @@ int ptyk_set_positions(ptyk_ctx* c, const float* p) {
   c->have_pos = true;
   ++c->dm_gen;
   // DM's frame lists depend on the positions; rebuild them on the next DM call.
-  if (c->row_ptr) {
-    hipFree(c->row_ptr);
-    hipFree(c->row_frames);
-    c->row_ptr = c->row_frames = nullptr;
+  if (c->tile_ptr) {
+    hipFree(c->tile_ptr);
+    hipFree(c->tile_frames);
+    c->tile_ptr = c->tile_frames = nullptr;
   }
-  if (c->wave_row_ptr) {
-    hipFree(c->wave_row_ptr);
-    hipFree(c->wave_row_frames);
-    c->wave_row_ptr = c->wave_row_frames = nullptr;
+  if (c->wave_tile_ptr) {
+    hipFree(c->wave_tile_ptr);
+    hipFree(c->wave_tile_frames);
+    c->wave_tile_ptr = c->wave_tile_frames = nullptr;
     c->dm_wave = c->dm_waves = 0;
   }
   return PTYK_OK;
@@ -684,61 +684,60 @@ static int dm_wave_frames(const ptyk_ctx* c) {
   return (int)std::max(1L, std::min((long)n, w));
 }
 
+// Appends the CSR lists of frames [f0, f1) per object tile (ascending ids): dm_tiles + 1 offsets into
+// *frames, and the range of tile rows they touch.
+static void dm_tile_lists(const ptyk_ctx* c, int f0, int f1, std::vector<int>* ptr, std::vector<int>* frames, int* lo,
+                          int* hi) {
+  const int m = c->cfg.frame_size, tw = dm_tile_width(m), tc = dm_tile_cols(c->cfg.obj_cols, m), tr = dm_tile_rows(c->cfg.obj_rows);
+  std::vector<int> at((size_t)tr * tc + 1, 0);
+  int rlo = tr, rhi = 0;
+  auto tiles = [&](int j, auto&& visit) {
+    const int r0 = c->roi[j].x / PTYK_DM_TR, r1 = (c->roi[j].x + m - 1) / PTYK_DM_TR;
+    const int c0 = c->roi[j].y / tw, c1 = (c->roi[j].y + m - 1) / tw;
+    rlo = std::min(rlo, r0);
+    rhi = std::max(rhi, r1 + 1);
+    for (int r = r0; r <= r1; ++r)
+      for (int q = c0; q <= c1; ++q) visit(r * tc + q);
+  };
+  for (int j = f0; j < f1; ++j) tiles(j, [&](int t) { ++at[t + 1]; });
+  at[0] = (int)frames->size();
+  for (size_t t = 1; t < at.size(); ++t) at[t] += at[t - 1];
+  ptr->insert(ptr->end(), at.begin(), at.end());
+  frames->resize(at.back());
+  for (int j = f0; j < f1; ++j) tiles(j, [&](int t) { (*frames)[at[t]++] = j; });
+  if (lo) *lo = rlo;
+  if (hi) *hi = rhi;
+}
+
 static int dm_prepare(ptyk_ctx* c) {
   const int n = c->cfg.n_frames, m = c->cfg.frame_size, rows = c->cfg.obj_rows;
   int r = ensure_psi(c);
   if (r) return r;
   const int wave = dm_wave_frames(c);
-  if (wave == 0 && !c->row_ptr) {
-    // frames covering each object row, ascending frame id
-    std::vector<int> cnt(rows + 1, 0);
-    for (int j = 0; j < n; ++j)
-      for (int q = 0; q < m; ++q) cnt[c->roi[j].x + q + 1]++;
-    for (int p = 0; p < rows; ++p) cnt[p + 1] += cnt[p];
-    std::vector<int> fill(cnt.begin(), cnt.end() - 1), frames((size_t)n * m);
-    for (int j = 0; j < n; ++j)
-      for (int q = 0; q < m; ++q) frames[fill[c->roi[j].x + q]++] = j;
-    HIPCHK(c, dalloc(&c->row_ptr, rows + 1));
-    HIPCHK(c, dalloc(&c->row_frames, (size_t)n * m));
-    HIPCHK(c, hipMemcpyAsync(c->row_ptr, cnt.data(), (rows + 1) * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->row_frames, frames.data(), frames.size() * sizeof(int), hipMemcpyHostToDevice,
+  if (wave == 0 && !c->tile_ptr) {
+    std::vector<int> ptr, frames;
+    dm_tile_lists(c, 0, n, &ptr, &frames, nullptr, nullptr);
+    HIPCHK(c, dalloc(&c->tile_ptr, ptr.size()));
+    HIPCHK(c, dalloc(&c->tile_frames, frames.size()));
+    HIPCHK(c, hipMemcpyAsync(c->tile_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->tile_frames, frames.data(), frames.size() * sizeof(int), hipMemcpyHostToDevice,
                              c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));  // host vectors die at the end of this block
     ++c->dm_gen;
   }
   if (wave > 0 && c->dm_wave != wave) {
-    // per wave: frames covering each object row (offsets into one frame-id array)
+    // per wave: frames touching each object tile (offsets into one frame-id array)
     const int nw = (n + wave - 1) / wave;
-    std::vector<int> ptr((size_t)nw * (rows + 1)), frames((size_t)n * m);
-    std::vector<int> lo(nw), hi(nw);
-    int off = 0;
-    for (int w = 0; w < nw; ++w) {
-      const int f0 = w * wave, f1 = std::min(n, f0 + wave);
-      std::vector<int> cnt(rows + 1, 0);
-      int rlo = rows, rhi = 0;
-      for (int j = f0; j < f1; ++j) {
-        rlo = std::min(rlo, c->roi[j].x);
-        rhi = std::max(rhi, c->roi[j].x + m);
-        for (int q = 0; q < m; ++q) cnt[c->roi[j].x + q + 1]++;
-      }
-      for (int p = 0; p < rows; ++p) cnt[p + 1] += cnt[p];
-      int* wp = ptr.data() + (size_t)w * (rows + 1);
-      for (int p = 0; p <= rows; ++p) wp[p] = off + cnt[p];
-      std::vector<int> fill(rows);
-      for (int p = 0; p < rows; ++p) fill[p] = wp[p];
-      for (int j = f0; j < f1; ++j)
-        for (int q = 0; q < m; ++q) frames[fill[c->roi[j].x + q]++] = j;
-      off += cnt[rows];
-      lo[w] = rlo;
-      hi[w] = rhi;
-    }
-    if (c->wave_row_ptr) hipFree(c->wave_row_ptr);
-    if (c->wave_row_frames) hipFree(c->wave_row_frames);
-    c->wave_row_ptr = c->wave_row_frames = nullptr;
-    HIPCHK(c, dalloc(&c->wave_row_ptr, ptr.size()));
-    HIPCHK(c, dalloc(&c->wave_row_frames, frames.size()));
-    HIPCHK(c, hipMemcpyAsync(c->wave_row_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->wave_row_frames, frames.data(), frames.size() * sizeof(int), hipMemcpyHostToDevice,
+    std::vector<int> ptr, frames, lo(nw), hi(nw);
+    for (int w = 0; w < nw; ++w)
+      dm_tile_lists(c, w * wave, std::min(n, (w + 1) * wave), &ptr, &frames, &lo[w], &hi[w]);
+    if (c->wave_tile_ptr) hipFree(c->wave_tile_ptr);
+    if (c->wave_tile_frames) hipFree(c->wave_tile_frames);
+    c->wave_tile_ptr = c->wave_tile_frames = nullptr;
+    HIPCHK(c, dalloc(&c->wave_tile_ptr, ptr.size()));
+    HIPCHK(c, dalloc(&c->wave_tile_frames, frames.size()));
+    HIPCHK(c, hipMemcpyAsync(c->wave_tile_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->wave_tile_frames, frames.data(), frames.size() * sizeof(int), hipMemcpyHostToDevice,
                              c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));  // host vectors die at the end of this block
     c->wave_lo = lo;
@@ -747,7 +746,7 @@ static int dm_prepare(ptyk_ctx* c) {
     c->dm_waves = nw;
     ++c->dm_gen;
     if (!c->d_obj) HIPCHK(c, dalloc(&c->d_obj, (size_t)rows * c->cfg.obj_cols));
-    if (!c->d_probe) HIPCHK(c, dalloc(&c->d_probe, (size_t)c->mm));
+    if (!c->d_probe) HIPCHK(c, dalloc(&c->d_probe, (size_t)dm_wave_probe_chunks(m) * c->mm));
   }
   if (!c->probe_partial) {
     const int rpw = m >= PTYK_NT ? 1 : PTYK_NT / m;
@@ -756,7 +755,8 @@ static int dm_prepare(ptyk_ctx* c) {
     c->frames_per_chunk = (n + c->probe_chunks - 1) / c->probe_chunks;
     c->probe_chunks = (n + c->frames_per_chunk - 1) / c->frames_per_chunk;
     HIPCHK(c, dalloc(&c->probe_partial, (size_t)c->probe_chunks * c->mm));
-    HIPCHK(c, dalloc(&c->obj_partial, (size_t)rows * dm_obj_col_chunks(c->cfg.obj_cols)));
+    HIPCHK(c, dalloc(&c->obj_partial, (size_t)rows * std::max(dm_tile_cols(c->cfg.obj_cols, m),
+                                                              (c->cfg.obj_cols + PTYK_NT - 1) / PTYK_NT)));
     HIPCHK(c, dalloc(&c->probe_partial_sum, (size_t)std::max(gp, (int)((c->mm + PTYK_NT - 1) / PTYK_NT))));
   }
   if (!c->dm_started) {
@@ -804,10 +804,10 @@ static int dm_launch(ptyk_ctx* c, uint32_t flags, float* kernel_ms) {
     a.amp = c->amp;
     a.amp_scale = c->amp_scale;
     a.roi = c->roi_dev;
-    a.wave_row_ptr = c->wave_row_ptr;
-    a.wave_row_frames = c->wave_row_frames;
-    a.wave_row_lo = c->wave_lo.data();
-    a.wave_row_hi = c->wave_hi.data();
+    a.wave_tile_ptr = c->wave_tile_ptr;
+    a.wave_tile_frames = c->wave_tile_frames;
+    a.wave_tile_lo = c->wave_lo.data();
+    a.wave_tile_hi = c->wave_hi.data();
     a.d_obj = c->d_obj;
     a.d_probe = c->d_probe;
     a.obj_partial = c->obj_partial;
@@ -832,8 +832,8 @@ static int dm_launch(ptyk_ctx* c, uint32_t flags, float* kernel_ms) {
     a.amp = c->amp;
     a.amp_scale = c->amp_scale;
     a.roi = c->roi_dev;
-    a.row_ptr = c->row_ptr;
-    a.row_frames = c->row_frames;
+    a.tile_ptr = c->tile_ptr;
+    a.tile_frames = c->tile_frames;
     a.probe_partial = c->probe_partial;
     a.obj_partial = c->obj_partial;
     a.probe_partial_sum = c->probe_partial_sum;
@@ -1286,9 +1286,9 @@ struct ptyk_batch {
 };
 
 static std::vector<uintptr_t> dm_signature(const ptyk_ctx* c) {
-  return {(uintptr_t)c->psi, (uintptr_t)c->row_ptr, (uintptr_t)c->row_frames, (uintptr_t)c->probe_partial,
+  return {(uintptr_t)c->psi, (uintptr_t)c->tile_ptr, (uintptr_t)c->tile_frames, (uintptr_t)c->probe_partial,
           (uintptr_t)c->obj_partial, (uintptr_t)c->probe_partial_sum, (uintptr_t)c->d_obj, (uintptr_t)c->d_probe,
-          (uintptr_t)c->wave_row_ptr, (uintptr_t)c->wave_row_frames, (uintptr_t)c->dm_wave, (uintptr_t)c->dm_waves,
+          (uintptr_t)c->wave_tile_ptr, (uintptr_t)c->wave_tile_frames, (uintptr_t)c->dm_wave, (uintptr_t)c->dm_waves,
           (uintptr_t)c->probe_chunks, (uintptr_t)c->frames_per_chunk, (uintptr_t)dm_wave_frames(c),
           (uintptr_t)c->dm_gen};
 }

@@ -19,11 +19,12 @@
 //                      removes the need to keep psi_old or X.
 //   k_dm_rows_inv : psi_new = RowIFFT_u(Z)
 //   k_dm_probe_partial : probe increment partial sums over frame chunks (reads O at start)
-//   k_dm_object   : object increment gathered per object row over the frames that cover
-//                   it (CSR list, ascending frame id; reads P at start, rewrites O)
+//   k_dm_object   : object increment gathered per object tile over the frames that touch it
+//                   (CSR list, ascending frame id; reads P at start, rewrites O)
 //   k_dm_probe_apply : P += s_P * sum of partials (fixed chunk order)
 //   k_dm_finish   : FP64 sums -> objMax, probeMax; cached factor update (|delta| > 1e-3)
 #include "ptyk_device.h"
+#include "ptyk_dm_gather.h"
 #include "ptyk_internal.h"
 
 namespace ptyk {
@@ -35,8 +36,6 @@ struct DmCfg {
   static constexpr int PCPT = M >= PTYK_NT ? M / PTYK_NT : 1;   // probe columns per thread
   static constexpr int PRPW = M >= PTYK_NT ? 1 : PTYK_NT / M;   // probe rows per workgroup
 };
-
-#define PTYK_OBJ_CHUNK 256
 
 template <int M>
 __global__ __launch_bounds__(PTYK_NT) void k_dm_rows_fwd(float2* __restrict__ psi, const float2* __restrict__ obj,
@@ -209,50 +208,33 @@ __global__ __launch_bounds__(PTYK_NT) void k_dm_probe_apply(float2* __restrict__
   if (threadIdx.x == 0) block_sums[blockIdx.x] = acc;
 }
 
+// O += the increments (obj_row_sum; one rounding); per-block sum |O|^2.
 template <int M>
 __global__ __launch_bounds__(PTYK_NT) void k_dm_object(float2* __restrict__ obj, int obj_cols,
                                                        const float2* __restrict__ psi,
                                                        const float2* __restrict__ probe,
                                                        const int2* __restrict__ roi,
-                                                       const int* __restrict__ row_ptr,
-                                                       const int* __restrict__ row_frames,
+                                                       const int* __restrict__ tile_ptr,
+                                                       const int* __restrict__ tile_frames,
                                                        const float* __restrict__ factors, int phase_constraint,
                                                        double* __restrict__ block_sums) {
   __shared__ double red[PTYK_NT / 64];
-  const int p = blockIdx.x;
-  const int c = blockIdx.y * PTYK_OBJ_CHUNK + threadIdx.x;
-  const int cbeg = blockIdx.y * PTYK_OBJ_CHUNK;
-  const int cend = cbeg + PTYK_OBJ_CHUNK;
-  const float so = factors[1];
-  double ax = 0.0, ay = 0.0;
-  const int k0 = row_ptr[p], k1 = row_ptr[p + 1];
-  for (int k = k0; k < k1; ++k) {
-    const int j = row_frames[k];
-    const int2 r = roi[j];
-    if (r.y >= cend || r.y + M <= cbeg) continue;  // frame does not touch this column chunk
-    const int q = p - r.x;
-    const int cc = c - r.y;
-    if (c < obj_cols && cc >= 0 && cc < M) {
-      float2 u = cmulcj(probe[q * M + cc], psi[((long)j * M + q) * M + cc]);
-      u = cscale(u, so);
-      if (phase_constraint) u = clamp_phase(u);
-      ax += u.x;
-      ay += u.y;
-    }
-  }
+  constexpr int TC = dm_tile_width(M);
+  const int p = blockIdx.x, c = blockIdx.y * TC + threadIdx.x % TC;
+  const int t = p / PTYK_DM_TR * gridDim.y + blockIdx.y;
+  const double2 a = obj_row_sum<M>(p, c, psi, probe, roi, tile_frames, tile_ptr[t], tile_ptr[t + 1], factors[1],
+                                   phase_constraint);
   double s2 = 0.0;
-  if (c < obj_cols) {
+  if (threadIdx.x < TC && c < obj_cols) {
     float2 o = obj[(long)p * obj_cols + c];
-    o.x = (float)((double)o.x + ax);
-    o.y = (float)((double)o.y + ay);
+    o.x = (float)((double)o.x + a.x);
+    o.y = (float)((double)o.y + a.y);
     obj[(long)p * obj_cols + c] = o;
     s2 = (double)o.x * o.x + (double)o.y * o.y;
   }
   s2 = block_sum<PTYK_NT>(s2, red);
   if (threadIdx.x == 0) block_sums[(long)blockIdx.x * gridDim.y + blockIdx.y] = s2;
 }
-
-int dm_obj_col_chunks(int obj_cols) { return (obj_cols + PTYK_OBJ_CHUNK - 1) / PTYK_OBJ_CHUNK; }
 
 template <int M>
 static hipError_t dm_impl(const DmArgs& a, hipStream_t s, DmTimer* tm) {
@@ -276,15 +258,15 @@ static hipError_t dm_impl(const DmArgs& a, hipStream_t s, DmTimer* tm) {
     hipLaunchKernelGGL((k_dm_probe_partial<M>), dim3(gp, a.probe_chunks), dim3(PTYK_NT), 0, s, a.psi, a.obj,
                        a.obj_cols, a.roi, a.n_frames, a.frames_per_chunk, a.probe_partial);
   }
-  const int cch = dm_obj_col_chunks(a.obj_cols);
   rec(DM_T_OBJ_GATHER);
-  hipLaunchKernelGGL((k_dm_object<M>), dim3(a.obj_rows, cch), dim3(PTYK_NT), 0, s, a.obj, a.obj_cols, a.psi,
-                     a.probe, a.roi, a.row_ptr, a.row_frames, a.factors, a.phase_constraint, a.obj_partial);
+  hipLaunchKernelGGL((k_dm_object<M>), dim3(a.obj_rows, dm_tile_cols(a.obj_cols, M)), dim3(PTYK_NT), 0, s, a.obj,
+                     a.obj_cols, a.psi, a.probe, a.roi, a.tile_ptr, a.tile_frames, a.factors,
+                     a.phase_constraint, a.obj_partial);
   rec(DM_T_PROBE_APPLY);
   hipLaunchKernelGGL((k_dm_probe_apply<M>), dim3(gp), dim3(PTYK_NT), 0, s, a.probe, a.probe_partial,
                      a.probe_chunks, a.factors, a.update_probe, a.probe_partial_sum);
   rec(DM_T_FINISH);
-  hipLaunchKernelGGL((k_dm_finish<PTYK_NT>), dim3(1), dim3(PTYK_NT), 0, s, a.obj_partial, a.obj_rows * cch,
+  hipLaunchKernelGGL((k_dm_finish<PTYK_NT>), dim3(1), dim3(PTYK_NT), 0, s, a.obj_partial, a.obj_rows * dm_tile_cols(a.obj_cols, M),
                      a.probe_partial_sum, (int)gp, a.scal, a.factors);
   rec(-1);
   return hipGetLastError();

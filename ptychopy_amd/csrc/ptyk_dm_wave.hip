@@ -15,6 +15,7 @@
 #include <hip/hip_ext.h>
 
 #include "ptyk_device.h"
+#include "ptyk_dm_gather.h"
 #include "ptyk_internal.h"
 
 namespace ptyk {
@@ -332,61 +333,31 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_pass_c(float2* __restrict__ psi
   }
 }
 
-#define PTYK_OBJ_CHUNK 256
-
-// dO[p][c] += sum over this wave's frames covering object row p (ascending frame id) of the
-// (optionally phase-clamped) increments s_O conj(P) psi_new.
+// dO += this wave's increments (obj_row_sum) on the object rows from row0.
 template <int M>
-__global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_accum(double2* __restrict__ d_obj, int obj_cols, int row_lo,
+__global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_accum(double2* __restrict__ d_obj, int row0, int obj_cols,
                                                            const float2* __restrict__ psi,
                                                            const float2* __restrict__ probe,
                                                            const int2* __restrict__ roi,
-                                                           const int* __restrict__ row_ptr,
-                                                           const int* __restrict__ row_frames,
+                                                           const int* __restrict__ tile_ptr,
+                                                           const int* __restrict__ tile_frames,
                                                            const float* __restrict__ factors, int phase_constraint) {
-  const int p = row_lo + blockIdx.x;
-  const int c = blockIdx.y * PTYK_OBJ_CHUNK + threadIdx.x;
-  const float so = factors[1];
-  double ax = 0.0, ay = 0.0;
-  const int k0 = row_ptr[p], k1 = row_ptr[p + 1];
-  // frames in ascending order, four at a time: all loads of a step are issued before the
-  // (in-order) accumulation, so the sum is the same as one frame at a time
-  constexpr int U = 4;
-  for (int kb = k0; kb < k1; kb += U) {
-    float2 pv[U], sv[U];
-    bool act[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      act[u] = false;
-      if (kb + u < k1) {
-        const int j = row_frames[kb + u];
-        const int2 r = roi[j];
-        const int q = p - r.x, cc = c - r.y;
-        act[u] = c < obj_cols && cc >= 0 && cc < M;
-        if (act[u]) {
-          pv[u] = probe[q * M + cc];
-          sv[u] = psi[((long)j * M + q) * M + cc];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (!act[u]) continue;
-      float2 t = cscale(cmulcj(pv[u], sv[u]), so);
-      if (phase_constraint) t = clamp_phase(t);
-      ax += t.x;
-      ay += t.y;
-    }
-  }
-  if (c < obj_cols && k1 > k0) {
+  constexpr int TC = dm_tile_width(M);
+  const int p = row0 + blockIdx.x, c = blockIdx.y * TC + threadIdx.x % TC;
+  const int t = p / PTYK_DM_TR * gridDim.y + blockIdx.y;
+  const int k0 = tile_ptr[t], k1 = tile_ptr[t + 1];
+  const double2 a = obj_row_sum<M>(p, c, psi, probe, roi, tile_frames, k0, k1, factors[1], phase_constraint);
+  if (threadIdx.x < TC && c < obj_cols && k1 > k0) {
     double2 d = d_obj[(long)p * obj_cols + c];
-    d.x += ax;
-    d.y += ay;
+    d.x += a.x;
+    d.y += a.y;
     d_obj[(long)p * obj_cols + c] = d;
   }
 }
 
-// dP[q][c] += sum over frames [f0, f1) of conj(O[r_j + (q, c)]) psi_new_j[q][c].
+// dP[chunk][q][c] += sum over the chunk's share of frames [f0, f1) of conj(O[r_j + (q, c)])
+// psi_new_j[q][c].  The frames are shared out so that 512 workgroups run: 128^2 has 64 blocks of pixels,
+// and one share each took 52 us for 400 frames, eight 12 us.
 template <int M>
 __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_accum(double2* __restrict__ d_probe,
                                                              const float2* __restrict__ psi,
@@ -396,11 +367,12 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_accum(double2* __restrict
   constexpr int RPW = M >= PTYK_NT ? 1 : PTYK_NT / M;
   const int q = blockIdx.x * RPW + (RPW > 1 ? threadIdx.x / M : 0);
   const int c0 = RPW > 1 ? threadIdx.x % M : threadIdx.x;
+  const long j0 = f0 + (f1 - f0) * blockIdx.y / gridDim.y, j1 = f0 + (f1 - f0) * (blockIdx.y + 1) / gridDim.y;
   double ax[CPT], ay[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) ax[k] = ay[k] = 0.0;
 #pragma unroll 4
-  for (long j = f0; j < f1; ++j) {
+  for (long j = j0; j < j1; ++j) {
     const int2 r = roi[j];
     const float2* prow = psi + (j * M + q) * M;
     const float2* orow = obj + (long)(r.x + q) * obj_cols + r.y;
@@ -412,13 +384,14 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_accum(double2* __restrict
       ay[k] += t.y;
     }
   }
+  double2* out = d_probe + (long)blockIdx.y * M * M;
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int c = c0 + k * PTYK_NT;
-    double2 d = d_probe[q * M + c];
+    double2 d = out[q * M + c];
     d.x += ax[k];
     d.y += ay[k];
-    d_probe[q * M + c] = d;
+    out[q * M + c] = d;
   }
 }
 
@@ -426,7 +399,7 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_accum(double2* __restrict
 __global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_apply(float2* __restrict__ obj, double2* __restrict__ d_obj,
                                                            int obj_cols, double* __restrict__ block_sums) {
   __shared__ double red[PTYK_NT / 64];
-  const int p = blockIdx.x, c = blockIdx.y * PTYK_OBJ_CHUNK + threadIdx.x;
+  const int p = blockIdx.x, c = blockIdx.y * PTYK_NT + threadIdx.x;
   double s2 = 0.0;
   if (c < obj_cols) {
     const long i = (long)p * obj_cols + c;
@@ -442,9 +415,9 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_apply(float2* __restrict__ 
   if (threadIdx.x == 0) block_sums[(long)blockIdx.x * gridDim.y + blockIdx.y] = s2;
 }
 
-// P += s_P dP when updating, dP <- 0, per-block sum |P|^2.
+// P += s_P dP (the chunks in order) when updating, dP <- 0, per-block sum |P|^2.
 __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_apply(float2* __restrict__ probe, double2* __restrict__ d_probe,
-                                                             long mm, const float* __restrict__ factors, int update,
+                                                             long mm, int chunks, const float* __restrict__ factors, int update,
                                                              double* __restrict__ block_sums) {
   __shared__ double red[PTYK_NT / 64];
   const long i = (long)blockIdx.x * PTYK_NT + threadIdx.x;
@@ -452,12 +425,17 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_apply(float2* __restrict_
   if (i < mm) {
     float2 p = probe[i];
     if (update) {
-      const double2 d = d_probe[i];
+      double2 d = make_double2(0.0, 0.0);
+      for (int k = 0; k < chunks; ++k) {
+        const double2 t = d_probe[k * mm + i];
+        d.x += t.x;
+        d.y += t.y;
+        d_probe[k * mm + i] = make_double2(0.0, 0.0);
+      }
       const double sp = (double)factors[0];
       p.x = (float)((double)p.x + sp * d.x);
       p.y = (float)((double)p.y + sp * d.y);
       probe[i] = p;
-      d_probe[i] = make_double2(0.0, 0.0);
     }
     s2 = (double)p.x * p.x + (double)p.y * p.y;
   }
@@ -468,7 +446,7 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_apply(float2* __restrict_
 template <int M>
 static hipError_t wave_impl(const DmWaveArgs& a, hipStream_t s, DmTimer* tm) {
   using C = WaveCfg<M>;
-  const int cch = (a.obj_cols + PTYK_OBJ_CHUNK - 1) / PTYK_OBJ_CHUNK;
+  const int tcols = dm_tile_cols(a.obj_cols, M), cch = (a.obj_cols + PTYK_NT - 1) / PTYK_NT;
   constexpr int RPW = M >= PTYK_NT ? 1 : PTYK_NT / M;
   for (int w = 0; w < a.n_waves; ++w) {
     const long f0 = (long)w * a.wave, f1 = f0 + a.wave < a.n_frames ? f0 + a.wave : a.n_frames;
@@ -484,20 +462,21 @@ static hipError_t wave_impl(const DmWaveArgs& a, hipStream_t s, DmTimer* tm) {
     hipLaunchKernelGGL((k_dmw_pass_c<M>), dim3(ga), dim3(PTYK_NT), 0, s, a.psi, f0, groups, a.tw);
     if (a.update_probe) {
       if (tm) tm->mark(s, DM_T_PROBE_GATHER);
-      hipLaunchKernelGGL((k_dmw_probe_accum<M>), dim3(M / RPW), dim3(PTYK_NT), 0, s, a.d_probe, a.psi, a.obj,
-                         a.obj_cols, a.roi, f0, f1);
+      hipLaunchKernelGGL((k_dmw_probe_accum<M>), dim3(M / RPW, dm_wave_probe_chunks(M)), dim3(PTYK_NT), 0, s, a.d_probe,
+                         a.psi, a.obj, a.obj_cols, a.roi, f0, f1);
     }
-    const int lo = a.wave_row_lo[w], hi = a.wave_row_hi[w];
+    const int lo = a.wave_tile_lo[w] * PTYK_DM_TR, hi = min(a.wave_tile_hi[w] * PTYK_DM_TR, a.obj_rows);
     if (hi > lo) {
       if (tm) tm->mark(s, DM_T_OBJ_GATHER);
-      hipLaunchKernelGGL((k_dmw_obj_accum<M>), dim3(hi - lo, cch), dim3(PTYK_NT), 0, s, a.d_obj, a.obj_cols, lo,
-                         a.psi, a.probe, a.roi, a.wave_row_ptr + (long)w * (a.obj_rows + 1), a.wave_row_frames,
-                         a.factors, a.phase_constraint);
+      hipLaunchKernelGGL((k_dmw_obj_accum<M>), dim3(hi - lo, tcols), dim3(PTYK_NT), 0, s, a.d_obj, lo, a.obj_cols, a.psi,
+                         a.probe, a.roi, a.wave_tile_ptr + (long)w * (dm_tiles(a.obj_rows, a.obj_cols, M) + 1),
+                         a.wave_tile_frames, a.factors, a.phase_constraint);
     }
   }
   if (tm) tm->mark(s, DM_T_PROBE_APPLY);
   const unsigned gpa = (unsigned)((M * M + PTYK_NT - 1) / PTYK_NT);
-  hipLaunchKernelGGL(k_dmw_probe_apply, dim3(gpa), dim3(PTYK_NT), 0, s, a.probe, a.d_probe, (long)M * M, a.factors,
+  hipLaunchKernelGGL(k_dmw_probe_apply, dim3(gpa), dim3(PTYK_NT), 0, s, a.probe, a.d_probe, (long)M * M,
+                     dm_wave_probe_chunks(M), a.factors,
                      a.update_probe, a.probe_partial_sum);
   if (tm) tm->mark(s, DM_T_OBJ_APPLY);
   hipLaunchKernelGGL(k_dmw_obj_apply, dim3(a.obj_rows, cch), dim3(PTYK_NT), 0, s, a.obj, a.d_obj, a.obj_cols,
@@ -1473,6 +1452,7 @@ hipError_t mls_shift_passes(float2* pu, const float2* chi, const float2* op, int
 }
 
 bool dm_wave_supported(int m) { return m == 128 || m == 256 || m == 512; }
+int dm_wave_probe_chunks(int m) { return m == 128 ? 8 : m == 256 ? 2 : 1; }
 int dm_wave_probe_blocks(int m) { return (m * m + PTYK_NT - 1) / PTYK_NT; }
 
 hipError_t dm_wave_iteration(const DmWaveArgs& a, hipStream_t s, DmTimer* tm) {

@@ -30,6 +30,13 @@ hipError_t fft2_pair(float2* dst, const float2* a, const float2* b, int m, const
 // The row half of fft2_pair alone (m in {128, 256, 512}): dst holds the row spectra of a and b.
 hipError_t fft_rows_pair(float2* dst, const float2* a, const float2* b, int m, const float2* tw, hipStream_t s);
 
+// Object tiles of the DM gathers: PTYK_DM_TR rows x dm_tile_width(m) columns.
+#define PTYK_DM_TR 8
+__host__ __device__ constexpr int dm_tile_width(int m) { return m >= 256 ? 128 : 64; }
+inline int dm_tile_rows(int obj_rows) { return (obj_rows + PTYK_DM_TR - 1) / PTYK_DM_TR; }
+inline int dm_tile_cols(int obj_cols, int m) { return (obj_cols + dm_tile_width(m) - 1) / dm_tile_width(m); }
+inline int dm_tiles(int obj_rows, int obj_cols, int m) { return dm_tile_rows(obj_rows) * dm_tile_cols(obj_cols, m); }
+
 // ---- DM (difference map) per-iteration launches; see ptyk_dm.hip for the equations.
 struct DmArgs {
   float2* psi;            // N x M x M exit-wave state
@@ -38,10 +45,10 @@ struct DmArgs {
   const __half* amp;      // N x M x M amplitudes (FP16)
   const float* amp_scale; // N per-frame scales
   const int2* roi;        // N rounded ROI origins (row, col)
-  const int* row_ptr;     // obj_rows + 1 : CSR of frames covering each object row
-  const int* row_frames;  // N*M frame ids, ascending per object row
+  const int* tile_ptr;    // dm_tiles + 1: CSR of the frames that touch each object tile
+  const int* tile_frames; // frame ids, ascending per tile
   double2* probe_partial; // probe_chunks x M x M
-  double* obj_partial;    // obj_rows * obj_col_chunks
+  double* obj_partial;    // obj_rows x dm_tile_cols
   double* probe_partial_sum;  // M (one per probe row block)
   float* factors;         // device: [0] = 1/objMax cached, [1] = 1/probeMax cached
   double* scal;           // device: [0] objSum, [1] probeSum
@@ -81,7 +88,6 @@ struct LaunchTimer {
 typedef LaunchTimer DmTimer;
 
 hipError_t dm_iteration(const DmArgs& a, hipStream_t s, DmTimer* tm /* nullable */);
-int dm_obj_col_chunks(int obj_cols);
 
 // Wave-scheduled DM (ptyk_dm_wave.hip), M in {128, 256, 512}.
 struct DmWaveArgs {
@@ -91,12 +97,12 @@ struct DmWaveArgs {
   const __half* amp;
   const float* amp_scale;
   const int2* roi;
-  const int* wave_row_ptr;    // device: n_waves x (obj_rows + 1) offsets into wave_row_frames
-  const int* wave_row_frames; // device: frame ids, ascending per (wave, object row)
-  const int* wave_row_lo;     // host: first object row touched by each wave
-  const int* wave_row_hi;     // host: one past the last
+  const int* wave_tile_ptr;    // device: n_waves x (dm_tiles + 1) offsets into wave_tile_frames
+  const int* wave_tile_frames; // device: frame ids, ascending per (wave, object tile)
+  const int* wave_tile_lo;     // host: first row of object tiles touched by each wave
+  const int* wave_tile_hi;     // host: one past the last
   double2* d_obj;             // FP64 object increment accumulator (canvas)
-  double2* d_probe;           // FP64 probe increment accumulator (M x M)
+  double2* d_probe;           // FP64 probe increment accumulators (dm_wave_probe_chunks x M x M)
   double* obj_partial;
   double* probe_partial_sum;
   float* factors;
@@ -107,6 +113,7 @@ struct DmWaveArgs {
   int phase_constraint, update_probe;
 };
 bool dm_wave_supported(int m);
+int dm_wave_probe_chunks(int m);
 int dm_wave_probe_blocks(int m);
 hipError_t dm_wave_iteration(const DmWaveArgs& a, hipStream_t s, DmTimer* tm /* nullable */);
 // MLs forward FFT + multi-mode modulus step + inverse FFT of K mode-major planes of G frames in

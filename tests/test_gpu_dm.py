@@ -188,3 +188,21 @@ def test_dm_timed_iteration_reports_every_pass(gpu):
         ms = e.dm_iteration_timed(_flags(12))
     assert ms.shape == (len(E.DM_KERNELS),)
     assert np.all(ms[[0, 1, 2, 3, 4]] > 0)
+
+
+@pytest.mark.parametrize("m,n_side,step,wave", [(64, 1, 3.0, -1), (64, 9, 2.3, -1), (128, 1, 3.0, 0), (128, 7, 5.1, 5),
+                                                (256, 4, 6.3, 3), (512, 2, 129.7, 0)])
+def test_gathers_over_short_and_long_frame_lists(gpu, orc, m, n_side, step, wave):
+    """Fewer frames than shares of them, lists that end inside a step, tiles with no frame, and canvases
+    that end inside a tile."""
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=m, n_side=n_side, step=step, seed=m + n_side, jitter=0.6)
+    with _engine_for(p) as e:
+        e.set_object((0.9 * p["obj"]).astype(np.complex64))
+        e.set_probe(p["probe"])
+        e.refresh_maxima()
+        e.set_tuning(E.TUNE_DM_WAVE, wave)
+        amp = e.get_frames().astype(np.float64)
+        psi = np.zeros((p["n"], m, m))
+        for i in range(2):
+            psi, _ = _check_step(e, orc, p, amp, E.FLAG_UPDATE_PROBE, psi, first_call=(i == 0))
