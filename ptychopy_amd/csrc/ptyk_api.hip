@@ -301,8 +301,7 @@ int ptyk_get_frames_f32(ptyk_ctx* c, float* out) {
   float* tmp = nullptr;
   HIPCHK(c, hipMalloc((void**)&tmp, total * sizeof(float)));
   hipError_t e = dequantize_frames(c->amp, c->amp_scale, tmp, n, c->cfg.frame_size, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, total * sizeof(float), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = copy_to_host(out, tmp, total * sizeof(float), c->cfg.device, c->stream);
   hipFree(tmp);
   HIPCHK(c, e);
   return PTYK_OK;
@@ -1533,7 +1532,7 @@ int ptyk_preprocess_frames(ptyk_ctx* c, const float* raw, int64_t count, const p
   if (e == hipSuccess) e = hipMalloc((void**)&d_out, nout * sizeof(float));
   if (e == hipSuccess) e = hipMemcpyAsync(d_raw, raw, nraw * sizeof(float), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = ingest_frames(d_raw, d_out, count, a, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, nout * sizeof(float), hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = copy_to_host(out, d_out, nout * sizeof(float), c->cfg.device, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (d_raw) hipFree(d_raw);
   if (d_out) hipFree(d_out);
@@ -1572,25 +1571,25 @@ int ptyk_simulate(ptyk_ctx* c, const float* obj, int32_t rows, int32_t cols, con
   for (int64_t i = 0; i < n; ++i)
     if (!std::isfinite(pos[2 * i]) || !std::isfinite(pos[2 * i + 1]))
       return fail(c, PTYK_EINVAL, "non-finite position");
-  const size_t canvas = (size_t)rows * cols;
-  float2 *d_obj = nullptr, *d_probe = nullptr, *d_pos = nullptr, *d_psi = nullptr;
-  float* d_out = nullptr;
-  hipError_t e = hipMalloc((void**)&d_obj, canvas * sizeof(float2));
-  if (e == hipSuccess) e = hipMalloc((void**)&d_probe, c->mm * sizeof(float2));
-  if (e == hipSuccess) e = hipMalloc((void**)&d_pos, (n ? n : 1) * sizeof(float2));
-  if (e == hipSuccess) e = hipMalloc((void**)&d_psi, (n ? n : 1) * c->mm * sizeof(float2));
-  if (e == hipSuccess) e = hipMalloc((void**)&d_out, (n ? n : 1) * c->mm * sizeof(float));
-  if (e == hipSuccess) e = hipMemcpyAsync(d_obj, obj, canvas * sizeof(float2), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_probe, probe, c->mm * sizeof(float2), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess && n) e = hipMemcpyAsync(d_pos, pos, n * sizeof(float2), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess && n)
-    e = simulate_exit_waves(d_obj, rows, cols, d_probe, d_pos, d_psi, n, m, c->cfg.tex_quantize, c->stream);
-  if (e == hipSuccess && n) e = fft2_batch(d_psi, n, m, false, c->tw, c->stream);
-  if (e == hipSuccess && n) e = abs_frames(d_psi, d_out, n * c->mm, squared, c->stream);
-  if (e == hipSuccess && n) e = hipMemcpyAsync(out, d_out, n * c->mm * sizeof(float), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  for (void* p : {(void*)d_obj, (void*)d_probe, (void*)d_pos, (void*)d_psi, (void*)d_out})
-    if (p) hipFree(p);
+  const size_t canvas = (size_t)rows * cols, px = (size_t)n * c->mm;
+  // one allocation: probe, exit waves, amplitudes (whole frames), object, positions
+  float2* work = nullptr;
+  hipError_t e = hipMalloc((void**)&work, (c->mm + px + px / 2 + canvas + n) * sizeof(float2));
+  if (e == hipSuccess) {
+    float2 *d_probe = work, *d_psi = d_probe + c->mm, *d_canvas = d_psi + px + px / 2, *d_pos = d_canvas + canvas;
+    float* d_out = reinterpret_cast<float*>(d_psi + px);
+    e = hipMemcpyAsync(d_canvas, obj, canvas * sizeof(float2), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(d_probe, probe, c->mm * sizeof(float2), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess && n) e = hipMemcpyAsync(d_pos, pos, n * sizeof(float2), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess && n)
+      e = simulate_exit_waves(d_canvas, rows, cols, d_probe, d_pos, d_psi, n, m, c->cfg.tex_quantize, c->stream);
+    if (e == hipSuccess && n) e = fft2_batch(d_psi, n, m, false, c->tw, c->stream);
+    if (e == hipSuccess && n) e = abs_frames(d_psi, d_out, n * c->mm, squared, c->stream);
+    if (e == hipSuccess && n) e = copy_to_host(out, d_out, px * sizeof(float), c->cfg.device, c->stream);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = es;
+    hipFree(work);
+  }
   HIPCHK(c, e);
   return PTYK_OK;
 }

@@ -375,4 +375,9 @@ hipError_t abs_frames(const float2* psi, float* out, long count, int squared, hi
 hipError_t modes_from_base(float2* probe, float* probe_int, int k_total, int m, float factor, hipStream_t s);
 hipError_t orthogonalize_modes(float2* probe, float2* tmp, int k_total, int m, hipStream_t s);
 
+// Device to pageable host memory after what stream s holds so far; returns when dst is filled
+// (ptyk_hostcopy.hip).  With `ready`, byte b is copied after event ready[b / per_event] as well.
+hipError_t copy_to_host(void* dst, const void* src, size_t bytes, int device, hipStream_t s,
+                        const hipEvent_t* ready = nullptr, size_t per_event = 0);
+
 }  // namespace ptyk
