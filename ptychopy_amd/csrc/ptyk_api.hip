@@ -44,7 +44,8 @@ struct ptyk_ctx {
   // ePIE scratch
   float2* e_psi_old = nullptr;
   float2* e_psi = nullptr;
-  unsigned long long* e_flags = nullptr;  // team form: barrier flags (they stand at e_epoch)
+  // team form, in scal's allocation: barrier flags (they stand at e_epoch), row maxima, error parts
+  unsigned long long* e_flags = nullptr;
   float* e_rowmax = nullptr;
   double* e_err = nullptr;
   unsigned e_epoch = 1;
@@ -161,7 +162,7 @@ static void free_all(ptyk_ctx* c) {
     if (p) hipFree(p);
   void* ptrs[] = {c->tw, c->obj, c->obj_int, c->probe, c->probe_int, c->probe_tmp, c->amp, c->amp_scale,
                   c->amp_sum, c->avg, c->pos_dev, c->roi_dev, c->order_dev, c->scal, c->factors, c->e_psi_old,
-                  c->e_psi, c->e_flags, c->e_rowmax, c->e_err, c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial,
+                  c->e_psi, c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial,
                   c->probe_partial_sum, c->d_obj, c->d_probe, c->wave_tile_ptr, c->wave_tile_frames};
   for (void* p : ptrs)
     if (p) hipFree(p);
@@ -222,17 +223,23 @@ int ptyk_create(const ptyk_config* cfg, ptyk_ctx** out) {
   if ((e = dalloc(&c->pos_dev, n)) != hipSuccess) return bail(e, "positions");
   if ((e = dalloc(&c->roi_dev, n)) != hipSuccess) return bail(e, "roi");
   if ((e = dalloc(&c->order_dev, n)) != hipSuccess) return bail(e, "order");
-  if ((e = dalloc(&c->scal, PTYK_SCAL_COUNT + 1)) != hipSuccess) return bail(e, "scalars");
+  if ((e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, cfg->device)) != hipSuccess)
+    return bail(e, "device attribute");
+  {
+    // the scalars (and the team form's slot) with the team form's state behind them: one allocation
+    const size_t ns = (PTYK_SCAL_COUNT + 1 + 15) / 16 * 16, nf = PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE;
+    const bool team = epie_team_size((int)m, c->cus) > 0;
+    if ((e = dalloc(&c->scal, ns + (team ? nf + PTYK_EPIE_TEAM_MAX + ((size_t)cfg->obj_rows + 1) / 2 : 0))) != hipSuccess)
+      return bail(e, "scalars");
+    if (team) {
+      c->e_flags = reinterpret_cast<unsigned long long*>(c->scal + ns);
+      c->e_err = c->scal + ns + nf;
+      c->e_rowmax = reinterpret_cast<float*>(c->e_err + PTYK_EPIE_TEAM_MAX);
+    }
+  }
   if ((e = dalloc(&c->factors, 2)) != hipSuccess) return bail(e, "factors");
   if ((e = dalloc(&c->e_psi_old, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
   if ((e = dalloc(&c->e_psi, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
-  if ((e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, cfg->device)) != hipSuccess)
-    return bail(e, "device attribute");
-  if (epie_team_size((int)m, c->cus) > 0) {
-    if ((e = dalloc(&c->e_flags, PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE)) != hipSuccess) return bail(e, "epie flags");
-    if ((e = dalloc(&c->e_rowmax, cfg->obj_rows)) != hipSuccess) return bail(e, "epie row maxima");
-    if ((e = dalloc(&c->e_err, PTYK_EPIE_TEAM_MAX)) != hipSuccess) return bail(e, "epie errors");
-  }
   for (auto& ev : c->ev)
     if ((e = hipEventCreate(&ev)) != hipSuccess) return bail(e, "events");
   // Probe::m_maxIntensity starts at 1 (Probe.cpp:54-58); objMax at 0.
