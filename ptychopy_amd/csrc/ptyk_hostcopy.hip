@@ -14,7 +14,8 @@ namespace ptyk {
 // 0.93).  Here a few threads move pieces through pinned buffers, two each, so that the pages, the copies
 // and the transfers overlap.  Pieces are huge pages of dst: two threads that meet in one would both clear
 // it.  52 MB with its simulation: 6.0 -> 2.2 ms; 8 threads instead of 4 the same, pieces of 1 MiB 2.5 and
-// of 512 KiB 3.3 ms.  8 MB: 0.95 -> 0.6 ms.  Below HC_MIN the threads and buffers cost what they save.
+// of 512 KiB 3.3 ms.  4 MB with theirs: 0.51 -> 0.43 ms.  Below HC_MIN the threads and buffers cost what
+// they save.
 static constexpr size_t HC_PIECE = 2 << 20;
 static constexpr int HC_THREADS = 4;
 static constexpr size_t HC_MIN = 4 << 20;
