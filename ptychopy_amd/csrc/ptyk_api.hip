@@ -43,7 +43,7 @@ struct ptyk_ctx {
   float* factors = nullptr;
   // ePIE scratch
   float2* e_psi_old = nullptr;
-  float2* e_psi = nullptr;
+  float2* e_psi = nullptr;  // in e_psi_old's allocation
   // team form, in scal's allocation: barrier flags (they stand at e_epoch), row maxima, error parts
   unsigned long long* e_flags = nullptr;
   float* e_rowmax = nullptr;
@@ -162,7 +162,7 @@ static void free_all(ptyk_ctx* c) {
     if (p) hipFree(p);
   void* ptrs[] = {c->tw, c->obj, c->obj_int, c->probe, c->probe_int, c->probe_tmp, c->amp, c->amp_scale,
                   c->amp_sum, c->avg, c->pos_dev, c->roi_dev, c->order_dev, c->scal, c->factors, c->e_psi_old,
-                  c->e_psi, c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial,
+                  c->psi, c->tile_ptr, c->tile_frames, c->probe_partial, c->obj_partial,
                   c->probe_partial_sum, c->d_obj, c->d_probe, c->wave_tile_ptr, c->wave_tile_frames};
   for (void* p : ptrs)
     if (p) hipFree(p);
@@ -238,8 +238,8 @@ int ptyk_create(const ptyk_config* cfg, ptyk_ctx** out) {
     }
   }
   if ((e = dalloc(&c->factors, 2)) != hipSuccess) return bail(e, "factors");
-  if ((e = dalloc(&c->e_psi_old, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
-  if ((e = dalloc(&c->e_psi, k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
+  if ((e = dalloc(&c->e_psi_old, 2 * k * c->mm)) != hipSuccess) return bail(e, "epie scratch");
+  c->e_psi = c->e_psi_old + k * c->mm;
   for (auto& ev : c->ev)
     if ((e = hipEventCreate(&ev)) != hipSuccess) return bail(e, "events");
   // Probe::m_maxIntensity starts at 1 (Probe.cpp:54-58); objMax at 0.
