@@ -17,6 +17,7 @@
 #include "../../include/ptyk.h"
 #include "ptyk_device.h"
 #include "ptyk_internal.h"
+#include "ptyk_team.h"
 
 using namespace ptyk;
 
@@ -670,7 +671,7 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
     c->e_epoch += epie_team_barriers(n);
     if (!done) {  // the flags stand anywhere: bring them to where the next iteration starts
       const std::vector<unsigned long long> at(PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE,
-                                               (unsigned long long)c->e_epoch << 32);
+                                               team_flag(c->e_epoch, 0));
       HIPCHK(c, hipMemcpy(c->e_flags, at.data(), at.size() * sizeof(at[0]), hipMemcpyHostToDevice));
       return fail(c, PTYK_EDEVICE, "ePIE: the workgroups of a team were not on the device together; the iteration is incomplete");
     }

@@ -13,6 +13,7 @@
 #include "../../include/ptyk.h"
 #include "ptyk_device.h"
 #include "ptyk_internal.h"
+#include "ptyk_team.h"
 
 #include <algorithm>
 
@@ -298,14 +299,15 @@ __device__ __forceinline__ void st_dev(float* p, float v) {
 // arrive: this workgroup's stores have reached the coherence point (a store leaves vmcnt when it is
 // acknowledged there), then its flag: the epoch and a value of the workgroup (read by thread 0 from
 // LDS, in *value; a non-negative float).  wait: one wave polls all W flags, one per lane, and leaves
-// the largest of the values in *most.  The wait is bounded (limit ticks of the 100 MHz clock): the
+// the largest of the values in *most.  Why a slow reader cannot meet a later barrier's value: see
+// team_word (ptyk_team.h).  The wait is bounded (limit ticks of the 100 MHz clock): the
 // host admits no more workgroups than the device can hold at once, so it ends unless the device is
 // lost to something else; then every workgroup gives up and the host reports it.
 __device__ __forceinline__ void team_arrive(unsigned long long* flags, int w, unsigned epoch, const unsigned* value) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
-    __hip_atomic_store(flags + w * PTYK_EPIE_FLAG_STRIDE, ((unsigned long long)epoch << 32) | *value, __ATOMIC_RELAXED,
+    __hip_atomic_store(flags + team_word(w, epoch), team_flag(epoch, *value), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ float wave_max_pos(float v);
@@ -316,24 +318,24 @@ __device__ __forceinline__ bool team_wait(const unsigned long long* flags, unsig
     const int l = threadIdx.x;
     bool ok = false;
     long long t0 = 0;
-    unsigned long long v = 0;
+    unsigned v = 0;
     for (int i = 0;; ++i) {
       bool here = true;
       v = 0;
 #pragma unroll
       for (int q = 0; q < (W + 63) / 64; ++q)
         if (W >= 64 || l < W) {
-          const unsigned long long f = __hip_atomic_load(flags + (l + q * 64) * PTYK_EPIE_FLAG_STRIDE, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT);
-          here = here && (int)((unsigned)(f >> 32) - epoch) >= 0;
-          v = max(v, f & 0xffffffffull);  // values are non-negative floats: ordered as integers
+          const unsigned long long f =
+              __hip_atomic_load(flags + team_word(l + q * 64, epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          here = here && team_here(f, epoch);
+          v = max(v, team_value(f));  // values are non-negative floats: ordered as integers
         }
       ok = __all(here);
       if (ok) break;
       if (i == 1024) t0 = wall_clock64();
       if (i > 1024 && (i & 255) == 0 && wall_clock64() - t0 > limit) break;
     }
-    const float m = wave_max_pos(__uint_as_float((unsigned)v));
+    const float m = wave_max_pos(__uint_as_float(v));
     if (l == 0) {
       *most = m;
       if (!ok) *gone = 1;

@@ -215,8 +215,6 @@ struct EpieArgs {
   unsigned long long* team_flags; float* team_rowmax; double* team_err;
   unsigned team_epoch; int team_size, k_res; long long team_limit;
 };
-#define PTYK_EPIE_TEAM_MAX 128                     // workgroups of the largest team
-#define PTYK_EPIE_FLAG_STRIDE 16                   // flags (epoch, value) of one team: one 128-byte line each
 #define PTYK_EPIE_DONE PTYK_SCAL_COUNT             // scal slot the team form sets to team_epoch when the iteration ran
 int epie_team_size(int m, int cus);                // workgroups that share a frame; 0: one workgroup
 unsigned epie_team_barriers(int n_pos);

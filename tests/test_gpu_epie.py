@@ -190,3 +190,53 @@ def test_teams_of_several_threads_give_their_own_results(gpu):
     for i in range(6):
         for a, b in zip(alone[i], together[i]):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def _wide_problem(cols, n, seed, m=64, rows=100, modes=1):
+    """Frames scattered over a canvas many times as wide as they are, some of them overlapping and two at
+    its left and right ends."""
+    import oracle
+    from ptychopy_amd import sim
+    rng = np.random.default_rng(seed)
+    pos = np.stack([rng.uniform(0, rows - m, n), rng.uniform(0, cols - m, n)], axis=1).astype(np.float32)
+    pos[:2, 1] = 0, cols - m
+    pos[2:n // 2, 1] = (pos[0, 1] + rng.uniform(0, 1.5 * m, n // 2 - 2)).astype(np.float32)
+    obj = sim.random_field_object((rows, cols), rng, phase_std=0.5)
+    probe = sim.gaussian_probe(m, fwhm=m / 3, defocus_edge=2.0)
+    amp = sim.poisson_amplitudes(oracle.simulate(obj, probe, pos, squared=True), 100.0 * m * m, rng)
+    return dict(pos=pos, obj=obj, probe=probe, amp=amp, shape=(rows, cols), m=m, n=n, k=modes)
+
+
+@pytest.mark.parametrize("m,cols,modes", [(64, 2200, 1), (64, 4173, 2), (128, 2500, 1)])
+def test_teams_on_wide_canvases_match_oracle(gpu, orc, m, cols, modes):
+    """A long row of |O|^2 beside the frame: the maximum of the whole canvas enters every probe update,
+    whatever a workgroup is at when the others announce theirs."""
+    from ptychopy_amd import _engine as E
+    p = _wide_problem(cols, 12, cols, m=m, rows=m + 36, modes=modes)
+    rng = np.random.default_rng(cols)
+    flags = E.FLAG_UPDATE_PROBE | (E.FLAG_UPDATE_MODES if modes > 1 else 0)
+    with _near_engine(p, _flat_counts(p)) as e:
+        amp = e.get_frames().astype(np.float64)
+        for f in (flags | E.FLAG_RMS, flags & ~E.FLAG_UPDATE_PROBE, flags):
+            _check(e, orc, p, amp, rng.permutation(p["n"]), f, k_use=modes, modal=modes > 1)
+
+
+def test_teams_on_wide_canvases_repeat_bitwise(gpu):
+    """The same iterations from the same state give the same bits, run after run."""
+    from ptychopy_amd import _engine as E
+    p = _wide_problem(2200, 24, 11)
+    orders = [np.random.default_rng(i).permutation(p["n"]) for i in range(4)]
+    first = None
+    with _near_engine(p) as e:
+        state = e.get_object(), e.get_probe(), e.get_scalars()
+        for _ in range(25):
+            e.set_object(state[0])
+            e.set_probe(state[1])
+            e.refresh_maxima()
+            e.set_scalars(state[2])
+            for o in orders:
+                e.epie_iteration(o, E.FLAG_UPDATE_PROBE)
+            out = [a.view(np.uint32) for a in (e.get_object(), e.get_probe())] + [e.get_scalars().view(np.uint64)]
+            first = first or out
+            for a, b in zip(first, out):
+                assert np.array_equal(a, b)
