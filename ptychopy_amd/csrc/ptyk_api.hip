@@ -45,9 +45,10 @@ struct ptyk_ctx {
   // ePIE scratch
   float2* e_psi_old = nullptr;
   float2* e_psi = nullptr;  // in e_psi_old's allocation
-  // team form, in scal's allocation: barrier flags (they stand at e_epoch), row maxima, error parts
+  // team form, in scal's allocation: barrier flags (they stand at e_epoch), segment and row maxima, error
+  // parts
   unsigned long long* e_flags = nullptr;
-  float* e_rowmax = nullptr;
+  float *e_segmax = nullptr, *e_rowmax = nullptr;
   double* e_err = nullptr;
   unsigned e_epoch = 1;
   int cus = 0;  // compute units of the device
@@ -230,12 +231,14 @@ int ptyk_create(const ptyk_config* cfg, ptyk_ctx** out) {
     // the scalars (and the team form's slot) with the team form's state behind them: one allocation
     const size_t ns = (PTYK_SCAL_COUNT + 1 + 15) / 16 * 16, nf = PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE;
     const bool team = epie_team_size((int)m, c->cus) > 0;
-    if ((e = dalloc(&c->scal, ns + (team ? nf + PTYK_EPIE_TEAM_MAX + ((size_t)cfg->obj_rows + 1) / 2 : 0))) != hipSuccess)
+    const size_t nm = (size_t)cfg->obj_rows * (1 + epie_segments(cfg->obj_cols));  // floats
+    if ((e = dalloc(&c->scal, ns + (team ? nf + PTYK_EPIE_TEAM_MAX + (nm + 1) / 2 : 0))) != hipSuccess)
       return bail(e, "scalars");
     if (team) {
       c->e_flags = reinterpret_cast<unsigned long long*>(c->scal + ns);
       c->e_err = c->scal + ns + nf;
       c->e_rowmax = reinterpret_cast<float*>(c->e_err + PTYK_EPIE_TEAM_MAX);
+      c->e_segmax = c->e_rowmax + cfg->obj_rows;
     }
   }
   if ((e = dalloc(&c->factors, 2)) != hipSuccess) return bail(e, "factors");
@@ -653,6 +656,7 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
   const int team = epie_team_size(a.m, c->cus);
   a.team_size = team;
   a.team_flags = c->e_flags;
+  a.team_segmax = c->e_segmax;
   a.team_rowmax = c->e_rowmax;
   a.team_err = c->e_err;
   a.team_epoch = c->e_epoch;

@@ -209,13 +209,15 @@ struct EpieArgs {
   const float2* tw;
   int n_pos, m, k_use, k_total, obj_rows, obj_cols;
   int phase_constraint, update_probe, modal, rms, tex_quantize;
-  // team form (team_size = epie_team_size(m, CUs) > 0): barrier flags, row maxima of |O|^2 and the
-  // workgroups' errors; the flags stand at team_epoch and move by epie_team_barriers(n_pos);
+  // team form (team_size = epie_team_size(m, CUs) > 0): barrier flags, maxima of |O|^2 over segments of
+  // canvas rows (rows x epie_segments) and over rows, and the workgroups' errors; the flags stand at team_epoch and move by epie_team_barriers(n_pos);
   // team_limit bounds a barrier's wait (ticks of the 100 MHz clock); k_res is set by the launch
-  unsigned long long* team_flags; float* team_rowmax; double* team_err;
+  unsigned long long* team_flags; float *team_segmax, *team_rowmax; double* team_err;
   unsigned team_epoch; int team_size, k_res; long long team_limit;
 };
 #define PTYK_EPIE_DONE PTYK_SCAL_COUNT             // scal slot the team form sets to team_epoch when the iteration ran
+#define PTYK_EPIE_SEG 64                           // canvas columns of a segment
+__host__ __device__ constexpr int epie_segments(int obj_cols) { return (obj_cols + PTYK_EPIE_SEG - 1) / PTYK_EPIE_SEG; }
 int epie_team_size(int m, int cus);                // workgroups that share a frame; 0: one workgroup
 unsigned epie_team_barriers(int n_pos);
 hipError_t epie_iteration(const EpieArgs& a, hipStream_t s);

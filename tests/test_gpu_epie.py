@@ -240,3 +240,41 @@ def test_teams_on_wide_canvases_repeat_bitwise(gpu):
             first = first or out
             for a, b in zip(first, out):
                 assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("m,rows,cols,at", [
+    (64, 64, 64, (0, 0)),        # nothing beside the frame
+    (64, 70, 128, (3, 64)),      # whole segments on both sides
+    (64, 66, 129, (1, 1)),       # one pixel on each side, a last segment of one column
+    (64, 200, 200, (70, 63)),
+    (64, 1100, 333, (1000, 65)),
+    (64, 71, 9000, (2, 4500)),   # more segments than a thread reads at once
+    (128, 130, 383, (2, 127)),
+    (256, 257, 700, (0, 300)),
+    (512, 513, 1100, (1, 500)),
+])
+def test_canvas_maximum_wherever_it_lies(gpu, orc, m, rows, cols, at):
+    """The probe step divides by max |O|^2 of the canvas: one bright pixel at the edges of the frame, of
+    its segments and of the canvas has to be seen (it makes the step 4 times shorter)."""
+    import oracle
+    from ptychopy_amd import _engine as E
+    from ptychopy_amd import sim
+    rng = np.random.default_rng(cols)
+    pos = np.array([at, (rows - m, cols - m)], np.float32)
+    obj = sim.random_field_object((rows, cols), rng, phase_std=0.5)
+    probe = sim.gaussian_probe(m, fwhm=m / 3, defocus_edge=2.0)
+    amp = sim.poisson_amplitudes(oracle.simulate(obj, probe, pos, squared=True), 100.0 * m * m, rng)
+    p = dict(pos=pos, obj=obj, probe=probe, amp=amp, shape=(rows, cols), m=m, n=2, k=1)
+    r, c = at
+    lo, hi = c // 64 * 64, (c + m + 63) // 64 * 64
+    spots = {(y, x) for y in (r, r + m - 1) for x in (0, lo - 1, lo, c - 1, c + m, hi - 1, hi, cols - 1)}
+    spots |= {(y, x) for y in (0, r - 1, r + m, rows - 1) for x in (c, cols - 1)}
+    with _near_engine(p, _flat_counts(p)) as e:
+        a64 = e.get_frames().astype(np.float64)
+        for y, x in sorted(s for s in spots if 0 <= s[0] < rows and 0 <= s[1] < cols):
+            o = (0.95 * obj).astype(np.complex64)
+            o[y, x] *= 2.0 * np.abs(o).max() / abs(o[y, x])
+            e.set_object(o)
+            e.set_probe(probe * np.exp(0.3j * rng.standard_normal(probe.shape)))
+            e.refresh_maxima()
+            _check(e, orc, p, a64, [0, 1], E.FLAG_UPDATE_PROBE)
