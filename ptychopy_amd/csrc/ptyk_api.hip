@@ -5,7 +5,6 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <condition_variable>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -18,6 +17,7 @@
 #include "ptyk_device.h"
 #include "ptyk_internal.h"
 #include "ptyk_team.h"
+#include "ptyk_team_slots.h"
 
 using namespace ptyk;
 
@@ -573,44 +573,12 @@ int ptyk_end_modal(ptyk_ctx* c) {
 }
 
 // ---------------------------------------------------------------- ePIE
-// The workgroups of an ePIE team wait for one another, so all of them have to be on the device at
-// once.  Iterations of several handles (from several threads) take their workgroups out of one
-// budget per device, one per CU whatever else fits there, and wait for their turn when it is spent.
-struct TeamBudget {
-  std::mutex mu;
-  std::condition_variable cv;
-  int left = -1;  // workgroups; set by the first use
-};
-class TeamSlots {
- public:
-  TeamSlots(int device, int cus, int want) : b_(want > 0 ? budget(device) : nullptr), want_(want) {
-    if (!b_) return;
-    std::unique_lock<std::mutex> l(b_->mu);
-    if (b_->left < 0) b_->left = cus;
-    b_->cv.wait(l, [&] { return b_->left >= want_; });
-    b_->left -= want_;
-  }
-  ~TeamSlots() {
-    if (!b_) return;
-    {
-      std::lock_guard<std::mutex> l(b_->mu);
-      b_->left += want_;
-    }
-    b_->cv.notify_all();
-  }
-  TeamSlots(const TeamSlots&) = delete;
-  TeamSlots& operator=(const TeamSlots&) = delete;
-
- private:
-  static TeamBudget* budget(int device) {
-    static std::mutex mu;
-    static std::map<int, TeamBudget> all;  // by device ordinal; elements stay where they are
-    std::lock_guard<std::mutex> l(mu);
-    return &all[device];
-  }
-  TeamBudget* b_;
-  int want_;
-};
+static TeamBudget* team_budget(int device) {
+  static std::mutex mu;
+  static std::map<int, TeamBudget> all;  // by device ordinal; elements stay where they are
+  std::lock_guard<std::mutex> l(mu);
+  return &all[device];
+}
 
 int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, double* err) {
   if (!c || !order) return fail(c, PTYK_EINVAL, "null argument");
@@ -663,7 +631,7 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
   a.team_limit = 1000000000LL;  // 10 s
   double s[PTYK_SCAL_COUNT + 1];
   {
-    TeamSlots slots(c->cfg.device, c->cus, team);
+    TeamSlots slots(team_budget(c->cfg.device), c->cus, team);  // one workgroup per CU, whatever else fits there
     hipError_t e = epie_iteration(a, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->stream);
     const hipError_t es = hipStreamSynchronize(c->stream);  // before the team's place is given back

@@ -28,3 +28,12 @@ def test_one_word_a_workgroup_would_not(tmp_path):
     """The check finds the fault of a single word: a late reader gets the next barrier's value."""
     r = _run(tmp_path, "-DONE_WORD")
     assert r.returncode == 1 and "gives" in r.stdout, r.stdout
+
+
+def test_teams_get_their_place_in_the_order_they_come(tmp_path):
+    """A large team is not overtaken for ever by small ones that fit beside what others hold."""
+    exe = tmp_path / "team_slots"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-pthread", f"-I{ROOT / 'ptychopy_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "seam" / "team_slots.cpp"), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
