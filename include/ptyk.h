@@ -121,7 +121,8 @@ int ptyk_orthogonalize_modes(ptyk_ctx* ctx);
 
 /* One ePIE iteration over all positions in the given order (ePIE::iteration,
  * ePIE.cpp:65-129).  order: N frame indices (a permutation).  err (nullable)
- * receives the averaged Fourier error when PTYK_FLAG_RMS is set, else 0. */
+ * receives the averaged Fourier error when PTYK_FLAG_RMS is set, else 0.  PTYK_EDEVICE: object and
+ * probe may be half updated; set both again before going on. */
 int ptyk_epie_iteration(ptyk_ctx* ctx, const int32_t* order, uint32_t flags, double* err);
 
 /* One DM iteration (DM::iteration, DM.cu:80-128).  The first call takes the cached
@@ -148,9 +149,18 @@ int ptyk_dm_iteration_timed(ptyk_ctx* ctx, uint32_t flags, float* kernel_ms);
  * PTYK_TUNE_MLS_ROW_WAVES: 1 (default) runs the MLs exit-wave and inverse row passes and the
  * probe-mode update for M in {128, 256} as wave tiles (one wave per tile of whole row groups,
  * no workgroup barrier between its transform stages); 0 as workgroup tiles.  The row passes give
- * bitwise the same values either way; the probe-mode sums add their frames in another order. */
+ * bitwise the same values either way; the probe-mode sums add their frames in another order.
+ * PTYK_TUNE_EPIE_TEAM: 1 (default) shares an ePIE frame of 64^2 or more among a team of workgroups
+ * where the device has a CU for each; 0 leaves it to one workgroup.  get returns the number of
+ * workgroups (0: one workgroup, no team).
+ * PTYK_TUNE_EPIE_TEAM_WAIT: how long (0..60000 ms; default 10000) a team's workgroup waits for the
+ * others.  If they do not come together (other processes hold the device; always with 0), one
+ * workgroup takes the iteration.
+ * PTYK_TUNE_EPIE_RESIDENT: most modes whose spectra a team keeps in LDS; 0 (default) = as many as
+ * fit.  get returns the number for the handle's modes. */
 enum { PTYK_TUNE_DM_WAVE = 1, PTYK_TUNE_MLS_MOD_CB = 2, PTYK_TUNE_MLS_PUM_FPC = 3, PTYK_TUNE_MLS_GRAPHS = 4,
-       PTYK_TUNE_DM_GRAPH = 5, PTYK_TUNE_MLS_ROW_WAVES = 6 };
+       PTYK_TUNE_DM_GRAPH = 5, PTYK_TUNE_MLS_ROW_WAVES = 6, PTYK_TUNE_EPIE_TEAM = 7, PTYK_TUNE_EPIE_TEAM_WAIT = 8,
+       PTYK_TUNE_EPIE_RESIDENT = 9 };
 int ptyk_set_tuning(ptyk_ctx* ctx, int32_t key, int32_t value);
 int ptyk_get_tuning(ptyk_ctx* ctx, int32_t key, int32_t* value);
 

@@ -52,6 +52,7 @@ struct ptyk_ctx {
   double* e_err = nullptr;
   unsigned e_epoch = 1;
   int cus = 0;  // compute units of the device
+  int epie_team = 1, epie_wait_ms = 10000, epie_resident = 0;  // PTYK_TUNE_EPIE_*
   // DM state
   float2* psi = nullptr;
   int* tile_ptr = nullptr;
@@ -580,6 +581,8 @@ static TeamBudget* team_budget(int device) {
   return &all[device];
 }
 
+static int epie_team(const ptyk_ctx* c) { return c->epie_team ? epie_team_size(c->cfg.frame_size, c->cus) : 0; }
+
 int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, double* err) {
   if (!c || !order) return fail(c, PTYK_EINVAL, "null argument");
   if (!c->have_frames || !c->have_pos || !c->have_probe)
@@ -621,31 +624,35 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
   a.update_probe = (flags & PTYK_FLAG_UPDATE_PROBE) ? 1 : 0;
   a.rms = (flags & PTYK_FLAG_RMS) ? 1 : 0;
   a.tex_quantize = c->cfg.tex_quantize;
-  const int team = epie_team_size(a.m, c->cus);
-  a.team_size = team;
+  a.team_size = epie_team(c);
   a.team_flags = c->e_flags;
   a.team_segmax = c->e_segmax;
   a.team_rowmax = c->e_rowmax;
   a.team_err = c->e_err;
   a.team_epoch = c->e_epoch;
-  a.team_limit = 1000000000LL;  // 10 s
+  a.team_limit = 100000LL * c->epie_wait_ms;
+  a.k_res = c->epie_resident;
   double s[PTYK_SCAL_COUNT + 1];
-  {
-    TeamSlots slots(team_budget(c->cfg.device), c->cus, team);  // one workgroup per CU, whatever else fits there
+  auto pass = [&] {
+    TeamSlots slots(team_budget(c->cfg.device), c->cus, a.team_size);  // one workgroup per CU, whatever else fits there
     hipError_t e = epie_iteration(a, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(s, c->scal, sizeof(s), hipMemcpyDeviceToHost, c->stream);
     const hipError_t es = hipStreamSynchronize(c->stream);  // before the team's place is given back
-    HIPCHK(c, e);
-    HIPCHK(c, es);
-  }
-  if (team) {
-    const bool done = s[PTYK_EPIE_DONE] == (double)c->e_epoch;
+    return e != hipSuccess ? e : es;
+  };
+  HIPCHK(c, pass());
+  if (a.team_size) {
+    const double mark = s[PTYK_EPIE_MARK], epoch = c->e_epoch;
     c->e_epoch += epie_team_barriers(n);
-    if (!done) {  // the flags stand anywhere: bring them to where the next iteration starts
+    if (mark != epoch) {  // the flags stand anywhere: bring them to where the next iteration starts
       const std::vector<unsigned long long> at(PTYK_EPIE_TEAM_MAX * PTYK_EPIE_FLAG_STRIDE,
                                                team_flag(c->e_epoch, 0));
       HIPCHK(c, hipMemcpy(c->e_flags, at.data(), at.size() * sizeof(at[0]), hipMemcpyHostToDevice));
-      return fail(c, PTYK_EDEVICE, "ePIE: the workgroups of a team were not on the device together; the iteration is incomplete");
+      if (mark == -epoch)
+        return fail(c, PTYK_EDEVICE,
+                    "ePIE: a workgroup of a team was lost; object and probe are undefined and have to be set again");
+      a.team_size = 0;  // they never were on the device together, and have changed nothing
+      HIPCHK(c, pass());
     }
   }
   if (err) *err = a.rms ? s[PTYK_SCAL_ERROR] / n : 0.0;
@@ -916,6 +923,21 @@ int ptyk_set_tuning(ptyk_ctx* c, int32_t key, int32_t value) {
     c->mls_row_waves = value;
     return PTYK_OK;
   }
+  if (key == PTYK_TUNE_EPIE_TEAM) {
+    if (value != 0 && value != 1) return fail(c, PTYK_EINVAL, "ePIE teams: 0 or 1");
+    c->epie_team = value;
+    return PTYK_OK;
+  }
+  if (key == PTYK_TUNE_EPIE_TEAM_WAIT) {
+    if (value < 0 || value > 60000) return fail(c, PTYK_EINVAL, "ePIE team wait: 0 to 60000 ms");
+    c->epie_wait_ms = value;
+    return PTYK_OK;
+  }
+  if (key == PTYK_TUNE_EPIE_RESIDENT) {
+    if (value < 0) return fail(c, PTYK_EINVAL, "ePIE modes in LDS: 0 (as many as fit) or a number of modes");
+    c->epie_resident = value;
+    return PTYK_OK;
+  }
   if (key == PTYK_TUNE_DM_GRAPH) {
     if (value != 0 && value != 1) return fail(c, PTYK_EINVAL, "DM graphs: 0 or 1");
     c->dm_graph = value;
@@ -929,6 +951,12 @@ int ptyk_get_tuning(ptyk_ctx* c, int32_t key, int32_t* value) {
   if (!c || !value) return PTYK_EINVAL;
   if (key == PTYK_TUNE_DM_WAVE) {
     *value = dm_wave_frames(c);
+    return PTYK_OK;
+  }
+  if (key == PTYK_TUNE_EPIE_TEAM || key == PTYK_TUNE_EPIE_TEAM_WAIT || key == PTYK_TUNE_EPIE_RESIDENT) {
+    *value = key == PTYK_TUNE_EPIE_TEAM        ? epie_team(c)
+             : key == PTYK_TUNE_EPIE_TEAM_WAIT ? c->epie_wait_ms
+                                               : epie_team_resident(c->cfg.frame_size, c->cfg.n_modes, c->epie_resident);
     return PTYK_OK;
   }
   if (key == PTYK_TUNE_DM_GRAPH) {

@@ -297,15 +297,20 @@ __device__ __forceinline__ float ld_dev(const float* p) {
 __device__ __forceinline__ void st_dev(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void st_dev(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Team barrier in two halves, so that work which needs nothing from the others can stand between.
 // arrive: this workgroup's stores have reached the coherence point (a store leaves vmcnt when it is
 // acknowledged there), then its flag: the epoch and a value of the workgroup (read by thread 0 from
 // LDS, in *value; a non-negative float).  wait: one wave polls all W flags, one per lane, and leaves
 // the largest of the values in *most.  Why a slow reader cannot meet a later barrier's value: see
-// team_word (ptyk_team.h).  The wait is bounded (limit ticks of the 100 MHz clock): the
-// host admits no more workgroups than the device can hold at once, so it ends unless the device is
-// lost to something else; then every workgroup gives up and the host reports it.
+// team_word (ptyk_team.h).  The wait is bounded (limit ticks of the 100 MHz clock; 0: one
+// look): the host admits no more workgroups than the device can hold at once, but other processes may
+// have theirs there.  Who passes the second barrier, behind which the object is written, knows that
+// all have passed the first, so that all are there; if nobody does, nothing has changed and one workgroup
+// can take the iteration instead.
 __device__ __forceinline__ void team_arrive(unsigned long long* flags, int w, unsigned epoch, const unsigned* value) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -334,7 +339,7 @@ __device__ __forceinline__ bool team_wait(const unsigned long long* flags, unsig
           v = max(v, team_value(f));  // values are non-negative floats: ordered as integers
         }
       ok = __all(here);
-      if (ok) break;
+      if (ok || limit == 0) break;
       if (i == 1024) t0 = wall_clock64();
       if (i > 1024 && (i & 255) == 0 && wall_clock64() - t0 > limit) break;
     }
@@ -760,6 +765,7 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
       if (lane == 0) atomicMax(&value[2], __float_as_uint(o));
     }
     if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[1])) return;
+    if (s == 0 && tid == 0) st_dev(a.scal + PTYK_EPIE_MARK, -(double)a.team_epoch);  // from here on the state changes
 
     // ---- rows: psi - psi_old, object update at the rounded position (d_updateObjectArray(M))
     float2 d[PPT], up[PPT];
@@ -899,7 +905,7 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
     if (lane == 0) atomicMax(&value[0], __float_as_uint(m));
   }
   err = block_sum<NT>(err, redd);
-  if (tid == 0) __hip_atomic_store(a.team_err + w, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) st_dev(a.team_err + w, err);
   team_arrive(flags, w, ++epoch, value);
   if (w != 0) return;
   if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[0])) return;
@@ -909,7 +915,7 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
     a.scal[0] = a.update_probe ? obj_max : most[0];
     a.scal[1] = a.update_probe ? most[0] : probe_max;
     a.scal[2] = e;
-    a.scal[PTYK_EPIE_DONE] = a.team_epoch;  // the whole chain ran
+    st_dev(a.scal + PTYK_EPIE_MARK, (double)a.team_epoch);  // the whole chain ran
   }
 }
 
@@ -922,20 +928,29 @@ static hipError_t epie_impl(const EpieArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int M>
+struct TeamLds {
+  using T = Team<M>;
+  static constexpr size_t base = (size_t)(T::TILE + T::TILE_B) * sizeof(float2), tile = (size_t)T::TILE * sizeof(float2);
+  static constexpr int room = (int)((128 * 1024 - base) / tile);  // modes; of the CU's 160 KiB, beside the static arrays
+  static int resident(int k_use, int most) {
+    return k_use > 1 ? std::min({k_use, room, most > 0 ? most : room}) : 0;
+  }
+};
 template <int M, bool MULTI>
 static hipError_t epie_team_launch(EpieArgs a, hipStream_t s) {
   using T = Team<M>;
-  constexpr size_t base = (size_t)(T::TILE + T::TILE_B) * sizeof(float2), tile = (size_t)T::TILE * sizeof(float2);
-  constexpr size_t room = 128 * 1024;  // of the CU's 160 KiB, beside the static arrays
-  a.k_res = MULTI ? (int)std::min<size_t>(a.k_use, (room - base) / tile) : 0;
-  const size_t lds = base + a.k_res * tile;
+  a.k_res = TeamLds<M>::resident(a.k_use, a.k_res);
+  const size_t lds = TeamLds<M>::base + a.k_res * TeamLds<M>::tile;
   hipError_t e = hipFuncSetAttribute((const void*)k_epie_team<M, MULTI>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds);
   if (e != hipSuccess) return e;
   if (a.update_probe)
     hipLaunchKernelGGL(k_canvas_maxima, dim3((unsigned)((a.obj_rows + 3) / 4)), dim3(256), 0, s, a.obj_int, a.obj_rows,
                        a.obj_cols, a.team_segmax, a.team_rowmax);
-  hipLaunchKernelGGL((k_epie_team<M, MULTI>), dim3(T::W), dim3(T::NT), lds, s, a);
+  // with no wait at all, one workgroup stays out: the others find it missing and end (what becomes of a
+  // team that does not come together, for tests)
+  hipLaunchKernelGGL((k_epie_team<M, MULTI>), dim3(a.team_limit ? T::W : T::W - 1), dim3(T::NT), lds, s, a);
   return hipGetLastError();
 }
 template <int M>
@@ -949,6 +964,15 @@ static hipError_t epie_team_impl(const EpieArgs& a, hipStream_t s) {
 int epie_team_size(int m, int cus) {
   const int w = m == 64 ? Team<64>::W : m == 128 ? Team<128>::W : m == 256 ? Team<256>::W : m == 512 ? Team<512>::W : 0;
   return w <= cus ? w : 0;
+}
+int epie_team_resident(int m, int k_use, int most) {
+  switch (m) {
+    case 64: return TeamLds<64>::resident(k_use, most);
+    case 128: return TeamLds<128>::resident(k_use, most);
+    case 256: return TeamLds<256>::resident(k_use, most);
+    case 512: return TeamLds<512>::resident(k_use, most);
+    default: return 0;
+  }
 }
 unsigned epie_team_barriers(int n_pos) { return 3u * (unsigned)n_pos + 1u; }
 

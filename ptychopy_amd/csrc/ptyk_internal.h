@@ -211,14 +211,18 @@ struct EpieArgs {
   int phase_constraint, update_probe, modal, rms, tex_quantize;
   // team form (team_size = epie_team_size(m, CUs) > 0): barrier flags, maxima of |O|^2 over segments of
   // canvas rows (rows x epie_segments) and over rows, and the workgroups' errors; the flags stand at team_epoch and move by epie_team_barriers(n_pos);
-  // team_limit bounds a barrier's wait (ticks of the 100 MHz clock); k_res is set by the launch
+  // team_limit bounds a barrier's wait (ticks of the 100 MHz clock; 0: one look); k_res: most modes whose
+  // spectra stay in LDS (0: as many as fit)
   unsigned long long* team_flags; float *team_segmax, *team_rowmax; double* team_err;
   unsigned team_epoch; int team_size, k_res; long long team_limit;
 };
-#define PTYK_EPIE_DONE PTYK_SCAL_COUNT             // scal slot the team form sets to team_epoch when the iteration ran
+// scal slot of the team form: team_epoch when the iteration ran, -team_epoch from where it may have changed the
+// state (anything else: it has not)
+#define PTYK_EPIE_MARK PTYK_SCAL_COUNT
 #define PTYK_EPIE_SEG 64                           // canvas columns of a segment
 __host__ __device__ constexpr int epie_segments(int obj_cols) { return (obj_cols + PTYK_EPIE_SEG - 1) / PTYK_EPIE_SEG; }
 int epie_team_size(int m, int cus);                // workgroups that share a frame; 0: one workgroup
+int epie_team_resident(int m, int k_use, int most); // modes whose spectra stay in LDS
 unsigned epie_team_barriers(int n_pos);
 hipError_t epie_iteration(const EpieArgs& a, hipStream_t s);
 

@@ -149,7 +149,7 @@ def _flat_counts(p):
     (256, 2, 40.2, 1, True, True),
     (256, 2, 21.9, 4, True, False),
     (512, 2, 33.3, 1, False, False),
-    (512, 2, 27.1, 3, True, False),   # more modes than LDS tiles
+    (512, 2, 27.1, 3, True, False),
 ])
 def test_team_iterations_match_oracle(gpu, orc, m, n_side, step, modes, rms, pc):
     """Frames shared by a team of workgroups: sizes, modes in and out of LDS, small and wide canvases."""
@@ -278,3 +278,63 @@ def test_canvas_maximum_wherever_it_lies(gpu, orc, m, rows, cols, at):
             e.set_probe(probe * np.exp(0.3j * rng.standard_normal(probe.shape)))
             e.refresh_maxima()
             _check(e, orc, p, a64, [0, 1], E.FLAG_UPDATE_PROBE)
+
+
+@pytest.mark.parametrize("m,modes,most", [(64, 3, 1), (128, 4, 2), (256, 14, 0), (512, 7, 0)])
+def test_modes_beyond_lds_match_oracle(gpu, orc, m, modes, most):
+    """More modes than a workgroup's LDS holds (or is let hold): the others' spectra wait in the exchange
+    buffer, with an even and an odd number of transform stages."""
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=m, n_side=2, step=27.1, seed=m + modes, modes=modes, photons=100.0 * m * m)
+    rng = np.random.default_rng(m)
+    flags = E.FLAG_UPDATE_PROBE | E.FLAG_UPDATE_MODES
+    with _near_engine(p, _flat_counts(p)) as e:
+        e.set_tuning(E.TUNE_EPIE_RESIDENT, most)
+        assert 0 < e.get_tuning(E.TUNE_EPIE_RESIDENT) < modes
+        amp = e.get_frames().astype(np.float64)
+        for f in (flags, flags | E.FLAG_RMS):
+            _check(e, orc, p, amp, rng.permutation(p["n"]), f, k_use=modes, modal=True)
+
+
+@pytest.mark.parametrize("m,modes", [(64, 1), (64, 2), (128, 1), (128, 3), (256, 1), (256, 2), (512, 1), (512, 2)])
+def test_one_workgroup_matches_oracle(gpu, orc, m, modes):
+    """The form without a team (devices that cannot hold one), at the sizes that have a team."""
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=m, n_side=2, step=27.1, seed=m + modes, modes=modes, photons=100.0 * m * m)
+    rng = np.random.default_rng(m)
+    flags = E.FLAG_UPDATE_PROBE | (E.FLAG_UPDATE_MODES if modes > 1 else 0)
+    with _near_engine(p, _flat_counts(p)) as e:
+        assert e.get_tuning(E.TUNE_EPIE_TEAM) > 0
+        e.set_tuning(E.TUNE_EPIE_TEAM, 0)
+        assert e.get_tuning(E.TUNE_EPIE_TEAM) == 0
+        amp = e.get_frames().astype(np.float64)
+        for f in (flags, (flags & ~E.FLAG_UPDATE_PROBE) | E.FLAG_PHASE_CONSTRAINT, flags | E.FLAG_RMS):
+            _check(e, orc, p, amp, rng.permutation(p["n"]), f, k_use=modes, modal=modes > 1)
+
+
+@pytest.mark.parametrize("m,modes", [(64, 1), (128, 2), (256, 1), (512, 1)])
+def test_a_team_that_does_not_come_together(gpu, m, modes):
+    """A team whose workgroups do not wait for one another gives up at once: one workgroup takes the
+    iteration, with its own result to the bit, and the next team starts as if nothing had been."""
+    from ptychopy_amd import _engine as E
+    p = make_problem(m=m, n_side=2, step=27.1, seed=m, modes=modes)
+    order = np.random.default_rng(m).permutation(p["n"])
+    flags = E.FLAG_UPDATE_PROBE | E.FLAG_RMS | (E.FLAG_UPDATE_MODES if modes > 1 else 0)
+
+    def states(*tuning):
+        out = []
+        with _near_engine(p) as e:
+            for t in tuning:
+                for key, value in t.items():
+                    e.set_tuning(key, value)
+                err = e.epie_iteration(order, flags)
+                out.append([e.get_object().view(np.uint32), e.get_probe().view(np.uint32),
+                            e.get_scalars().view(np.uint64), np.float64(err).view(np.uint64)])
+        return out
+
+    one, team = {E.TUNE_EPIE_TEAM: 0}, {E.TUNE_EPIE_TEAM: 1, E.TUNE_EPIE_TEAM_WAIT: 10000}
+    want = states(one, one, team, team)
+    got = states({E.TUNE_EPIE_TEAM_WAIT: 0}, {}, team, team)
+    for a, b in zip(want, got):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
