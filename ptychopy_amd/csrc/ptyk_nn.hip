@@ -16,12 +16,12 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <random>
 #include <string>
 #include <vector>
 
 #include "../../include/ptyk.h"
 #include "ptyk_device.h"
+#include "ptyk_draw.h"
 #include "ptyk_internal.h"
 
 namespace ptyk {
@@ -1264,11 +1264,10 @@ int ptyk_net_create(int32_t device, int32_t size, int32_t base_channels, int32_t
   }
   // He-normal weights (seeded), zero biases
   std::vector<float> w(h->n.nparam, 0.f);
-  std::mt19937_64 g(seed);
-  std::normal_distribution<double> nd(0.0, 1.0);
+  NormalDraw nd(seed);
   for (const auto& L : h->n.layers) {
     const double sd = std::sqrt(2.0 / (L.cin * L.ks * L.ks));
-    for (long i = 0; i < (long)L.cout * L.cin * L.ks * L.ks; ++i) w[L.woff + i] = (float)(sd * nd(g));
+    for (long i = 0; i < (long)L.cout * L.cin * L.ks * L.ks; ++i) w[L.woff + i] = (float)(sd * nd());
   }
   int r = ptyk_net_set_params(h, w.data());
   if (r) {

@@ -1,6 +1,11 @@
 """Pins of the FP64 network oracle (oracle/oracle_nn.cpp): one convolution against scipy's
 correlation, the full backward pass against central finite differences."""
+import shutil
+import subprocess
+from pathlib import Path
+
 import numpy as np
+import pytest
 from scipy import signal
 
 
@@ -66,3 +71,13 @@ def test_weighted_loss_closed_form_and_gradient(orc):
         lm = orc.nn_forward_backward(pm.astype(np.float32), x, t, c, grad=False, weight=w)[1]
         fd = (lp - lm) / (float(np.float32(pp[i])) - float(np.float32(pm[i])))
         assert abs(fd - g[i]) <= 1e-4 * max(1e-3, abs(g[i])) + 1e-7, (i, fd, g[i])
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_initial_weights_draw_as_the_standard_library(tmp_path):
+    root = Path(__file__).resolve().parent.parent
+    exe = tmp_path / "normal_draw"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{root / 'ptychopy_amd' / 'csrc'}",
+                    str(root / "tests" / "seam" / "normal_draw.cpp"), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
