@@ -1218,7 +1218,7 @@ struct ptyk_net {
   int64_t data_cap = 0;  // samples the device buffers hold room for
   int64_t* idx = nullptr;
   int64_t idx_cap = 0;
-  hipStream_t copy = nullptr;  // the predictions' copies to and from the host
+  hipStream_t copy = nullptr;  // the predictions' copies to and from the host; made by the first one
   float* io = nullptr;         // `held` batches of samples and of results
   int64_t held = 0;
 };
@@ -1252,13 +1252,11 @@ int ptyk_net_create(int32_t device, int32_t size, int32_t base_channels, int32_t
   ptyk_net* h = new ptyk_net();
   h->device = device;
   hipError_t e = hipStreamCreateWithFlags(&h->n.stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->copy, hipStreamNonBlocking);
   if (e == hipSuccess) e = nn_create(h->n, size, base_channels, batch);
   if (e != hipSuccess) {
     g_net_err = std::string("network allocation: ") + hipGetErrorString(e);
     nn_free(h->n);
-    for (hipStream_t st : {h->n.stream, h->copy})
-      if (st) hipStreamDestroy(st);
+    if (h->n.stream) hipStreamDestroy(h->n.stream);
     delete h;
     return e == hipErrorOutOfMemory ? PTYK_ENOMEM : PTYK_EDEVICE;
   }
@@ -1498,6 +1496,7 @@ static int net_predict(ptyk_net* h, const float* inputs, int64_t n, float* outpu
   hipSetDevice(h->device);
   const long ss = (long)h->n.s * h->n.s;
   const int B = h->n.batch;
+  if (!h->copy) NCHK(h, hipStreamCreateWithFlags(&h->copy, hipStreamNonBlocking));
   const hipStream_t s = h->n.stream, cs = h->copy;
   const size_t batch_bytes = (size_t)B * 3 * ss * sizeof(float);
   // batches held at once: 32, and 64 MiB of samples and results
