@@ -495,7 +495,7 @@ __device__ __forceinline__ void store_weight(const LayerTable& tb, long i, float
   int l = 0;
   while (l + 1 < NN_LAYERS && i >= tb.l[l + 1].woff) ++l;
   const LayerMap& m = tb.l[l];
-  if (i >= m.boff || m.ks != 3 || m.cin == 1) return;
+  if (i >= m.boff || m.ks != 3 || l == 0) return;
   const int k = (int)(i - m.woff), t = k % 9, ci = pad_channel(m, k / 9 % m.cin), co = k / (9 * m.cin);
   auto frag = [](int o, int chunks, int c, int tap) {
     return ((((long)(o >> 5) * chunks + (c >> 5)) * 9 + tap) * 2 + (c >> 4 & 1)) * 512 + ((o & 31) + 32 * (c >> 3 & 1)) * 8 +

@@ -196,3 +196,28 @@ def test_tile_shapes_agree_between_batch_sizes(s, c, batch):
     for li, (wl, bl) in enumerate(sl):
         for part in (wl, bl):
             assert rel(g[part], gs[part]) <= 1e-4, (li, rel(g[part], gs[part]))
+
+
+@pytest.mark.parametrize("s,c,batch", [(16, 1, 2)])
+def test_channels_that_fill_no_chunk_match_oracle(s, c, batch):
+    """Channel counts whose tensors end inside a chunk of 32 or inside a group of 8, skip concatenations
+    among them, or one channel throughout; bounds as in the gradient test."""
+    rng = np.random.default_rng(c)
+    x, t = sample(rng, batch, s)
+    with warmstart.Net(size=s, c=c, batch=batch, seed=3) as net:
+        sl, _ = layer_slices(c)
+        p = net.get_params()
+        for _, b in sl:
+            p[b] = rng.normal(0, 0.05, size=b.stop - b.start)
+        net.set_params(p)
+        loss, g = net.gradient(x, t)
+        out = net.predict(x)
+    ref_out, ref_loss, ref_g = oracle.nn_forward_backward(p, x, t, c, emulate_bf16=True)
+    pp = (p * (1 + 1e-6 * np.random.default_rng(99).standard_normal(p.size))).astype(np.float32)
+    n_out, _, n_g = oracle.nn_forward_backward(pp, x, t, c, emulate_bf16=True)
+    assert rel(out, ref_out) <= max(1.5e-2, 3 * rel(n_out, ref_out))
+    assert abs(loss - ref_loss) <= 1e-2 * ref_loss
+    for li, (wl, bl) in enumerate(sl):
+        for part in (wl, bl):
+            err, floor = rel(g[part], ref_g[part]), rel(n_g[part], ref_g[part])
+            assert err <= max(2e-2, 3 * floor), (li, err, floor)
