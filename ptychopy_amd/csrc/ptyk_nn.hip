@@ -2,8 +2,10 @@
 // c, 2c, 4c, 8c with c = 32 by default) mapping a log-scaled diffraction amplitude (1 x S x S)
 // to the object patch's amplitude and phase (2 x S x S).  No reference counterpart.
 //
-// Tensors are pixel-major (NHWC) with the channels padded to a multiple of 32 by zeros, so that the
-// 8 channels a lane feeds to a matrix instruction are 16 contiguous bytes.  Every 3 x 3 convolution
+// Tensors are pixel-major (NHWC) with the channels padded to a multiple of 8 by zeros, so that the
+// 8 channels a lane feeds to a matrix instruction are 16 contiguous bytes; the products run over chunks
+// of 32 channels, of which those past a tensor's last are zeros in LDS and never stored (a network of 8
+// channels would else hold twice its tensors' bytes).  Every 3 x 3 convolution
 // between them is an implicit GEMM on v_mfma_f32_32x32x16_bf16 (BF16 operands, FP32 accumulation;
 // no im2col buffer): k_conv3 for the forward pass and the data gradient, k_wgrad3 for the weight
 // gradient (split over pixels into partial tiles summed in a fixed order).  The first layer (one
@@ -38,36 +40,37 @@ namespace {
 constexpr int CT = 256;      // threads of the convolution kernels (4 waves)
 constexpr int NN_LAYERS = 15;
 inline int pad32(int c) { return (c + 31) / 32 * 32; }
+inline int pad8(int c) { return (c + 7) / 8 * 8; }
 
 __device__ __forceinline__ bf16 to_bf(float v) { return (bf16)v; }
 __device__ __forceinline__ unsigned bf_bits(float v) { return __builtin_bit_cast(u16, to_bf(v)); }
 __device__ __forceinline__ float bf_val(unsigned bits16) { return __uint_as_float(bits16 << 16); }
 __device__ __forceinline__ unsigned bf_pair(float a, float b) { return bf_bits(a) | (bf_bits(b) << 16); }
 
-// A layer's input: channels [0, cp0) from p0, [cp0, cp0 + cp1) from p1, both NHWC with those padded
-// channel counts; up0: p0 has half the resolution (nearest upsampling).
+// A layer's input: p0's channels, then p1's, both NHWC with cp0 and cp1 stored channels, each in chunks
+// of 32; up0: p0 has half the resolution (nearest upsampling).
 struct Src {
   const void* p0;
   const void* p1;
   int cp0, cp1, up0;
 };
 
-// Element offset of 8-channel group c8 (of 32-channel chunk ch) of pixel (b, y, x), and its tensor.
+// The tensor behind chunk ch: its stored channels, the chunk's first among them, and whether it is upsampled.
 __device__ __forceinline__ const void* src_base(const Src& s, int ch, int* cp, int* coff, int* up) {
   const bool first = ch * 32 < s.cp0;
   *cp = first ? s.cp0 : s.cp1;
-  *coff = first ? ch * 32 : ch * 32 - s.cp0;
+  *coff = (first ? ch : ch - (s.cp0 + 31) / 32) * 32;
   *up = first ? s.up0 : 0;
   return first ? s.p0 : s.p1;
 }
 
-// Where a tile of 32 output channels goes.  Forward: bias, ReLU, BF16.  Data gradient: FP32, zeroed
+// Where a tile of 32 output channels goes (cp of them in all are stored).  Forward: bias, ReLU, BF16.  Data gradient: FP32, zeroed
 // where the BF16 activation mask is not positive (the ReLU of the layer that made it; NULL: no ReLU);
 // sum4: the 2 x 2 sums go to a half-resolution tensor (the gradient of the upsampling).
 struct Dst {
   void* p;
   const bf16* mask;
-  int cp, coff, sum4;
+  int cp, sum4;
 };
 
 struct ConvArgs {
@@ -92,7 +95,9 @@ struct ConvArgs {
 // reversed and their channels exchanged).
 // AHEAD: the next chunk's loads are in flight during a chunk's products (as long as the registers for
 // them are there).
-template <int NCO, int ROWS, bool GRAD>
+// PART: some tensor's channels do not fill its last chunk (the tests for it cost 4 % of a training step of
+// 32 channels, where all do).
+template <int NCO, int ROWS, bool GRAD, bool PART>
 __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
   constexpr bool AHEAD = NCO * ROWS <= 4;
   constexpr int TR = 4 * ROWS + 2, TC = 34, XN = TR * TC * 4, WF = 9 * 2 * 64, WN = NCO * WF;  // 16-byte pieces
@@ -124,11 +129,12 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
 #define PTYK_CONV_PIECE(i)                                                                              \
   const int e = tid + (i)*CT, q = e & 3, pc = e >> 2, r = pc / TC, c = pc - r * TC;                     \
   const int y = y0 + r - 1, x = x0 + c - 1;                                                             \
-  const bool in = e < XN && y >= 0 && y < a.h && x >= 0 && x < a.w_px;                                  \
+  const bool in = e < XN && y >= 0 && y < rows && x >= 0 && x < a.w_px;                                  \
   const long off = in ? (img + (y >> up) * sw + (x >> up)) * cp + coff + q * 8 : 0
 #define PTYK_CONV_CHUNK(ch)                                                                             \
   int cp, coff, up;                                                                                     \
   const void* const base = src_base(a.in, ch, &cp, &coff, &up);                                         \
+  const int rows = !PART || coff + (tid & 3) * 8 < cp ? a.h : 0; /* of this thread's channels, if any */ \
   const int sw = a.w_px >> up;                                                                          \
   const long img = (long)b * (a.h >> up) * sw
 #define PTYK_CONV_LOAD(ch)                                                                              \
@@ -210,7 +216,10 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
   for (int t = 0; t < NCO; ++t) {
     const int ot = grp * NCO + t;
     const Dst d = ot < a.out0_tiles ? a.out0 : a.out1;
-    const int c0 = (ot < a.out0_tiles ? ot : ot - a.out0_tiles) * 32 + d.coff;
+    const int c0 = (ot < a.out0_tiles ? ot : ot - a.out0_tiles) * 32;
+    bool kept[4];  // groups of 8 channels
+#pragma unroll
+    for (int g = 0; g < 4; ++g) kept[g] = !PART || c0 + 8 * g < d.cp;
     if (!GRAD) {
       float bias[16];
 #pragma unroll
@@ -231,7 +240,7 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
             v[i] = acc[t][r][4 * g + i] + bias[4 * g + i];
             if (a.relu) v[i] = fmaxf(v[i], 0.f);
           }
-          *reinterpret_cast<uint2*>(o + 8 * g) = make_uint2(bf_pair(v[0], v[1]), bf_pair(v[2], v[3]));
+          if (kept[g]) *reinterpret_cast<uint2*>(o + 8 * g) = make_uint2(bf_pair(v[0], v[1]), bf_pair(v[2], v[3]));
         }
       }
     } else if (d.sum4) {  // image sizes are even here: whole 2 x 2 blocks, rows in pairs, columns in lane pairs
@@ -249,7 +258,7 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
               const float sx = __shfl_xor(s, 1, 64), ux = __shfl_xor(u, 1, 64);
               v[i] = s + sx + u + ux;
             }
-            if (y < a.h && x < a.w_px && !(lane & 1)) {
+            if (y < a.h && x < a.w_px && !(lane & 1) && kept[g]) {
               const long o = px * d.cp + c0 + 8 * g + 4 * half;
               const uint2 m = *reinterpret_cast<const uint2*>(d.mask + o);
               const unsigned mm[4] = {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16};
@@ -269,6 +278,7 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
         const long o0 = (((long)b * a.h + y) * a.w_px + x) * d.cp + c0 + 4 * half;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+          if (!kept[g]) continue;
           float v[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] = acc[t][r][4 * g + i];
@@ -292,10 +302,10 @@ __global__ __launch_bounds__(CT, 2) void k_conv3(ConvArgs a) {
 
 struct WgradArgs {
   Src x;              // BF16 input of the layer
-  const float* dz;    // FP32 gradient of its pre-activation output, NHWC with cpo channels
+  const float* dz;    // FP32 gradient of its pre-activation output, NHWC with cz channels
   float* part;        // [chunk][output tile][input tile][tap][32][32] (output, input channel)
   double* bpart;      // [chunk][cpo]: bias gradient
-  int batch, h, w_px, cpo, tiles_o, tiles_i, tiles_x, tiles_y, chunks;
+  int batch, h, w_px, cz, cpo, tiles_o, tiles_i, tiles_x, tiles_y, chunks;
 };
 
 // Weight gradient: D[co][ci] per tap = sum over pixels of dZ[p][co] x[p + tap][ci], a GEMM whose
@@ -306,6 +316,7 @@ struct WgradArgs {
 // every operand is one aligned 16-byte read.  Per wave and 16 pixels: 2 + 12 reads for 18
 // instructions.  Channel pitches of 528 and 656 bytes spread 8 lanes over the banks.
 constexpr int WG_R = 8, WG_ZP = WG_R * 64 + 16, WG_XP = (WG_R + 2) * 64 + 16;  // bytes per channel
+template <bool PART>  // as for k_conv3
 __global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
   extern __shared__ __align__(16) unsigned char wg_lds[];
   unsigned char* const zs = wg_lds;                // 32 x WG_ZP
@@ -317,6 +328,8 @@ __global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
   const void* base = src_base(a.x, it, &cp, &coff, &up);
   const int sw = a.w_px >> up, sh = a.h >> up;
   const int cpair = tid & 15, slot = tid >> 4;  // 2 channels, one of 16 pixel groups of 8
+  // rows of this thread's channels: none where they are not stored
+  const int zh = !PART || ot * 32 + cpair * 2 < a.cz ? a.h : 0, xh = !PART || coff + cpair * 2 < cp ? a.h : 0;
   v16f acc[9];
 #pragma unroll
   for (int t = 0; t < 9; ++t)
@@ -334,11 +347,11 @@ __global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
     for (int i = 0; i < WG_R * 4 / 16; ++i) {
       const int g = slot + i * 16, r = g >> 2, xg = (g & 3) * 8, y = y0 + r;
       float2 v[8];
-      const int left = y < a.h ? a.w_px - (x0 + xg) : 0;  // pixels from here to the row's end
-      const float* zp = a.dz + (((long)b * a.h + min(y, a.h - 1)) * a.w_px + x0 + xg) * a.cpo + ot * 32 + cpair * 2;
+      const int left = y < zh ? a.w_px - (x0 + xg) : 0;  // pixels from here to the row's end
+      const float* zp = a.dz + (((long)b * a.h + min(y, a.h - 1)) * a.w_px + x0 + xg) * a.cz + ot * 32 + cpair * 2;
 #pragma unroll
       for (int p = 0; p < 8; ++p)
-        v[p] = p < left ? *reinterpret_cast<const float2*>(zp + p * a.cpo) : make_float2(0.f, 0.f);
+        v[p] = p < left ? *reinterpret_cast<const float2*>(zp + p * a.cz) : make_float2(0.f, 0.f);
       if (it == 0) {
 #pragma unroll
         for (int p = 0; p < 8; ++p) {
@@ -358,7 +371,7 @@ __global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
       const int g = slot + i * 16, r = g >> 2, xg = (g & 3) * 8, y = y0 + r - 1;
       if (g >= (WG_R + 2) * 4) break;
       unsigned v[10];  // two channels of pixels xg - 1 .. xg + 8
-      const int left = y >= 0 && y < a.h ? a.w_px - (x0 + xg - 1) : 0;
+      const int left = y >= 0 && y < xh ? a.w_px - (x0 + xg - 1) : 0;
       const bf16* xp = (const bf16*)base + ((long)b * sh + (max(y, 0) >> up)) * sw * cp + coff + cpair * 2;
 #pragma unroll
       for (int p = 0; p < 10; ++p)
@@ -442,7 +455,7 @@ __global__ __launch_bounds__(CT, 2) void k_wgrad3(WgradArgs a) {
 struct LayerMap {
   long woff, boff, foff, goff;  // parameters; forward and data-gradient fragments
   int cin, cout, ks, c0;        // c0: real channels of the first input tensor (cin when there is one)
-  int cp0, cpi, cpo;            // padded: first input tensor, all inputs, outputs
+  int cp0, cpi, cpo;            // in chunks of 32: first input tensor, all inputs, outputs
 };
 struct LayerTable {
   LayerMap l[NN_LAYERS];
@@ -565,15 +578,17 @@ __global__ __launch_bounds__(256) void k_first_fwd(const bf16* __restrict__ x, c
 
 // Its weight and bias gradient: thread = one of 32 channels (blockIdx.y) x one of 8 lanes, which take
 // segments of up to 16 pixels of a row and slide the 3 x 3 window along them; the block's sums go to
-// part[block][tap][cp] and bpart[block][cp].
-__global__ __launch_bounds__(256) void k_first_wgrad(const bf16* __restrict__ x, const float* __restrict__ dz, int cp,
+// part[block][tap][channel] and bpart[block][channel], the channels in whole 32s.
+// Four waves a SIMD hide its loads: 65 us for 16 samples of 256 x 256, and 101 with the two registers more
+// that leave three.
+__global__ __launch_bounds__(256, 4) void k_first_wgrad(const bf16* __restrict__ x, const float* __restrict__ dz, int cp,
                                                      long npx, int sh, int s, float* __restrict__ part,
                                                      double* __restrict__ bpart) {
   __shared__ float red[8][9][32];
   __shared__ double redb[8][32];
   constexpr int SEG = 16;
-  const int c = threadIdx.x & 31, pl = threadIdx.x >> 5, co = blockIdx.y * 32 + c;
-  const int len = min(SEG, s);
+  const int c = threadIdx.x & 31, pl = threadIdx.x >> 5, co = blockIdx.y * 32 + c, pp = gridDim.y * 32;
+  const int len = min(SEG, s), cz = min(co, cp - 1);  // sums of channels past the stored ones are not read
   float acc[9] = {};
   double bs = 0.0;
   for (long sg = (long)blockIdx.x * 8 + pl; sg < npx / len; sg += (long)gridDim.x * 8) {
@@ -582,7 +597,7 @@ __global__ __launch_bounds__(256) void k_first_wgrad(const bf16* __restrict__ x,
     const bool up = yy > 0, dn = yy + 1 < s;
     float d[SEG], v[3][SEG + 2];
 #pragma unroll
-    for (int i = 0; i < SEG; ++i) d[i] = i < len ? dz[(px + i) * cp + co] : 0.f;
+    for (int i = 0; i < SEG; ++i) d[i] = i < len ? dz[(px + i) * cp + cz] : 0.f;
 #pragma unroll
     for (int i = 0; i < SEG + 2; ++i) {
       const int cx = xx + i - 1;
@@ -606,12 +621,12 @@ __global__ __launch_bounds__(256) void k_first_wgrad(const bf16* __restrict__ x,
   for (int i = threadIdx.x; i < 9 * 32; i += 256) {
     float v = 0.f;
     for (int p = 0; p < 8; ++p) v += red[p][i / 32][i % 32];
-    part[((long)blockIdx.x * 9 + i / 32) * cp + blockIdx.y * 32 + i % 32] = v;
+    part[((long)blockIdx.x * 9 + i / 32) * pp + blockIdx.y * 32 + i % 32] = v;
   }
   if (threadIdx.x < 32) {
     double v = 0.0;
     for (int p = 0; p < 8; ++p) v += redb[p][c];
-    bpart[(long)blockIdx.x * cp + co] = v;
+    bpart[(long)blockIdx.x * pp + co] = v;
   }
 }
 // g[co][t] and the bias from the blocks' sums, one wave per value
@@ -852,7 +867,7 @@ struct NnNet {
   double* lpart = nullptr;
   long step = 0;
   struct Buf {
-    int cp = 0, h = 0;
+    int cp = 0, h = 0;   // stored channels, pixels a side
     bf16* a = nullptr;   // activation
     float* g = nullptr;  // its gradient
   };
@@ -904,11 +919,11 @@ static long conv3_blocks(const ConvArgs& a, int out_tiles) {
   const long tiles = (long)a.batch * ((a.w_px + 31) / 32) * ((a.h + 4 * ROWS - 1) / (4 * ROWS));
   return (tiles + 7) / 8 * 8 * (out_tiles / NCO);
 }
-template <int NCO, int ROWS, bool GRAD>
+template <int NCO, int ROWS, bool GRAD, bool PART>
 static hipError_t conv3_launch(ConvArgs a, int out_tiles, hipStream_t st) {
   constexpr size_t lds = (size_t)((4 * ROWS + 2) * 34 * 4 + NCO * 9 * 2 * 64) * sizeof(uint4);
   static_assert(lds <= 80 * 1024, "two workgroups per CU");
-  const hipError_t e = hipFuncSetAttribute((const void*)k_conv3<NCO, ROWS, GRAD>,
+  const hipError_t e = hipFuncSetAttribute((const void*)k_conv3<NCO, ROWS, GRAD, PART>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   a.tiles_x = (a.w_px + 31) / 32;
@@ -916,21 +931,26 @@ static hipError_t conv3_launch(ConvArgs a, int out_tiles, hipStream_t st) {
   a.groups = out_tiles / NCO;
   const long blocks = conv3_blocks<NCO, ROWS, GRAD>(a, out_tiles);
   if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_conv3<NCO, ROWS, GRAD>), dim3((unsigned)blocks), dim3(CT), lds, st, a);
+  hipLaunchKernelGGL((k_conv3<NCO, ROWS, GRAD, PART>), dim3((unsigned)blocks), dim3(CT), lds, st, a);
   return hipGetLastError();
 }
 // The largest tile that still gives the 256 CUs two workgroups each: two output tiles of 32 channels
 // halve the input reads, 16 rows halve the border; the small levels (32 x 32 and 64 x 64 pixels of 8
 // samples) run on finer tiles instead of on a quarter of the chip.
-template <bool GRAD>
-static hipError_t conv3(const ConvArgs& a, int out_tiles, hipStream_t st) {
+template <bool GRAD, bool PART>
+static hipError_t conv3_tiled(const ConvArgs& a, int out_tiles, hipStream_t st) {
   constexpr long FULL = 512;
   if (out_tiles % 2 == 0 && a.h > 8 && conv3_blocks<2, 4, GRAD>(a, out_tiles) >= FULL)
-    return conv3_launch<2, 4, GRAD>(a, out_tiles, st);
+    return conv3_launch<2, 4, GRAD, PART>(a, out_tiles, st);
   if (out_tiles % 2 == 0 && conv3_blocks<2, 2, GRAD>(a, out_tiles) >= FULL)
-    return conv3_launch<2, 2, GRAD>(a, out_tiles, st);
-  if (a.h > 8 && conv3_blocks<1, 4, GRAD>(a, out_tiles) >= FULL) return conv3_launch<1, 4, GRAD>(a, out_tiles, st);
-  return conv3_launch<1, 2, GRAD>(a, out_tiles, st);
+    return conv3_launch<2, 2, GRAD, PART>(a, out_tiles, st);
+  if (a.h > 8 && conv3_blocks<1, 4, GRAD>(a, out_tiles) >= FULL) return conv3_launch<1, 4, GRAD, PART>(a, out_tiles, st);
+  return conv3_launch<1, 2, GRAD, PART>(a, out_tiles, st);
+}
+template <bool GRAD>
+static hipError_t conv3(const ConvArgs& a, int out_tiles, hipStream_t st) {
+  const bool part = (a.in.cp0 | a.in.cp1 | a.out0.cp | a.out1.cp) % 32 != 0;
+  return part ? conv3_tiled<GRAD, true>(a, out_tiles, st) : conv3_tiled<GRAD, false>(a, out_tiles, st);
 }
 
 static Src conv_src(const NnNet& n, const ConvStep& s) {
@@ -946,7 +966,7 @@ static hipError_t conv_fwd(NnNet& n, const ConvStep& s) {
   a.in = conv_src(n, s);
   a.w = n.wf + m.foff;
   a.bias = n.w + m.boff;
-  a.out0 = Dst{n.bufs[s.out].a, nullptr, m.cpo, 0, 0};
+  a.out0 = Dst{n.bufs[s.out].a, nullptr, n.bufs[s.out].cp, 0};
   a.out0_tiles = m.cpo / 32;
   a.cout = m.cout;
   a.batch = n.batch;
@@ -977,6 +997,7 @@ static hipError_t conv_bwd(NnNet& n, const ConvStep& s) {
     a.bpart = n.bpart;
     a.batch = n.batch;
     a.h = a.w_px = hw;
+    a.cz = n.bufs[s.out].cp;
     a.cpo = m.cpo;
     a.tiles_o = m.cpo / 32;
     a.tiles_i = m.cpi / 32;
@@ -985,20 +1006,21 @@ static hipError_t conv_bwd(NnNet& n, const ConvStep& s) {
     a.chunks = wgrad_chunks(m, n.batch, hw);
     constexpr size_t lds = 32 * WG_ZP + 3 * 32 * WG_XP;
     static_assert(lds >= 9 * 1024 * sizeof(float) && lds <= 80 * 1024, "reduction scratch; two workgroups per CU");
-    const hipError_t e = hipFuncSetAttribute((const void*)k_wgrad3, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const auto kernel = (a.x.cp0 | a.x.cp1 | a.cz) % 32 ? k_wgrad3<true> : k_wgrad3<false>;
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_wgrad3, dim3((unsigned)(a.tiles_o * a.tiles_i * a.chunks)), dim3(CT), lds, n.stream, a);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_o * a.tiles_i * a.chunks)), dim3(CT), lds, n.stream, a);
     hipLaunchKernelGGL(k_wgrad_sum, dim3((unsigned)(a.tiles_o * a.tiles_i * 9 * 32 + a.tiles_o)), dim3(256), 0, n.stream, m,
                        n.partial, n.bpart, a.chunks, n.g);
   }
   ConvArgs a{};
-  a.in = Src{dz, nullptr, m.cpo, 0, 0};
+  a.in = Src{dz, nullptr, n.bufs[s.out].cp, 0, 0};
   a.w = n.wg + m.goff;
   const auto& b0 = n.bufs[s.in0];
   const bool pooled = s.in0 == B_P0 || s.in0 == B_P1 || s.in0 == B_P2;
-  a.out0 = Dst{b0.g, pooled ? nullptr : b0.a, b0.cp, 0, s.in1 >= 0 ? 1 : 0};
-  a.out0_tiles = b0.cp / 32;
-  if (s.in1 >= 0) a.out1 = Dst{n.bufs[s.in1].g, nullptr, n.bufs[s.in1].cp, 0, 0};
+  a.out0 = Dst{b0.g, pooled ? nullptr : b0.a, b0.cp, s.in1 >= 0 ? 1 : 0};
+  a.out0_tiles = m.cp0 / 32;
+  if (s.in1 >= 0) a.out1 = Dst{n.bufs[s.in1].g, nullptr, n.bufs[s.in1].cp, 0};
   a.batch = n.batch;
   a.h = a.w_px = hw;
   a.chunks = m.cpo / 32;
@@ -1021,9 +1043,10 @@ static void pool_bwd(NnNet& n, int in, int out, int lv) {
 hipError_t nn_forward(NnNet& n) {
   const LayerMap &f = n.table.l[0], &l = n.table.l[14];
   const long npx = (long)n.batch * n.s * n.s;
-  for (int cg = 0; cg < f.cpo / 8; cg += 32)
+  const int cf = n.bufs[B_A0].cp, cl = n.bufs[B_D0].cp;
+  for (int cg = 0; cg < cf / 8; cg += 32)
     hipLaunchKernelGGL(k_first_fwd, dim3((unsigned)std::max<long>(1, std::min<long>(2048, npx / 64))), dim3(256), 0,
-                       n.stream, n.x, n.wb + f.woff, n.w + f.boff, n.bufs[B_A0].a, f.cout, f.cpo, cg, npx, ilog2(n.s), n.s);
+                       n.stream, n.x, n.wb + f.woff, n.w + f.boff, n.bufs[B_A0].a, f.cout, cf, cg, npx, ilog2(n.s), n.s);
   for (const ConvStep& s : kSteps) {
     const hipError_t e = conv_fwd(n, s);
     if (e != hipSuccess) return e;
@@ -1032,7 +1055,7 @@ hipError_t nn_forward(NnNet& n) {
     if (s.out == B_E2) pool_fwd(n, B_E2, B_P2, 2);
   }
   hipLaunchKernelGGL(k_last_fwd, dim3(loop_blocks(npx)), dim3(256), 0, n.stream, n.bufs[B_D0].a, n.wb + l.woff,
-                     n.w + l.boff, n.out, l.cin, l.cpi, npx, (long)n.s * n.s);
+                     n.w + l.boff, n.out, l.cin, cl, npx, (long)n.s * n.s);
   return hipGetLastError();
 }
 
@@ -1052,10 +1075,11 @@ hipError_t nn_backward(NnNet& n) {
   const long ss = (long)n.s * n.s, npx = n.batch * ss;
   {
     const unsigned nb = (unsigned)std::max<long>(1, std::min<long>(NN_FIRST_BLOCKS, npx / 64));
-    for (int cg = 0; cg < l.cpi / 8; cg += 32)
+    const int cl = n.bufs[B_D0].cp;
+    for (int cg = 0; cg < cl / 8; cg += 32)
       hipLaunchKernelGGL(k_last_bwd, dim3(nb), dim3(256), 0, n.stream, n.gout, n.bufs[B_D0].a, n.wb + l.woff,
-                         n.bufs[B_D0].g, l.cin, l.cpi, cg, npx, ss, n.partial, n.bpart);
-    hipLaunchKernelGGL(k_last_sum, dim3(l.cin + 1, 2), dim3(64), 0, n.stream, n.partial, n.bpart, (int)nb, l.cin, l.cpi,
+                         n.bufs[B_D0].g, l.cin, cl, cg, npx, ss, n.partial, n.bpart);
+    hipLaunchKernelGGL(k_last_sum, dim3(l.cin + 1, 2), dim3(64), 0, n.stream, n.partial, n.bpart, (int)nb, l.cin, cl,
                        n.g + l.woff, n.g + l.boff);
   }
   for (int i = 12; i >= 0; --i) {
@@ -1068,7 +1092,7 @@ hipError_t nn_backward(NnNet& n) {
     if (e != hipSuccess) return e;
   }
   const unsigned nb = (unsigned)std::max<long>(1, std::min<long>(NN_FIRST_BLOCKS, npx / 64));
-  hipLaunchKernelGGL(k_first_wgrad, dim3(nb, f.cpo / 32), dim3(256), 0, n.stream, n.x, n.bufs[B_A0].g, f.cpo, npx,
+  hipLaunchKernelGGL(k_first_wgrad, dim3(nb, f.cpo / 32), dim3(256), 0, n.stream, n.x, n.bufs[B_A0].g, n.bufs[B_A0].cp, npx,
                      ilog2(n.s), n.s, n.partial, n.bpart);
   hipLaunchKernelGGL(k_first_sum, dim3(f.cout, 10), dim3(64), 0, n.stream, n.partial, n.bpart, (int)nb, f.cpo,
                      n.g + f.woff, n.g + f.boff);
@@ -1122,14 +1146,14 @@ hipError_t nn_create(NnNet& n, int s, int c, int batch) {
   n.bufs.resize(B_COUNT);
   hipError_t e = hipSuccess;
   for (int i = 0; i < B_COUNT && e == hipSuccess; ++i) {
-    n.bufs[i].cp = pad32(ch[i]);
+    n.bufs[i].cp = pad8(ch[i]);
     n.bufs[i].h = s >> lv[i];
     const size_t cnt = (size_t)batch * n.bufs[i].cp * n.bufs[i].h * n.bufs[i].h;
     e = nn_alloc1((void**)&n.bufs[i].a, cnt * sizeof(bf16));
     if (e == hipSuccess) e = nn_alloc1((void**)&n.bufs[i].g, cnt * sizeof(float));
   }
   for (int l = 0; l < 3 && e == hipSuccess; ++l)
-    e = nn_alloc1((void**)&n.arg[l], (size_t)batch * pad32(c << l) * (s >> (l + 1)) * (s >> (l + 1)));
+    e = nn_alloc1((void**)&n.arg[l], (size_t)batch * pad8(c << l) * (s >> (l + 1)) * (s >> (l + 1)));
   const size_t outc = (size_t)batch * 2 * s * s;
   if (e == hipSuccess) e = nn_alloc1((void**)&n.x, outc / 2 * sizeof(bf16));
   if (e == hipSuccess) e = nn_alloc1((void**)&n.out, outc * sizeof(float));

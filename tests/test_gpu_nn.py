@@ -198,7 +198,7 @@ def test_tile_shapes_agree_between_batch_sizes(s, c, batch):
             assert rel(g[part], gs[part]) <= 1e-4, (li, rel(g[part], gs[part]))
 
 
-@pytest.mark.parametrize("s,c,batch", [(16, 1, 2)])
+@pytest.mark.parametrize("s,c,batch", [(16, 1, 2), (32, 5, 2), (32, 12, 2), (16, 20, 3), (16, 40, 2)])
 def test_channels_that_fill_no_chunk_match_oracle(s, c, batch):
     """Channel counts whose tensors end inside a chunk of 32 or inside a group of 8, skip concatenations
     among them, or one channel throughout; bounds as in the gradient test."""
@@ -221,3 +221,19 @@ def test_channels_that_fill_no_chunk_match_oracle(s, c, batch):
         for part in (wl, bl):
             err, floor = rel(g[part], ref_g[part]), rel(n_g[part], ref_g[part])
             assert err <= max(2e-2, 3 * floor), (li, err, floor)
+
+
+def test_narrow_networks_hold_their_own_channels(gpu):
+    """Device memory of a network of 8 channels: its 17 tensors at 2 + 4 bytes a value, the images, and at
+    most 64 MiB for parameters and partial sums (with the tensors padded to 32 channels it was twice that)."""
+    import torch
+    s, c, batch = 256, 8, 16
+    ch = [c, c, c, 2 * c, 2 * c, 2 * c, 4 * c, 4 * c, 4 * c, 8 * c, 8 * c, 4 * c, 4 * c, 2 * c, 2 * c, c, c]
+    lv = [0, 0, 1, 1, 1, 2, 2, 2, 3, 3, 3, 2, 2, 1, 1, 0, 0]
+    tensors = batch * sum(k * (s >> v) ** 2 for k, v in zip(ch, lv)) * 6
+    images = batch * s * s * (2 + 4 * 2 + 4 * 2 + 2 * 2)
+    before = torch.cuda.mem_get_info()[0]
+    with warmstart.Net(size=s, c=c, batch=batch, seed=1):
+        held = before - torch.cuda.mem_get_info()[0]
+    print("held", held / 2 ** 20, "MiB; tensors", tensors / 2 ** 20, "images", images / 2 ** 20)
+    assert held <= 1.05 * (tensors + images) + (64 << 20)
