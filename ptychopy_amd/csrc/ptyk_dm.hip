@@ -209,7 +209,7 @@ __global__ __launch_bounds__(PTYK_NT) void k_dm_probe_apply(float2* __restrict__
 }
 
 // O += the increments (obj_row_sum; one rounding); per-block sum |O|^2.
-template <int M>
+template <int M, bool SHARE>
 __global__ __launch_bounds__(PTYK_NT) void k_dm_object(float2* __restrict__ obj, int obj_cols,
                                                        const float2* __restrict__ psi,
                                                        const float2* __restrict__ probe,
@@ -219,13 +219,13 @@ __global__ __launch_bounds__(PTYK_NT) void k_dm_object(float2* __restrict__ obj,
                                                        const float* __restrict__ factors, int phase_constraint,
                                                        double* __restrict__ block_sums) {
   __shared__ double red[PTYK_NT / 64];
-  constexpr int TC = dm_tile_width(M);
-  const int p = blockIdx.x, c = blockIdx.y * TC + threadIdx.x % TC;
-  const int t = p / PTYK_DM_TR * gridDim.y + blockIdx.y;
-  const double2 a = obj_row_sum<M>(p, c, psi, probe, roi, tile_frames, tile_ptr[t], tile_ptr[t + 1], factors[1],
-                                   phase_constraint);
+  const ObjRow<M, SHARE> at;
+  const int p = blockIdx.x, c = at.c;
+  int k0, k1;
+  at.list(tile_ptr, p, obj_cols, &k0, &k1);
+  const double2 a = obj_row_sum<M, SHARE>(at, p, psi, probe, roi, tile_frames, k0, k1, factors[1], phase_constraint);
   double s2 = 0.0;
-  if (threadIdx.x < TC && c < obj_cols) {
+  if (at.have(obj_cols)) {
     float2 o = obj[(long)p * obj_cols + c];
     o.x = (float)((double)o.x + a.x);
     o.y = (float)((double)o.y + a.y);
@@ -259,14 +259,17 @@ static hipError_t dm_impl(const DmArgs& a, hipStream_t s, DmTimer* tm) {
                        a.obj_cols, a.roi, a.n_frames, a.frames_per_chunk, a.probe_partial);
   }
   rec(DM_T_OBJ_GATHER);
-  hipLaunchKernelGGL((k_dm_object<M>), dim3(a.obj_rows, dm_tile_cols(a.obj_cols, M)), dim3(PTYK_NT), 0, s, a.obj,
-                     a.obj_cols, a.psi, a.probe, a.roi, a.tile_ptr, a.tile_frames, a.factors,
+  constexpr bool MAY = dm_may_share(M);
+  const bool share = dm_share_lists(M, a.obj_rows, a.obj_cols);
+  const int cols = share ? ObjRow<M, MAY>::COLS : ObjRow<M, false>::COLS, ocols = (a.obj_cols + cols - 1) / cols;
+  hipLaunchKernelGGL((share ? k_dm_object<M, MAY> : k_dm_object<M, false>), dim3(a.obj_rows, ocols), dim3(PTYK_NT), 0, s,
+                     a.obj, a.obj_cols, a.psi, a.probe, a.roi, a.tile_ptr, a.tile_frames, a.factors,
                      a.phase_constraint, a.obj_partial);
   rec(DM_T_PROBE_APPLY);
   hipLaunchKernelGGL((k_dm_probe_apply<M>), dim3(gp), dim3(PTYK_NT), 0, s, a.probe, a.probe_partial,
                      a.probe_chunks, a.factors, a.update_probe, a.probe_partial_sum);
   rec(DM_T_FINISH);
-  hipLaunchKernelGGL((k_dm_finish<PTYK_NT>), dim3(1), dim3(PTYK_NT), 0, s, a.obj_partial, a.obj_rows * dm_tile_cols(a.obj_cols, M),
+  hipLaunchKernelGGL((k_dm_finish<PTYK_NT>), dim3(1), dim3(PTYK_NT), 0, s, a.obj_partial, a.obj_rows * ocols,
                      a.probe_partial_sum, (int)gp, a.scal, a.factors);
   rec(-1);
   return hipGetLastError();

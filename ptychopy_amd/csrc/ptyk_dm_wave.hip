@@ -334,7 +334,7 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_pass_c(float2* __restrict__ psi
 }
 
 // dO += this wave's increments (obj_row_sum) on the object rows from row0.
-template <int M>
+template <int M, bool SHARE>
 __global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_accum(double2* __restrict__ d_obj, int row0, int obj_cols,
                                                            const float2* __restrict__ psi,
                                                            const float2* __restrict__ probe,
@@ -342,12 +342,12 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_obj_accum(double2* __restrict__
                                                            const int* __restrict__ tile_ptr,
                                                            const int* __restrict__ tile_frames,
                                                            const float* __restrict__ factors, int phase_constraint) {
-  constexpr int TC = dm_tile_width(M);
-  const int p = row0 + blockIdx.x, c = blockIdx.y * TC + threadIdx.x % TC;
-  const int t = p / PTYK_DM_TR * gridDim.y + blockIdx.y;
-  const int k0 = tile_ptr[t], k1 = tile_ptr[t + 1];
-  const double2 a = obj_row_sum<M>(p, c, psi, probe, roi, tile_frames, k0, k1, factors[1], phase_constraint);
-  if (threadIdx.x < TC && c < obj_cols && k1 > k0) {
+  const ObjRow<M, SHARE> at;
+  const int p = row0 + blockIdx.x, c = at.c;
+  int k0, k1;
+  at.list(tile_ptr, p, obj_cols, &k0, &k1);
+  const double2 a = obj_row_sum<M, SHARE>(at, p, psi, probe, roi, tile_frames, k0, k1, factors[1], phase_constraint);
+  if (at.have(obj_cols) && k1 > k0) {
     double2 d = d_obj[(long)p * obj_cols + c];
     d.x += a.x;
     d.y += a.y;
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(PTYK_NT) void k_dmw_probe_apply(float2* __restrict_
 template <int M>
 static hipError_t wave_impl(const DmWaveArgs& a, hipStream_t s, DmTimer* tm) {
   using C = WaveCfg<M>;
-  const int tcols = dm_tile_cols(a.obj_cols, M), cch = (a.obj_cols + PTYK_NT - 1) / PTYK_NT;
+  const int cch = (a.obj_cols + PTYK_NT - 1) / PTYK_NT;
   constexpr int RPW = M >= PTYK_NT ? 1 : PTYK_NT / M;
   for (int w = 0; w < a.n_waves; ++w) {
     const long f0 = (long)w * a.wave, f1 = f0 + a.wave < a.n_frames ? f0 + a.wave : a.n_frames;
@@ -468,8 +468,12 @@ static hipError_t wave_impl(const DmWaveArgs& a, hipStream_t s, DmTimer* tm) {
     const int lo = a.wave_tile_lo[w] * PTYK_DM_TR, hi = min(a.wave_tile_hi[w] * PTYK_DM_TR, a.obj_rows);
     if (hi > lo) {
       if (tm) tm->mark(s, DM_T_OBJ_GATHER);
-      hipLaunchKernelGGL((k_dmw_obj_accum<M>), dim3(hi - lo, tcols), dim3(PTYK_NT), 0, s, a.d_obj, lo, a.obj_cols, a.psi,
-                         a.probe, a.roi, a.wave_tile_ptr + (long)w * (dm_tiles(a.obj_rows, a.obj_cols, M) + 1),
+      constexpr bool MAY = dm_may_share(M);
+      const bool share = dm_share_lists(M, hi - lo, a.obj_cols);
+      const int cols = share ? ObjRow<M, MAY>::COLS : ObjRow<M, false>::COLS;
+      hipLaunchKernelGGL((share ? k_dmw_obj_accum<M, MAY> : k_dmw_obj_accum<M, false>),
+                         dim3(hi - lo, (a.obj_cols + cols - 1) / cols), dim3(PTYK_NT), 0, s, a.d_obj, lo, a.obj_cols,
+                         a.psi, a.probe, a.roi, a.wave_tile_ptr + (long)w * (dm_tiles(a.obj_rows, a.obj_cols, M) + 1),
                          a.wave_tile_frames, a.factors, a.phase_constraint);
     }
   }

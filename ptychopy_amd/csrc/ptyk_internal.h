@@ -48,7 +48,7 @@ struct DmArgs {
   const int* tile_ptr;    // dm_tiles + 1: CSR of the frames that touch each object tile
   const int* tile_frames; // frame ids, ascending per tile
   double2* probe_partial; // probe_chunks x M x M
-  double* obj_partial;    // obj_rows x dm_tile_cols
+  double* obj_partial;    // obj_rows x (a workgroup's columns)
   double* probe_partial_sum;  // M (one per probe row block)
   float* factors;         // device: [0] = 1/objMax cached, [1] = 1/probeMax cached
   double* scal;           // device: [0] objSum, [1] probeSum

@@ -206,3 +206,11 @@ def test_gathers_over_short_and_long_frame_lists(gpu, orc, m, n_side, step, wave
         psi = np.zeros((p["n"], m, m))
         for i in range(2):
             psi, _ = _check_step(e, orc, p, amp, E.FLAG_UPDATE_PROBE, psi, first_call=(i == 0))
+
+
+@pytest.mark.parametrize("m,n_side,step,wave", [(16, 3, 190.3, -1), (64, 3, 301.7, -1), (128, 2, 1010.4, 0),
+                                                (256, 2, 1105.6, 0), (256, 2, 1105.6, -1), (512, 2, 33.3, -1)])
+def test_gathers_on_wide_canvases(gpu, orc, m, n_side, step, wave):
+    """Canvases large enough that a column's frame list is one thread's: few frames, empty tiles, and last
+    blocks that end inside a tile."""
+    test_gathers_over_short_and_long_frame_lists(gpu, orc, m, n_side, step, wave)
