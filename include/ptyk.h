@@ -153,9 +153,9 @@ int ptyk_dm_iteration_timed(ptyk_ctx* ctx, uint32_t flags, float* kernel_ms);
  * PTYK_TUNE_EPIE_TEAM: 1 (default) shares an ePIE frame of 64^2 or more among a team of workgroups
  * where the device has a CU for each; 0 leaves it to one workgroup.  get returns the number of
  * workgroups (0: one workgroup, no team).
- * PTYK_TUNE_EPIE_TEAM_WAIT: how long (0..60000 ms; default 10000) a team's workgroup waits for the
- * others.  If they do not come together (other processes hold the device; always with 0), one
- * workgroup takes the iteration.
+ * PTYK_TUNE_EPIE_TEAM_WAIT: how long (0..60000 ms; default 250) a team's workgroup waits for the
+ * others at the start.  If they do not come together (other processes hold the device; always
+ * with 0), one workgroup takes the iteration.
  * PTYK_TUNE_EPIE_RESIDENT: most modes whose spectra a team keeps in LDS; 0 (default) = as many as
  * fit.  get returns the number for the handle's modes. */
 enum { PTYK_TUNE_DM_WAVE = 1, PTYK_TUNE_MLS_MOD_CB = 2, PTYK_TUNE_MLS_PUM_FPC = 3, PTYK_TUNE_MLS_GRAPHS = 4,

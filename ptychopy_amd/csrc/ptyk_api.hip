@@ -52,7 +52,7 @@ struct ptyk_ctx {
   double* e_err = nullptr;
   unsigned e_epoch = 1;
   int cus = 0;  // compute units of the device
-  int epie_team = 1, epie_wait_ms = 10000, epie_resident = 0;  // PTYK_TUNE_EPIE_*
+  int epie_team = 1, epie_wait_ms = 250, epie_resident = 0;  // PTYK_TUNE_EPIE_*
   // DM state
   float2* psi = nullptr;
   int* tile_ptr = nullptr;
@@ -630,7 +630,8 @@ int ptyk_epie_iteration(ptyk_ctx* c, const int32_t* order, uint32_t flags, doubl
   a.team_rowmax = c->e_rowmax;
   a.team_err = c->e_err;
   a.team_epoch = c->e_epoch;
-  a.team_limit = 100000LL * c->epie_wait_ms;
+  a.team_first = 100000LL * c->epie_wait_ms;
+  a.team_limit = 1000000000LL;  // 10 s
   a.k_res = c->epie_resident;
   double s[PTYK_SCAL_COUNT + 1];
   auto pass = [&] {

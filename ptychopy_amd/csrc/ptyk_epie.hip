@@ -625,7 +625,7 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
         beside[u] = bs.both > 0 ? ld_dev(row + (i < bs.left ? bs.s0 * PTYK_EPIE_SEG + i : ry + M + i - bs.left)) : 0.f;
       }
     }
-    if (!team_wait<W>(flags, epoch, a.team_limit, &gone, &most[0])) return;
+    if (!team_wait<W>(flags, epoch, s ? a.team_limit : a.team_first, &gone, &most[0])) return;
     if (a.update_probe && s > 0) probe_max = most[0];
 
     // ---- columns
@@ -950,7 +950,7 @@ static hipError_t epie_team_launch(EpieArgs a, hipStream_t s) {
                        a.obj_cols, a.team_segmax, a.team_rowmax);
   // with no wait at all, one workgroup stays out: the others find it missing and end (what becomes of a
   // team that does not come together, for tests)
-  hipLaunchKernelGGL((k_epie_team<M, MULTI>), dim3(a.team_limit ? T::W : T::W - 1), dim3(T::NT), lds, s, a);
+  hipLaunchKernelGGL((k_epie_team<M, MULTI>), dim3(a.team_first ? T::W : T::W - 1), dim3(T::NT), lds, s, a);
   return hipGetLastError();
 }
 template <int M>

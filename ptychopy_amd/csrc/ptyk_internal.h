@@ -210,11 +210,12 @@ struct EpieArgs {
   int n_pos, m, k_use, k_total, obj_rows, obj_cols;
   int phase_constraint, update_probe, modal, rms, tex_quantize;
   // team form (team_size = epie_team_size(m, CUs) > 0): barrier flags, maxima of |O|^2 over segments of
-  // canvas rows (rows x epie_segments) and over rows, and the workgroups' errors; the flags stand at team_epoch and move by epie_team_barriers(n_pos);
-  // team_limit bounds a barrier's wait (ticks of the 100 MHz clock; 0: one look); k_res: most modes whose
-  // spectra stay in LDS (0: as many as fit)
+  // canvas rows (rows x epie_segments) and over rows, and the workgroups' errors; the flags stand at
+  // team_epoch and move by epie_team_barriers(n_pos); team_first bounds the first barrier's wait (ticks of
+  // the 100 MHz clock; 0: one look), after which one workgroup can take over, and team_limit the others';
+  // k_res: most modes whose spectra stay in LDS (0: as many as fit)
   unsigned long long* team_flags; float *team_segmax, *team_rowmax; double* team_err;
-  unsigned team_epoch; int team_size, k_res; long long team_limit;
+  unsigned team_epoch; int team_size, k_res; long long team_first, team_limit;
 };
 // scal slot of the team form: team_epoch when the iteration ran, -team_epoch from where it may have changed the
 // state (anything else: it has not)

@@ -332,7 +332,7 @@ def test_a_team_that_does_not_come_together(gpu, m, modes):
                             e.get_scalars().view(np.uint64), np.float64(err).view(np.uint64)])
         return out
 
-    one, team = {E.TUNE_EPIE_TEAM: 0}, {E.TUNE_EPIE_TEAM: 1, E.TUNE_EPIE_TEAM_WAIT: 10000}
+    one, team = {E.TUNE_EPIE_TEAM: 0}, {E.TUNE_EPIE_TEAM: 1, E.TUNE_EPIE_TEAM_WAIT: 250}
     want = states(one, one, team, team)
     got = states({E.TUNE_EPIE_TEAM_WAIT: 0}, {}, team, team)
     for a, b in zip(want, got):
