@@ -7,7 +7,7 @@
 //
 // ePIE is a chain of dependent position updates, so one launch walks every position of an
 // iteration in the given order, with no host round trip per position.  Frames of 64^2 and more
-// are shared by a team of 8 to 32 workgroups (k_epie_team); smaller ones go to one workgroup that
+// are shared by a team of 16 to 128 workgroups (k_epie_team); smaller ones go to one workgroup that
 // keeps the exit waves in an L2-resident scratch and stages each 2D transform through LDS in row
 // and column chunks (k_epie).
 #include "../../include/ptyk.h"
@@ -245,14 +245,15 @@ __global__ __launch_bounds__(PTYK_EPIE_NT) void k_epie(EpieArgs a) {
 // arithmetic.  So every value another workgroup reads (exchange buffer, object, |O|^2, maxima) is
 // written and read with device-scope accesses, which go to that cache by themselves, and a barrier
 // is a wait for the stores to be acknowledged, one flag store and a poll: no cache is written back
-// or invalidated (an agent-scope release here writes back a whole L2).  A thread holds 4 to 8
-// values, so a transform is 3 or 4 short stages between two LDS tiles with one workgroup barrier
-// each, its twiddles kept in registers for the whole iteration.
+// or invalidated (an agent-scope release here writes back a whole L2).  A thread holds 4 values, so a
+// transform is 3 or 4 short stages between two LDS tiles with one workgroup barrier each, its twiddles
+// kept in registers for the whole iteration.
 //
 // Team sizes: 4 rows a workgroup.  More rows mean fewer flags to wait for but more instructions per
 // thread in every step of the chain (64^2 in 8 workgroups of 8 rows: 14.0 us a position, in 16 of 4:
 // 10.7; 128^2 in 16: 15.0, in 32: 12.0; 256^2 with three modes in 32: 42.6, in 64: 28.6; 512^2 in 64:
-// 33, in 128: 27).  One workgroup on one CU took 14.7, 44, 1120 and 1730.  The radix order of 128
+// 33, in 128: 27; all with the copies to the host; the iteration alone is now 10.1, 10.9, 24.4 and 16.6).
+// One workgroup on one CU took 14.7, 44, 1120 and 1730.  The radix order of 128
 // is the one of the least error (median 1.5e-6 of the object over an iteration of the 12 x 12
 // benchmark scan; 2.0e-6 for 4 4 4 2).
 template <int M> struct TeamCfg;
@@ -274,7 +275,7 @@ struct Team : TeamCfg<M> {
   static constexpr int TPR = T::NT / R;      // threads per row of the scan beside the ROI
   static constexpr int NB = (2 * (PTYK_EPIE_SEG - 1) + TPR - 1) / TPR;  // pixels of it per thread
   static constexpr int CELLS = M / PTYK_EPIE_SEG + 1;                   // segments an ROI row may touch
-  static_assert(T::R0 * T::R1 * T::R2 * T::R3 == M, "radices");
+  static_assert(T::R0 * T::R1 * T::R2 * T::R3 == M && (T::S == 3 || T::S == 4), "radices");
   static_assert(PPT <= R && R % PPT == 0, "a thread's amplitudes lie in the workgroup's columns of one row");
   static_assert(TPR % 8 == 0, "threads beside the ROI: whole groups of 8 lanes per row");
   static_assert(M % PTYK_EPIE_SEG == 0 && PTYK_EPIE_SEG == 64 && R * CELLS <= 64, "a wave's pixels meet two segments");
@@ -453,7 +454,7 @@ struct TeamTw {
   float2 a[TeamStage<M, T::R1>::NW], b[TeamStage<M, T::R2>::NW], c[TeamStage<M, T::R3>::NW];
   __device__ __forceinline__ void load(const float2* __restrict__ tw, int tid) {
     team_twiddles<M, T::R1, T::R0>(a, tw, tid);
-    if constexpr (T::S > 2) team_twiddles<M, T::R2, T::R0 * T::R1>(b, tw, tid);
+    team_twiddles<M, T::R2, T::R0 * T::R1>(b, tw, tid);
     if constexpr (T::S > 3) team_twiddles<M, T::R3, T::R0 * T::R1 * T::R2>(c, tw, tid);
   }
 };
@@ -465,8 +466,7 @@ __device__ __forceinline__ float2* team_fft(float2* t0, float2* t1, const TeamTw
   __syncthreads();
   team_stage<M, T::R0, 1, INV>(t0, t1, nullptr, tid);
   team_stage<M, T::R1, T::R0, INV>(t1, t0, w.a, tid);
-  if constexpr (T::S == 2) return t0;
-  if constexpr (T::S > 2) team_stage<M, T::R2, T::R0 * T::R1, INV>(t0, t1, w.b, tid);
+  team_stage<M, T::R2, T::R0 * T::R1, INV>(t0, t1, w.b, tid);
   if constexpr (T::S > 3) {
     team_stage<M, T::R3, T::R0 * T::R1 * T::R2, INV>(t1, t0, w.c, tid);
     return t0;
@@ -566,7 +566,12 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
   load_object(pos);
   Halves ah = load_amps(fi);
 
+  const int thread = tid;
   for (int s = 0; s < a.n_pos; ++s) {
+    int tid = thread;
+    // addresses made anew per position: kept for all of them they filled the registers of the 512^2 form
+    // (256 and 42 spilled; now 217; three modes 40 -> 36 us a position)
+    if (MULTI && M == 512) asm volatile("" : "+v"(tid));
     const float ascale = a.amp_scale[fi];
     const int rx = (int)roundf(pos.x), ry = (int)roundf(pos.y);
     const Beside bs = beside_of(ry);
@@ -614,38 +619,21 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
       if (MULTI) __syncthreads();
     }
     team_arrive(flags, w, ++epoch, value);
-    // meanwhile: |O|^2 that this position does not write, for max |O|^2 after its update: the pixels
-    // beside the ROI in this workgroup's rows
-    float beside[T::NB];
-    if (a.update_probe) {
+    // |O|^2 that this position does not write, for max |O|^2 after its update: the pixels beside the ROI
+    // in this workgroup's rows, and (behind the barrier) the row's segments and a share of the rows apart
+    // from the ROI, one load a thread to 1024 columns and rows at 64^2, the rest in rounds of four.  With
+    // several modes all of it waits for the end of the column step: kept through the modes' transforms the
+    // values cost registers there (128^2, three modes: 23.2 us a position; at the end 21.9).
+    float beside[T::NB], segs = 0.f, rows = 0.f;
+    auto load_beside = [&]() __attribute__((always_inline)) {
       const float* row = a.obj_int + (long)(rx + w * R + brow) * a.obj_cols;
 #pragma unroll
       for (int u = 0; u < T::NB; ++u) {
         const int i = min(bcol + u * T::TPR, bs.both - 1);
         beside[u] = bs.both > 0 ? ld_dev(row + (i < bs.left ? bs.s0 * PTYK_EPIE_SEG + i : ry + M + i - bs.left)) : 0.f;
       }
-    }
-    if (!team_wait<W>(flags, epoch, s ? a.team_limit : a.team_first, &gone, &most[0])) return;
-    if (a.update_probe && s > 0) probe_max = most[0];
-
-    // ---- columns
-    float ms[PPT];
-    float2 sm[PPT];
-    if (MULTI) {
-#pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        ms[j] = 0.f;
-        sm[j] = make_float2(0.f, 0.f);
-      }
-    }
-    float2* const xc = a.psi + (long)w * R * M;  // this workgroup's columns (mode 0)
-    float2 g[PPT];
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) g[j] = ld_dev(xc + tid + j * NT);
-    // and the segments and rows apart from the ROI (the row's segments; a share of the rows): one load a
-    // thread to 1024 columns and rows at 64^2, the rest in rounds of four
-    float segs = 0.f, rows = 0.f;
-    if (a.update_probe) {
+    };
+    auto load_apart = [&]() __attribute__((always_inline)) {
       const float* seg = a.team_segmax + (long)(rx + w * R + brow) * nseg;
       const int nrest = nseg - bs.n, nrow = a.obj_rows - M;
       auto seg_at = [&](int i) __attribute__((always_inline)) {
@@ -669,7 +657,26 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
       };
       if (nrest > T::TPR) segs = fmaxf(segs, rounds(bcol + T::TPR, T::TPR, nrest, seg_at));
       if (nrow > W * 64) rows = fmaxf(rows, rounds(r0 + W * 64, W * 64, nrow, row_at));
+    };
+    if (a.update_probe && !MULTI) load_beside();
+    if (!team_wait<W>(flags, epoch, s ? a.team_limit : a.team_first, &gone, &most[0])) return;
+    if (a.update_probe && s > 0) probe_max = most[0];
+
+    // ---- columns
+    float ms[PPT];
+    float2 sm[PPT];
+    if (MULTI) {
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        ms[j] = 0.f;
+        sm[j] = make_float2(0.f, 0.f);
+      }
     }
+    float2* const xc = a.psi + (long)w * R * M;  // this workgroup's columns (mode 0)
+    float2 g[PPT];
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) g[j] = ld_dev(xc + tid + j * NT);
+    if (a.update_probe && !MULTI) load_apart();
     for (int k = 0; k < ku; ++k) {
       float2* x = xc + (long)k * MM;
       // a resident mode's spectrum has to end in its own tile
@@ -737,6 +744,10 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
         }
         __syncthreads();
       }
+    }
+    if (a.update_probe && MULTI) {
+      load_beside();
+      load_apart();
     }
     team_arrive(flags, w, ++epoch, value + 1);
     const float co = (float)(1.0 / (double)probe_max);
@@ -850,20 +861,22 @@ __global__ __launch_bounds__(TeamCfg<M>::NT) void k_epie_team(EpieArgs a) {
       const float cp = (float)(1.0 / (double)obj_max);
       float pm = rest, im[PPT];
       for (int k = 0; k < ku; ++k) {
+        const long q = (long)k * MM + px0 + tid;
+        // all loads before the stores, which the compiler takes to alias them (256^2, three modes: 26.5 us a
+        // position with loads and stores by turns, 24.4 so)
+        float2 dk[PPT], pk[PPT];
 #pragma unroll
         for (int j = 0; j < PPT; ++j) {
-          const long q = (long)k * MM + px0 + tid + j * NT;
-          if (MULTI) {
-            const float2 p = cadd(cscale(cmulcj(on[j], a.psi_old[q]), cp), a.probe[q]);
-            a.probe[q] = p;
-            if (k == 0) pv[j] = p;
-            const float ia = sqrtf(p.x * p.x + p.y * p.y);
-            im[j] = k ? im[j] + ia * ia : ia * ia;
-          } else {
-            pv[j] = cadd(cscale(cmulcj(on[j], d[j]), cp), pv[j]);
-            const float ia = sqrtf(pv[j].x * pv[j].x + pv[j].y * pv[j].y);
-            im[j] = ia * ia;
-          }
+          dk[j] = MULTI ? a.psi_old[q + j * NT] : d[j];
+          pk[j] = MULTI ? a.probe[q + j * NT] : pv[j];
+        }
+#pragma unroll
+        for (int j = 0; j < PPT; ++j) {
+          const float2 p = cadd(cscale(cmulcj(on[j], dk[j]), cp), pk[j]);
+          if (MULTI) a.probe[q + j * NT] = p;
+          if (!MULTI || k == 0) pv[j] = p;
+          const float ia = sqrtf(p.x * p.x + p.y * p.y);
+          im[j] = MULTI && k ? im[j] + ia * ia : ia * ia;
         }
       }
 #pragma unroll
