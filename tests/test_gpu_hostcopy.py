@@ -30,3 +30,17 @@ def test_predictions_of_many_batches_equal_those_of_one(gpu, n):
             whole = f(x)
             for i in range(0, n, 4):
                 assert np.array_equal(whole[i:i + 4], f(x[i:i + 4]))
+
+
+@pytest.mark.parametrize("m,rows,cols", [(256, 456, 456), (256, 457, 301), (128, 481, 487), (512, 700, 700)])
+def test_frames_simulated_together_equal_single_ones(gpu, m, rows, cols):
+    """Buffers in one allocation or in two, objects of odd sizes among them."""
+    from ptychopy_amd._engine import Engine
+    g = np.random.default_rng(rows + cols)
+    obj = (g.normal(size=(rows, cols)) + 1j * g.normal(size=(rows, cols))).astype(np.complex64)
+    probe = (g.normal(size=(m, m)) + 1j * g.normal(size=(m, m))).astype(np.complex64)
+    pos = (g.uniform(0, 1, size=(12, 2)) * (rows - m, cols - m)).astype(np.float32)
+    with Engine(1, m, (rows, cols)) as e:
+        whole = e.simulate(obj, probe, pos)
+        for i in range(len(pos)):
+            assert np.array_equal(whole[i:i + 1], e.simulate(obj, probe, pos[i:i + 1]))
